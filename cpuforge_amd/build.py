@@ -19,7 +19,7 @@ INCLUDE = os.path.join(ROOT, "include")
 OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcfattn.so")
 
-HIP_SOURCES = ["attn_fwd.hip", "attn_fwd_q64.hip", "attn_bwd.hip", "attn_dkdv.hip", "attn_f32.hip", "prologue.hip", "layer_ops.hip", "lora.hip",
+HIP_SOURCES = ["attn_fwd.hip", "attn_fwd_q64.hip", "attn_bwd.hip", "attn_dkdv.hip", "attn_f32.hip", "prologue.hip", "layer_ops.hip", "lora.hip", "gemm_f32.hip",
                "io_kernels.hip", "noalloc.hip", "probe.hip", "cfattn_capi.cpp", "cfops_capi.cpp", "cfio_capi.cpp", "host_stage.cpp"]
 ARCH = "gfx950"
 COMMON = ["-std=c++17", "-fPIC", "-O3", f"--offload-arch={ARCH}", f"-I{INCLUDE}", f"-I{CSRC}",
@@ -71,9 +71,7 @@ def build(verbose: bool = False) -> str:
     if failed:
         raise RuntimeError("hipcc failed:\n" + "\n".join(failed))
     tmp = LIB + ".tmp"
-    # hipBLASLt runs the plain f32 GEMMs of the layer ops (matmul_*, Linear).
-    cmd = [cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp, "-L/opt/rocm/lib", "-lhipblaslt",
-           "-pthread"]
+    cmd = [cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp, "-pthread"]
     out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if out.returncode != 0:
         raise RuntimeError("link failed:\n" + _filter(out.stdout))

@@ -289,7 +289,6 @@ int cfattn_destroy(cfattn_ctx* c) {
         if (c->fwd_settles) (void)hipFree(c->fwd_settles);
         for (int i = 0; i < cfattn_ctx::NSLOT; i++)
             if (c->buf[i]) (void)hipFree(c->buf[i]);
-        if (c->blas && c->blas_release) c->blas_release(c->blas);
     }
     delete c;
     return CFATTN_OK;

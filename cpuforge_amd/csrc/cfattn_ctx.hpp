@@ -120,11 +120,6 @@ struct cfattn_ctx {
     EventTimer* timer = nullptr;  // non-null while profiling is on
     unsigned prof_mask = ~0u;     // kernels profiling brackets (cfattn_profile_select)
     size_t ds_limit = (size_t)8 << 30;  // stored-dS scratch limit (cfattn_set_ds_limit)
-    // GEMM library state of the layer ops (hipBLASLt handle and per-shape
-    // plans), created on first use; released by cfattn_destroy through
-    // blas_release.
-    void* blas = nullptr;
-    void (*blas_release)(void*) = nullptr;
     size_t head_chunk_bytes = (size_t)512 << 20;  // logits buffer limit of cfops_lm_head_ce
     // Pinned staging of the on-disk formats (two host chunks and their
     // events), created on first use; released by cfattn_destroy.

@@ -48,6 +48,35 @@ hipError_t launch_ce_finish(const int64_t* targets, const float* row_loss, size_
 hipError_t launch_adamw(float* p, const float* g, float* m, float* v, size_t n, float lr, float beta1, float beta2,
                         float eps, float weight_decay, float bc1, float bc2, hipStream_t st);
 
+// f32 GEMMs over a common row count m (gemm_f32.hip).  Problem i is
+//   C_i[m, n_i] (+)= alpha * (sum over its segments s of A_s B_s),
+// the segments being runs of one long contraction (a base product and an
+// adapter's, or the products of several linears into one gradient).  A
+// element (row, k) is at a[row * lda + k], or a[k * lda + row] with
+// a_strided; B element (k, col) at b[col * ldb + k], or b[k * ldb + col] with
+// b_strided.  No operand needs more than its natural alignment.
+constexpr int kGemmSegs = 8, kGemmProblems = 4;
+struct GemmSeg {
+    const float *a, *b;
+    long lda, ldb;
+    int k;
+};
+struct GemmProblem {
+    GemmSeg seg[kGemmSegs];
+    int nseg = 0;
+    float* c = nullptr;
+    int n = 0;
+};
+struct GemmF32 {
+    GemmProblem pr[kGemmProblems];
+    int npr = 0, m = 0;
+    int acc = 0;  // 1: add to C, 0: overwrite it
+    float alpha = 1.0f;
+    bool a_strided = false, b_strided = false;
+};
+// `ws` is scratch for the partial sums of a split contraction.
+hipError_t launch_gemm_f32(const GemmF32& g, float* ws, size_t ws_floats, hipStream_t st);
+
 // LoRA adapter products of Linear::forward / backward (linear.rs:56-91) as
 // streaming kernels (lora.hip), for ranks 4, 8 and 16 with 16-byte aligned
 // rows; `part` is scratch of lora_partial_floats floats for the per-chunk

@@ -1,0 +1,486 @@
+// f32 GEMMs of the layer ops (matmul_nn / matmul_nt / matmul_tn,
+// crates/core/src/matmul.rs:127-147, and Linear's products,
+// crates/model/src/linear.rs:56-91) on the bf16 matrix cores, each f32
+// operand split into three bf16 pieces (split3.hpp).
+//
+// What bounds it: on a full chip the board's power.  2000 x 2048 x 8192 (m, k,
+// n) ran at 1.85 of 2.4 GHz with the matrix cores busy in 62% of the cycles:
+// 176-200 TFLOP/s of f32 work, 1050-1200 of bf16, against 140 for the f32 MFMA
+// library GEMM it replaced (the bf16 MFMA alone reaches 1704 on random
+// operands).  On the small grids of a layer (160 tiles of 128 x 128 for 4096
+// x 576) it is a workgroup's own chain: two waves to a SIMD, 49% matrix-core
+// busy between the splitting, the LDS reads and one barrier a step.  Before
+// and after, in us: 4096 x 1536 x 576 70 and 64; 4096 x 576 x 1536 69 and 58;
+// the LM head's 2730 x 576 x 49152 1200 and 939, its gradients 2730 x 49152 x 576
+// 2640 and 947 and 49152 x 2730 x 576 1220 and 936.
+//
+// A workgroup splits its tiles as it stores them to LDS (three planes), so
+// memory is read in f32, once per tile.  Two LDS buffers and two register
+// sets: the loads of a step are two steps old when they are split.  (One more
+// buffer, so that no wave waits at a step's first LDS read, and one wave to a SIMD:
+// slower, 73 us where this takes 60.  Unpacking with v_dot2_f32_bf16, one
+// instruction for two: slower, it needs wait states.)
+//
+// Relative error against 64 bits, normal values, before and after: k = 576
+// 4.3e-7 and 1.4e-7, k = 4096 1.1e-6 and 2.2e-7.  The leading product has its
+// own sums: in one sum with the other five the MFMA cuts off their low bits as it
+// aligns them to the larger values (towards minus infinity, so every sum came
+// out 4e-8 to 1.5e-7 of its size too small, and a training step's gradients four times
+// further off than before).
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdint>
+
+#include "cfops_kernels.hpp"
+#include "split3.hpp"
+
+namespace cfattn {
+namespace {
+
+constexpr int kOct = 4;       // octets (runs of eight k) of a step
+constexpr int kBK = 8 * kOct;  // k values of a step
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+struct GemmArgs {
+    GemmProblem pr[kGemmProblems];
+    int npr, m, acc;
+    int mt, nt;          // tiles over m, and over all problems' n
+    int per;             // k steps per split
+    int n_inner;
+    float alpha;
+    float* part;         // partial products of the splits, or null
+};
+
+template <bool STRIDED>
+__device__ __forceinline__ float elem(const float* __restrict__ p, long ld, long row, long k) {
+    return STRIDED ? p[k * ld + row] : p[row * ld + k];
+}
+
+// k steps of a problem: a step is kOct octets.  First the whole steps of each
+// segment in turn, then the segments' remaining octets, kOct to a step.
+__host__ __device__ __forceinline__ int whole_steps(const GemmProblem& p) {
+    int n = 0;
+    for (int s = 0; s < p.nseg; s++) n += p.seg[s].k / kBK;
+    return n;
+}
+__host__ __device__ __forceinline__ int all_steps(const GemmProblem& p) {
+    int n = 0;
+    for (int s = 0; s < p.nseg; s++) n += (p.seg[s].k % kBK + 7) / 8;
+    return whole_steps(p) + (n + kOct - 1) / kOct;
+}
+// The octet `o` of the rest: its segment, first k and length (0 past the last).
+struct Octet {
+    int seg, k, len;
+};
+__device__ __forceinline__ Octet rest_octet(const GemmProblem& p, int o) {
+    Octet r{0, 0, 0};
+    for (int s = 0; s < p.nseg; s++) {
+        const int k = p.seg[s].k, n = (k % kBK + 7) / 8;
+        if (o >= 0 && o < n) {
+            const int k0 = k / kBK * kBK + 8 * o;
+            r = Octet{s, k0, min(8, k - k0)};
+        }
+        o -= n;
+    }
+    return r;
+}
+
+// This thread's share of an operand tile of ROWS rows and kOct octets, NT
+// threads: U units of one row and eight consecutive k.
+//   k along memory: kOct lanes cover the 32 * kOct bytes of a row;
+//   STRIDED: a wave covers 64 consecutive rows at each of its eight k.
+// Off: type of a byte offset within a tile.
+template <bool STRIDED, int ROWS, int NT, typename Off>
+struct TileLoad {
+    static constexpr int U = ROWS * kOct / NT;
+    // 16-byte LDS chunks from octet to octet: eight lanes of a write (two rows,
+    // kOct octets) land on eight different 16-byte bank groups.
+    static constexpr int PITCH = ROWS + 2;
+    static_assert(U * NT == ROWS * kOct, "a tile must be whole units per thread");
+    float v[U][8];
+    __device__ __forceinline__ static int row(int tid, int u) {
+        return STRIDED ? (tid & 63) + 64 * (tid / (64 * kOct)) + (NT / kOct) * u : tid / kOct + (NT / kOct) * u;
+    }
+    __device__ __forceinline__ static int oct(int tid) {
+        return (STRIDED ? wave_uniform(tid >> 6) : tid) % kOct;
+    }
+    // Byte offset of unit u in a tile that starts at its first row and k.
+    // Rows past the last one repeat it (their results are not stored).
+    __device__ __forceinline__ static Off offset(int tid, int u, int last, Off ld) {
+        const Off r = min(row(tid, u), last);
+        return STRIDED ? 4 * r : 4 * (r * ld + oct(tid) * 8);
+    }
+    __device__ __forceinline__ void load(const float* __restrict__ base, long ld, const Off (&off)[U], int tid) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if constexpr (STRIDED) {
+                const float* q = base + oct(tid) * 8 * ld;
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    v[u][j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(q + j * ld) + off[u]);
+            } else {
+                const char* q = reinterpret_cast<const char*>(base) + off[u];
+                const f32x4u a = *reinterpret_cast<const f32x4u*>(q), b = *reinterpret_cast<const f32x4u*>(q + 16);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[u][j] = a[j], v[u][j + 4] = b[j];
+            }
+        }
+    }
+    // One octet of a segment, zero past its length.
+    __device__ __forceinline__ void load_octet(const float* __restrict__ p, long ld, int row0, int last, int k, int len,
+                                               int tid) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int r = row0 + min(row(tid, u), last);
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[u][j] = j < len ? elem<STRIDED>(p, ld, r, k + j) : 0.0f;
+        }
+    }
+    // Split and stored as three planes of [kOct][PITCH] chunks.
+    __device__ __forceinline__ void store(uint4* s, int tid) const {
+        constexpr int P = kOct * PITCH;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const Split8 sp = split8(v[u]);
+            uint4* d = s + oct(tid) * PITCH + row(tid, u);
+            d[0] = sp.p[0];
+            d[P] = sp.p[1];
+            d[2 * P] = sp.p[2];
+        }
+    }
+};
+
+// The LDS writes of this step are done in every wave; loads to registers stay
+// in flight (__syncthreads would wait for them).
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// C tile of BM x BN, NT / 64 waves in WR = NT / 128 rows of two.
+template <bool AS, bool BS, int BM, int BN, int NT, typename Off = uint32_t>
+__global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
+    constexpr int WR = NT / 128;
+    constexpr int MB = BM / WR / 32, NB = BN / 64;  // 32 x 32 blocks of a wave
+    using LoadA = TileLoad<AS, BM, NT, Off>;
+    using LoadB = TileLoad<BS, BN, NT, Off>;
+    constexpr int PA = kOct * LoadA::PITCH, PB = kOct * LoadB::PITCH;
+    __shared__ uint4 sA[2][3 * PA];
+    __shared__ uint4 sB[2][3 * PB];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = wave_uniform(tid >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+    int id = xcd_remap(blockIdx.x, gridDim.x, 1);
+    const int tiles = g.mt * g.nt;
+    const int split = id / tiles;
+    id %= tiles;
+    const int tm = g.n_inner ? id / g.nt : id % g.mt;
+    int tn = g.n_inner ? id % g.nt : id / g.mt;
+    int pi = 0;
+    long part_off = 0;  // columns of the problems before this one
+    for (; pi + 1 < g.npr && tn >= (g.pr[pi].n + BN - 1) / BN; pi++) {
+        tn -= (g.pr[pi].n + BN - 1) / BN;
+        part_off += g.pr[pi].n;
+    }
+    const GemmProblem& p = g.pr[pi];
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int lastA = g.m - 1 - m0, lastB = p.n - 1 - n0;
+    const int n_whole = whole_steps(p);
+    const int st0 = split * g.per, st1 = min(all_steps(p), st0 + g.per);
+
+    f32x16 acc[MB][NB], low[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[i][j] = low[i][j] = zero16();
+
+    const int ar = (wave >> 1) * (BM / WR) + l32, br = (wave & 1) * (BN / 2) + l32;
+    auto products = [&](int cur) {
+#pragma unroll
+        for (int s = 0; s < kOct / 2; s++) {
+            bf16x8 a[3][MB], b[3][NB];
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+#pragma unroll
+                for (int i = 0; i < MB; i++)
+                    a[q][i] = __builtin_bit_cast(bf16x8, sA[cur][q * PA + (2 * s + hh) * LoadA::PITCH + ar + 32 * i]);
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+                    b[q][j] = __builtin_bit_cast(bf16x8, sB[cur][q * PB + (2 * s + hh) * LoadB::PITCH + br + 32 * j]);
+            }
+            // The five products below the first go to sums of their own, smallest first.
+            constexpr int pa[5] = {2, 0, 1, 1, 0}, pb[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+#pragma unroll
+                for (int i = 0; i < MB; i++)
+#pragma unroll
+                    for (int j = 0; j < NB; j++) low[i][j] = mfma32(a[pa[q]][i], b[pb[q]][j], low[i][j]);
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++) acc[i][j] = mfma32(a[0][i], b[0][j], acc[i][j]);
+        }
+    };
+
+    // Whole k steps.  A step: the products of one LDS buffer; beside them the
+    // next step's tile (in registers since two steps ago) is split into the
+    // other buffer, and then the loads of the step three ahead go out into
+    // the same registers.  Past the end the last step's loads are repeated: a
+    // load that may or may not be in flight would make every wait one for
+    // all of them.
+    const int end = min(st1, n_whole);
+    if (st0 < end) {
+        struct Regs {
+            LoadA a;
+            LoadB b;
+        } r0, r1;
+        // Where the next load is: segment, its pointers and whole steps left.
+        int sg = 0, left = st0, todo = end - st0;
+        while (left >= p.seg[sg].k / kBK) left -= p.seg[sg++].k / kBK;
+        const float *pa, *pb;
+        long lda, ldb;
+        Off offa[LoadA::U], offb[LoadB::U];
+        auto enter = [&](int skip) {
+            const GemmSeg& s = p.seg[sg];
+            lda = s.lda, ldb = s.ldb;
+            left = s.k / kBK - skip;
+            pa = AS ? s.a + m0 + (long)skip * kBK * lda : s.a + m0 * lda + (long)skip * kBK;
+            pb = BS ? s.b + n0 + (long)skip * kBK * ldb : s.b + n0 * ldb + (long)skip * kBK;
+#pragma unroll
+            for (int u = 0; u < LoadA::U; u++) offa[u] = LoadA::offset(tid, u, lastA, (Off)lda);
+#pragma unroll
+            for (int u = 0; u < LoadB::U; u++) offb[u] = LoadB::offset(tid, u, lastB, (Off)ldb);
+        };
+        enter(left);
+        auto load = [&](Regs& r) {
+            r.a.load(pa, lda, offa, tid);
+            r.b.load(pb, ldb, offb, tid);
+            if (--todo > 0) {
+                if (--left > 0) {
+                    pa += AS ? kBK * lda : kBK;
+                    pb += BS ? kBK * ldb : kBK;
+                } else {
+                    do sg++;
+                    while (p.seg[sg].k < kBK);
+                    enter(0);
+                }
+            }
+        };
+        load(r0);
+        load(r1);
+        r0.a.store(sA[0], tid);
+        r0.b.store(sB[0], tid);
+        load(r0);
+        int st = st0;
+        auto step = [&](int cur, Regs& r) {
+            products(cur);
+            r.a.store(sA[cur ^ 1], tid);
+            r.b.store(sB[cur ^ 1], tid);
+            load(r);
+            lds_barrier();
+        };
+        lds_barrier();
+        for (; st + 1 < end; st += 2) {
+            step(0, r1);
+            step(1, r0);
+        }
+        if (st < end) step(0, r1);
+    }
+    for (int st = max(st0, n_whole); st < st1; st++) {
+        LoadA a;
+        LoadB b;
+        const Octet oa = rest_octet(p, kOct * (st - n_whole) + LoadA::oct(tid));
+        const Octet ob = rest_octet(p, kOct * (st - n_whole) + LoadB::oct(tid));
+        a.load_octet(p.seg[oa.seg].a, p.seg[oa.seg].lda, m0, lastA, oa.k, oa.len, tid);
+        b.load_octet(p.seg[ob.seg].b, p.seg[ob.seg].ldb, n0, lastB, ob.k, ob.len, tid);
+        a.store(sA[0], tid);
+        b.store(sB[0], tid);
+        lds_barrier();
+        products(0);
+        lds_barrier();
+    }
+
+    // A sum that is not finite may only be so in the pieces: such a wave
+    // forms its tile again in f32, in k order.
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            acc[i][j] += low[i][j];
+#pragma unroll
+            for (int r = 0; r < 16; r++) odd |= !(fabsf(acc[i][j][r]) < INFINITY);
+        }
+    const int mw = m0 + (wave >> 1) * (BM / WR) + 4 * hh, nw = n0 + br;
+    if (__any(odd)) {
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const long row = min(mw + 32 * i + 8 * (r >> 2) + (r & 3), g.m - 1), col = min(nw + 32 * j, p.n - 1);
+                    float sum = 0.0f;
+                    int first = 0;  // whole steps of the segments before
+                    auto run = [&](const GemmSeg& s, int k0, int k1) {
+                        for (int k = k0; k < k1; k++)
+                            sum = __builtin_fmaf(elem<AS>(s.a, s.lda, row, k), elem<BS>(s.b, s.ldb, col, k), sum);
+                    };
+                    for (int s = 0; s < p.nseg; s++) {
+                        const int n = p.seg[s].k / kBK;
+                        run(p.seg[s], (max(st0, first) - first) * kBK, (min(st1, first + n) - first) * kBK);
+                        first += n;
+                    }
+                    for (int o = kOct * (max(st0, n_whole) - n_whole); o < kOct * (st1 - n_whole); o++) {
+                        const Octet oc = rest_octet(p, o);
+                        run(p.seg[oc.seg], oc.k, oc.k + oc.len);
+                    }
+                    acc[i][j][r] = sum;
+                }
+    }
+
+    // Partial products: [split][m][all problems' columns, problem by problem].
+    float* out = p.c;
+    if (g.part) {
+        long cols = 0;
+        for (int i = 0; i < g.npr; i++) cols += g.pr[i].n;
+        out = g.part + (split * cols + part_off) * g.m;
+    }
+    const bool add = g.acc && !g.part;
+    const float alpha = g.part ? 1.0f : g.alpha;
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int col = nw + 32 * j;
+            if (col >= p.n) continue;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int row = mw + 32 * i + 8 * (r >> 2) + (r & 3);
+                if (row >= g.m) continue;
+                float* o = out + (long)row * p.n + col;
+                const float v = alpha * acc[i][j][r];
+                *o = add ? *o + v : v;
+            }
+        }
+}
+
+// C (+)= alpha * (the splits' partial products, added in split order).
+__global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmArgs g, int splits, long cols) {
+    const GemmProblem& p = g.pr[blockIdx.y];
+    long off = 0;
+    for (int i = 0; i < (int)blockIdx.y; i++) off += g.pr[i].n;
+    const long mn = (long)g.m * p.n, stride = cols * g.m;
+    const float* part = g.part + off * g.m;
+    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < mn; e += (long)gridDim.x * 256) {
+        float s = part[e];
+        for (int i = 1; i < splits; i++) s += part[i * stride + e];
+        s *= g.alpha;
+        p.c[e] = g.acc ? p.c[e] + s : s;
+    }
+}
+
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// The tiles.  A step (32 k) of each, measured with one workgroup to a CU and
+// with the chip full (power then holds the clock near 1.8 of 2.4 GHz):
+//   256 x 128, 8 waves of 64 x 64, 1 workgroup to a CU:  1.7-1.8 / 2.3 us
+//   128 x 128, 8 waves of 32 x 64, 1 to a CU:            0.93 / 1.15 us
+//   64 x 64, 4 waves of 32 x 32, 3 to a CU:              0.45 / 1.2 us for three
+// The larger the tile, the fewer times an operand is split and the fewer LDS
+// bytes a product takes; the smaller, the better a small grid fills the CUs.
+// (128 x 64 with two workgroups to a CU, 128 x 128 in steps of 16 k with two
+// or three, and 256 x 256 were never the best.)
+enum Tile { kTile256, kTile128, kTile64, kNumTiles };
+constexpr int kTileM[kNumTiles] = {256, 128, 64}, kTileN[kNumTiles] = {128, 128, 64};
+constexpr int kCus = 256;
+
+// Modelled time of one launch, in us: rounds over the CUs of a workgroup's steps
+// plus its first loads and stores.
+double tile_time(Tile tile, long wgs, int steps) {
+    const double rounds = (double)((wgs + kCus - 1) / kCus);
+    if (tile == kTile256) return rounds * (steps * (wgs > kCus / 2 ? 2.1 : 1.8) + 5.0);
+    if (tile == kTile128) return rounds * (steps * (wgs > kCus / 2 ? 1.1 : 0.95) + 4.0);
+    return rounds < 2 ? steps * 0.45 + 3.0 : rounds * steps * 0.41 + 3.0;
+}
+
+template <bool AS, bool BS>
+void launch_tile(const GemmArgs& g, Tile tile, bool far, int grid, hipStream_t st) {
+    if (far)
+        gemm_f32_kernel<AS, BS, 64, 64, 256, uint64_t><<<grid, 256, 0, st>>>(g);
+    else if (tile == kTile256)
+        gemm_f32_kernel<AS, BS, 256, 128, 512><<<grid, 512, 0, st>>>(g);
+    else if (tile == kTile128)
+        gemm_f32_kernel<AS, BS, 128, 128, 512><<<grid, 512, 0, st>>>(g);
+    else
+        gemm_f32_kernel<AS, BS, 64, 64, 256><<<grid, 256, 0, st>>>(g);
+}
+
+}  // namespace
+
+hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipStream_t st) {
+    GemmArgs g{};
+    int steps = 1;
+    long cols = 0;
+    bool far = false;  // offsets within a tile past 32 bits
+    for (int i = 0; i < in.npr; i++) {
+        const GemmProblem& p = g.pr[i] = in.pr[i];
+        const int n = all_steps(p);
+        if (n > steps) steps = n;
+        cols += p.n;
+        for (int s = 0; s < p.nseg; s++) {
+            const long lda = in.a_strided ? 0 : p.seg[s].lda, ldb = in.b_strided ? 0 : p.seg[s].ldb;
+            far |= (lda > ldb ? lda : ldb) >= 1L << 22;  // 256 rows of 4 bytes below 2^32
+        }
+    }
+    g.npr = in.npr, g.m = in.m, g.acc = in.acc, g.alpha = in.alpha;
+    // The tile and split of the least modelled time.  A split's partial sums
+    // cost their pass through memory (4 bytes written and read, at 4 TB/s)
+    // and a launch; a split is at least four steps.
+    Tile tile = kTile64;
+    int splits = 1;
+    double best = -1.0;
+    for (int ti = far ? kTile64 : kTile256; ti < kNumTiles; ti++) {
+        int nt = 0;
+        for (int i = 0; i < g.npr; i++) nt += cdiv(g.pr[i].n, kTileN[ti]);
+        const long tiles = (long)cdiv(g.m, kTileM[ti]) * nt;
+        for (int sp = 1; sp <= 32 && sp * 4 <= steps + 3; sp++) {
+            const int per = cdiv(steps, sp);
+            if (cdiv(steps, per) != sp) continue;
+            if (sp > 1 && (size_t)(sp * cols) * g.m > ws_floats) break;
+            double t = tile_time((Tile)ti, tiles * sp, per);
+            if (sp > 1) t += 4.0 + (2.0 * sp + 1.0) * cols * g.m * 4.0 / 4e6;
+            if (best < 0 || t < best) best = t, tile = (Tile)ti, splits = sp;
+        }
+    }
+    g.per = cdiv(steps, splits);
+    splits = cdiv(steps, g.per);
+    g.mt = cdiv(g.m, kTileM[tile]);
+    for (int i = 0; i < g.npr; i++) g.nt += cdiv(g.pr[i].n, kTileN[tile]);
+    g.part = splits > 1 ? ws : nullptr;
+    // Neighbouring workgroups share an XCD's L2: run over n first where B is
+    // the smaller operand (each XCD then reads all of it), else over m.
+    g.n_inner = cols < g.m;
+    const long grid = (long)g.mt * g.nt * splits;
+    if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
+    if (in.a_strided)
+        launch_tile<true, true>(g, tile, far, (int)grid, st);
+    else if (in.b_strided)
+        launch_tile<false, true>(g, tile, far, (int)grid, st);
+    else
+        launch_tile<false, false>(g, tile, far, (int)grid, st);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || splits == 1) return e;
+    int widest = 0;
+    for (int i = 0; i < g.npr; i++) widest = g.pr[i].n > widest ? g.pr[i].n : widest;
+    const long blocks = ((long)g.m * widest + 255) / 256;
+    gemm_f32_reduce_kernel<<<dim3((unsigned)(blocks < 2048 ? blocks : 2048), g.npr), 256, 0, st>>>(g, splits, cols);
+    return hipGetLastError();
+}
+
+}  // namespace cfattn

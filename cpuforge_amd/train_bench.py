@@ -23,7 +23,7 @@ the tier's metric. It follows the reference's `cpuforge bench-train`
 The attention of every layer is `cpuforge_amd.layer.layer_attention`, the
 fused RoPE + attention kernels.  With `backend="cfops"` (the default) every
 other op of the step also runs through libcfattn.so (include/cfops.h, via
-`cpuforge_amd.autograd`): RMSNorm, the LoRA linears (hipBLASLt GEMMs), the
+`cpuforge_amd.autograd`): RMSNorm, the LoRA linears, the
 SwiGLU gate and the LM head with its cross-entropy, whose [t, vocab] logits
 are formed a chunk of rows at a time.  Only the embedding gather and the
 residual adds stay torch ops.  `backend="torch"` runs those ops as plain torch
@@ -237,7 +237,7 @@ class SmolLM:
 def capture_step(model: SmolLM, tokens, targets, warmup: int = 2):
     """The training step (every trained parameter's .grad reset, forward,
     loss, backward) captured in a HIP graph: `warmup` eager steps on a side
-    stream (the capture recipe: the library's scratch, the GEMM plans and
+    stream (the capture recipe: the library's scratch and
     torch's allocations are made there), then the capture.  Returns the graph
     and the loss tensor its replays write; each replay leaves the step's
     gradients in the parameters' .grad.  Needs the cfops backend with
@@ -270,7 +270,7 @@ def train_tok_s(batch: int = 8, seq: int = 512, layers: int = 30, rank: int = 16
                 dtype=torch.float32, attn_dtype=None, device="cuda", backend: str = "cfops",
                 warmup: int = 3, graph: bool = False) -> dict:
     """Build the model, run `warmup` untimed steps (the first allocates the
-    library's scratch and plans; the clock settles over the next ones),
+    library's scratch; the clock settles over the next ones),
     then time `steps` forward+backward passes; returns tok/s and the step
     time.  With `graph` (cfops backend) the step is captured in a HIP graph
     after the warm-up steps and the timed steps are its replays: the same

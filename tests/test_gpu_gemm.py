@@ -1,0 +1,85 @@
+"""GPU tests of the f32 GEMM kernels (cpuforge_amd/csrc/gemm_f32.hip) at the
+edges of their tiles (64, 128, 256), steps (32 k) and splits, against float64,
+and on inputs whose bf16 pieces are not finite."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def product(kind, a, b, c, acc):
+    from cpuforge_amd import ops as P
+    m, n, k = c.shape[0], c.shape[1], a.shape[1]
+    if kind == "nn":
+        P.matmul_nn(a.contiguous(), b.contiguous(), c, m, k, n, acc)
+    elif kind == "nt":
+        P.matmul_nt(a.contiguous(), b.t().contiguous(), c, m, k, n, acc)
+    else:
+        P.matmul_tn(a.t().contiguous(), b.contiguous(), c, m, k, n, acc)
+    return c
+
+
+def check(kind, m, k, n, acc=False, scale_a=1.0, seed=1):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    a = torch.randn(m, k, generator=g, device=DEV) * scale_a
+    b = torch.randn(k, n, generator=g, device=DEV)
+    c0 = torch.randn(m, n, generator=g, device=DEV)
+    c = product(kind, a, b, c0.clone() if acc else torch.full((m, n), float("nan"), device=DEV), acc)
+    want = a.double() @ b.double() + (c0.double() if acc else 0)
+    # Sums in f32: at most one rounding of the partial sum per term (six per 16
+    # in one instruction chain, plus the splits' sums and the last one), each
+    # 2^-24 of it; the products left out are 2^-26 of |a b|.
+    bound = 2.0 ** -24 * (k + 8) * (a.abs().double() @ b.abs().double()) + 2.0 ** -22 * want.abs()
+    err = (c.double() - want).abs()
+    assert bool((err <= bound).all()), (kind, m, k, n, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (63, 7, 65), (64, 8, 64), (65, 31, 63), (127, 32, 129), (129, 33, 127),
+                                   (257, 100, 130), (255, 64, 383), (1, 1537, 300), (70, 4099, 5), (300, 1333, 501),
+                                   (4096, 96, 576), (4100, 160, 700), (2048, 1000, 2050)])
+def test_gemm_edges_match_f64(kind, m, k, n):
+    print(kind, m, k, n, flush=True)
+    check(kind, m, k, n)
+    check(kind, m, k, n, acc=True)
+
+
+def test_gemm_rows_longer_than_32_bit_offsets():
+    """A row stride of more than 2^22 values: 256 rows of it pass 2^32 bytes."""
+    check("nt", 65, (1 << 22) + 5, 3)
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+def test_gemm_small_and_large_magnitudes(kind):
+    """Inputs whose low pieces are bf16 subnormals keep their products'
+    accuracy; inputs near the f32 maximum round to infinity in bf16 and take
+    the f32 recomputation."""
+    check(kind, 70, 96, 66, scale_a=2.0 ** -108)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a = torch.randn(70, 96, generator=g, device=DEV)
+    b = torch.randn(96, 66, generator=g, device=DEV) * 2.0 ** -20
+    a[5, 7] = 3.4028e38  # rounds to infinity in bf16
+    c = product(kind, a, b, torch.empty(70, 66, device=DEV), False)
+    want = a.double() @ b.double()
+    assert bool(torch.isfinite(c).all())
+    bound = 2.0 ** -24 * 104 * (a.abs().double() @ b.abs().double())
+    assert bool(((c.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+def test_gemm_infinities_and_nan_are_f32s(kind):
+    """What f32 arithmetic gives where an input is infinite or NaN: the same
+    infinities and NaN, the other outputs untouched by them."""
+    a = np.ones((70, 40), np.float32)
+    b = np.ones((40, 66), np.float32)
+    a[3, 2], a[9, 39], a[65, 0] = np.inf, np.nan, -np.inf
+    b[5, 1], b[2, 4] = np.inf, 0.0
+    with np.errstate(invalid="ignore"):
+        want = a @ b
+    c = product(kind, torch.from_numpy(a).to(DEV), torch.from_numpy(b).to(DEV), torch.empty(70, 66, device=DEV), False)
+    got = c.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.array_equal(got[ok], want[ok])
