@@ -38,6 +38,12 @@ class PrologueC(C.Structure):
                 ("eps", C.c_float)]
 
 
+class LinearC(C.Structure):
+    """`cfops_linear` (include/cfops.h)."""
+    _fields_ = [("w", _vp), ("lora_a", _vp), ("lora_b", _vp), ("lora_scale", C.c_float), ("out", _sz), ("rank", _sz),
+                ("y", _vp), ("xs", _vp), ("dy", _vp), ("gw", _vp), ("ga", _vp), ("gb", _vp)]
+
+
 SIGNATURES = {
     "cfattn_create": (C.c_int, [C.c_int, C.POINTER(_vp)]),
     "cfattn_destroy": (C.c_int, [_vp]),
@@ -86,6 +92,8 @@ SIGNATURES = {
     "cfops_set_head_chunk_limit": (C.c_int, [_vp, _sz]),
     "cfops_linear_forward": (C.c_int, [_vp] * 5 + [C.c_float] + [_sz] * 4 + [_vp] * 3),
     "cfops_linear_backward": (C.c_int, [_vp] * 7 + [C.c_float] + [_sz] * 4 + [_vp] * 5),
+    "cfops_linears_forward": (C.c_int, [_vp, _vp, _sz, _sz, C.POINTER(LinearC), _sz, _vp]),
+    "cfops_linears_backward": (C.c_int, [_vp, _vp, _sz, _sz, _vp, C.POINTER(LinearC), _sz, C.c_int, _vp]),
     "cfops_adamw_update": (C.c_int, [_vp] * 5 + [_sz, C.c_uint64] + [C.c_float] * 5 + [_vp]),
     # include/cfio.h
     "cfio_bf16_to_f32": (C.c_int, [_vp, _vp, _vp, _sz, _vp]),

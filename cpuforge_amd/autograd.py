@@ -28,6 +28,13 @@ def _zeros(*likes):
     return out
 
 
+def _empty(*likes):
+    """_zeros without the fill, for buffers an op overwrites."""
+    sizes = [t.numel() if t is not None else 0 for t in likes]
+    flat = torch.empty(sum(sizes), device=next(t for t in likes if t is not None).device, dtype=torch.float32)
+    return [None if t is None else v.view(t.shape) for t, v in zip(likes, flat.split(sizes))]
+
+
 class RMSNormFn(torch.autograd.Function):
     """y = rmsnorm(x, w) over the last dim (crates/core/src/ops/rmsnorm.rs)."""
 
@@ -70,56 +77,29 @@ class SiluMulFn(torch.autograd.Function):
         return dg, du
 
 
-class LinearFn(torch.autograd.Function):
-    """y = x W^T (+ scale (x A^T) B^T) (crates/model/src/linear.rs:56-91)."""
-
-    @staticmethod
-    def forward(ctx, x, w, a, b, scale: float):
-        inn, out = w.shape[1], w.shape[0]
-        x2 = _flat(x, inn)
-        t = x2.shape[0]
-        y = torch.empty(t, out, device=x.device, dtype=torch.float32)
-        xs = torch.empty(t, a.shape[0], device=x.device, dtype=torch.float32) if a is not None else None
-        P.linear_forward(x2, w, t, inn, out, y, a, b, scale, xs)
-        ctx.save_for_backward(x2, xs, w, a, b)
-        ctx.scale = scale
-        return y.view(*x.shape[:-1], out)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x2, xs, w, a, b = ctx.saved_tensors
-        t, inn = x2.shape
-        out = w.shape[0]
-        need = ctx.needs_input_grad
-        dx, gw, ga, gb = _zeros(x2, w if need[1] else None, a if a is not None and need[2] else None,
-                                b if b is not None and need[3] else None)
-        P.linear_backward(x2, xs, _flat(dy, out), w, t, inn, out, dx, gw, ga, gb, a, b, ctx.scale)
-        return dx.view(*dy.shape[:-1], inn), gw, ga, gb, None
-
-
-class SharedInputLinearsFn(torch.autograd.Function):
-    """Several linears of one input (the q/k/v projections of a layer, or its
-    gate and up projections): each forward as LinearFn, and one backward that
-    accumulates every linear's dx into one zeroed buffer in order, as the
-    reference's Layer::backward does for dn2 (crates/model/src/layer.rs:170-171)
-    and dn1 (layer.rs:208-211).  `flat` holds (w, a, b) per linear."""
+class LinearsFn(torch.autograd.Function):
+    """y = x W^T (+ scale (x A^T) B^T) (crates/model/src/linear.rs:56-91) of one
+    linear or of several of one input (the q/k/v projections of a layer, or its
+    gate and up projections), whose dx is one sum, as the reference's
+    Layer::backward forms dn2 (crates/model/src/layer.rs:170-171) and dn1
+    (layer.rs:208-211).  `flat` holds (w, a, b) per linear."""
 
     @staticmethod
     def forward(ctx, x, scales, *flat):
         inn = flat[0].shape[1]
         x2 = _flat(x, inn)
         t = x2.shape[0]
-        ys, xss = [], []
+        lins, ys, xss = [], [], []
         for i, scale in enumerate(scales):
             w, a, b = flat[3 * i:3 * i + 3]
             y = torch.empty(t, w.shape[0], device=x.device, dtype=torch.float32)
             xs = torch.empty(t, a.shape[0], device=x.device, dtype=torch.float32) if a is not None else None
-            P.linear_forward(x2, w, t, inn, w.shape[0], y, a, b, scale, xs)
+            lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, y=y, xs=xs))
             ys.append(y.view(*x.shape[:-1], w.shape[0]))
             xss.append(xs)
-        ctx.save_for_backward(x2, *flat, *[xs if xs is not None else torch.empty(0) for xs in xss])
+        P.linears_forward(x2, t, inn, lins)
+        ctx.save_for_backward(x2, *flat, *xss)
         ctx.scales = scales
-        ctx.has_xs = [xs is not None for xs in xss]
         ctx.shape = x.shape
         return tuple(ys)
 
@@ -129,21 +109,23 @@ class SharedInputLinearsFn(torch.autograd.Function):
         n = len(ctx.scales)
         x2, flat, xss = saved[0], saved[1:1 + 3 * n], saved[1 + 3 * n:]
         t, inn = x2.shape
-        need = ctx.needs_input_grad[2:]
-        likes = [x2]
-        for i in range(3 * n):
-            likes.append(flat[i] if flat[i] is not None and need[i] else None)
-        bufs = _zeros(*likes)
-        dx, grads = bufs[0], bufs[1:]
+        need = [ctx.needs_input_grad[0]] + list(ctx.needs_input_grad[2:])
+        if not any(need):
+            return (None,) * (2 + 3 * n)
+        # Everything is overwritten, except where an output was not used: its
+        # linear's gradients stay zero.
+        likes = [x if f else None for x, f in zip((x2, *flat), need)]
+        dx, *grads = _zeros(*likes) if any(dy is None for dy in dys) else _empty(*likes)
+        lins = []
         for i, scale in enumerate(ctx.scales):
             w, a, b = flat[3 * i:3 * i + 3]
             if dys[i] is None:
                 continue
             gw, ga, gb = grads[3 * i:3 * i + 3]
-            xs = xss[i] if ctx.has_xs[i] else None
-            P.linear_backward(x2, xs, _flat(dys[i], w.shape[0]), w, t, inn, w.shape[0], dx, gw, ga, gb, a, b,
-                              scale)
-        return (dx.view(ctx.shape), None, *grads)
+            lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, xs=xss[i], dy=_flat(dys[i], w.shape[0]), gw=gw,
+                             ga=ga, gb=gb))
+        P.linears_backward(x2, t, inn, dx, lins, acc=False)
+        return (None if dx is None else dx.view(ctx.shape), None, *grads)
 
 
 class LMHeadCEFn(torch.autograd.Function):
@@ -205,14 +187,14 @@ def silu_mul(g, u):
 
 
 def linear(x, w, a=None, b=None, scale=1.0):
-    return LinearFn.apply(x, w, a, b, scale)
+    return LinearsFn.apply(x, (float(scale),), w, a, b)[0]
 
 
 def shared_input_linears(x, specs):
     """[(w, a, b, scale), ...] -> the linears' outputs for input x, with one
-    accumulated dx in the backward."""
+    dx in the backward."""
     flat = [t for w, a, b, _ in specs for t in (w, a, b)]
-    return SharedInputLinearsFn.apply(x, tuple(float(s) for *_, s in specs), *flat)
+    return LinearsFn.apply(x, tuple(float(s) for *_, s in specs), *flat)
 
 
 def lm_head_ce(hn, head, targets):

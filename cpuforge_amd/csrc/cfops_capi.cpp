@@ -24,10 +24,18 @@ constexpr size_t kGemmWorkspace = (size_t)32 << 20;
 
 bool fits_int(size_t x) { return x <= (size_t)INT_MAX; }
 
-// Row-major C[m,n] = alpha * op(A) op(B) (+ C when acc), as matmul.rs's
+int launch_gemm(cfattn_ctx* c, const cfattn::GemmF32& g, hipStream_t st) {
+    int rc = CFATTN_OK;
+    float* ws = static_cast<float*>(slot(c, cfattn_ctx::OPS_WS, kGemmWorkspace, &rc));
+    if (!ws) return rc;
+    CF_HIP(c, cfattn::launch_gemm_f32(g, ws, kGemmWorkspace / sizeof(float), st), "GEMM launch");
+    return CFATTN_OK;
+}
+
+// Row-major C[m,n] = op(A) op(B) (+ C when acc), as matmul.rs's
 // matmul_nn / matmul_nt / matmul_tn (core/src/matmul.rs:127-147).
-int gemm(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, size_t m, size_t k, size_t n,
-         float alpha, bool acc, hipStream_t st) {
+int gemm(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, size_t m, size_t k, size_t n, bool acc,
+         hipStream_t st) {
     if (m == 0 || n == 0) return CFATTN_OK;
     if (!fits_int(m) || !fits_int(n) || !fits_int(k))
         return fail(c, CFATTN_ERR_UNSUPPORTED, "GEMM dimension above 2^31 (m=%zu, k=%zu, n=%zu)", m, k, n);
@@ -37,15 +45,84 @@ int gemm(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, si
     }
     if (kind != CFOPS_NN && kind != CFOPS_NT && kind != CFOPS_TN)
         return fail(c, CFATTN_ERR_ARG, "unknown matmul kind %d", kind);
-    int rc = CFATTN_OK;
-    float* ws = static_cast<float*>(slot(c, cfattn_ctx::OPS_WS, kGemmWorkspace, &rc));
-    if (!ws) return rc;
     cfattn::GemmF32 g;
-    g.npr = 1, g.m = (int)m, g.acc = acc, g.alpha = alpha;
+    g.npr = 1, g.m = (int)m, g.acc = acc;
     g.a_strided = kind == CFOPS_TN, g.b_strided = kind != CFOPS_NT;
     g.pr[0].nseg = 1, g.pr[0].c = out, g.pr[0].n = (int)n;
     g.pr[0].seg[0] = {a, b, (long)(kind == CFOPS_TN ? m : k), (long)(kind == CFOPS_NT ? k : n), (int)k};
-    CF_HIP(c, cfattn::launch_gemm_f32(g, ws, kGemmWorkspace / sizeof(float), st), "GEMM launch");
+    return launch_gemm(c, g, st);
+}
+
+int check_linears(cfattn_ctx* c, size_t t, size_t in, const cfops_linear* lin, size_t n) {
+    if (!fits_int(t) || !fits_int(in)) return fail(c, CFATTN_ERR_UNSUPPORTED, "t=%zu, in=%zu above 2^31", t, in);
+    for (size_t i = 0; i < n; i++)
+        if (!fits_int(lin[i].out) || (lin[i].lora_a && !fits_int(lin[i].rank)))
+            return fail(c, CFATTN_ERR_UNSUPPORTED, "out=%zu, rank=%zu above 2^31", lin[i].out, lin[i].rank);
+    return CFATTN_OK;
+}
+
+// Linear::forward (linear.rs:58-69) of up to kGemmProblems linears of one
+// input: xs_i = scale_i x A_i^T in one launch, then y_i = [x xs_i] [W_i B_i]^T in one.
+int linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, const cfops_linear* lin, size_t n,
+                    hipStream_t st) {
+    cfattn::LoraDown d;
+    cfattn::GemmF32 g;
+    d.t = g.m = (int)t;
+    for (size_t i = 0; i < n; i++) {
+        const cfops_linear& l = lin[i];
+        if (l.lora_a)
+            d.job[d.njobs++] = {x, l.lora_a, l.xs, l.lora_scale, (int)in, (int)l.rank};
+        if (l.out == 0) continue;
+        cfattn::GemmProblem& p = g.pr[g.npr++];
+        p.c = l.y, p.n = (int)l.out;
+        p.seg[p.nseg++] = {x, l.w, (long)in, (long)in, (int)in};
+        if (l.lora_a) p.seg[p.nseg++] = {l.xs, l.lora_b, (long)l.rank, (long)l.rank, (int)l.rank};
+    }
+    CF_HIP(c, cfattn::launch_lora_down(d, true, st), "lora launch");
+    return g.npr ? launch_gemm(c, g, st) : CFATTN_OK;
+}
+
+// Linear::backward (linear.rs:75-90) of up to kGemmProblems linears of one
+// input: dxa_i = scale_i dy_i B_i in one launch; dx (+)= [dy_1 dxa_1 dy_2 ..]
+// [W_1; A_1; W_2; ..] in one; the adapters' gradients in two.
+int linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin, size_t n,
+                     bool acc_dx, bool acc, hipStream_t st) {
+    cfattn::LoraDown d;
+    cfattn::GemmF32 g;
+    cfattn::LoraGrad lg;
+    int rc = CFATTN_OK;
+    size_t dxa_floats = 0;
+    for (size_t i = 0; i < n; i++) dxa_floats += lin[i].lora_a ? t * lin[i].rank : 0;
+    float* dxa = nullptr;
+    if (dxa_floats) {
+        dxa = static_cast<float*>(slot(c, cfattn_ctx::OPS_DXA, dxa_floats * sizeof(float), &rc));
+        if (!dxa) return rc;
+    }
+    d.t = g.m = lg.t = (int)t;
+    g.b_strided = true, g.acc = acc_dx, lg.acc = acc;
+    g.npr = 1, g.pr[0].c = dx, g.pr[0].n = (int)in;
+    for (size_t i = 0; i < n; i++) {
+        const cfops_linear& l = lin[i];
+        cfattn::GemmSeg* seg = g.pr[0].seg;
+        seg[g.pr[0].nseg++] = {l.dy, l.w, (long)l.out, (long)in, (int)l.out};
+        if (!l.lora_a) continue;
+        if (dx || l.ga) {
+            d.job[d.njobs++] = {l.dy, l.lora_b, dxa, l.lora_scale, (int)l.out, (int)l.rank};
+            seg[g.pr[0].nseg++] = {dxa, l.lora_a, (long)l.rank, (long)in, (int)l.rank};
+        }
+        if (l.gb && l.out) lg.job[lg.njobs++] = {l.dy, l.xs, l.gb, (int)l.out, (int)l.rank, 0, 0};
+        if (l.ga && in) lg.job[lg.njobs++] = {x, dxa, l.ga, (int)in, (int)l.rank, 1, 0};
+        dxa += t * l.rank;
+    }
+    CF_HIP(c, cfattn::launch_lora_down(d, false, st), "lora launch");
+    if (dx && in) CF_TRY(launch_gemm(c, g, st));
+    for (size_t i = 0; i < n; i++)
+        if (lin[i].gw) CF_TRY(gemm(c, CFOPS_TN, lin[i].dy, x, lin[i].gw, lin[i].out, t, in, acc, st));
+    if (lg.njobs == 0) return CFATTN_OK;
+    lg.part = static_cast<float*>(
+        slot(c, cfattn_ctx::OPS_LORA, cfattn::lora_grad_plan(lg) * sizeof(float), &rc));
+    if (!lg.part) return rc;
+    CF_HIP(c, cfattn::launch_lora_grad(lg, st), "lora launch");
     return CFATTN_OK;
 }
 
@@ -94,7 +171,7 @@ int cfops_matmul(cfattn_ctx* c, int kind, const float* a, const float* b, float*
                  int acc, void* stream) {
     CF_LOCK(c);
     if ((m && n && !out) || (m && n && k && (!a || !b))) return fail(c, CFATTN_ERR_ARG, "null buffer");
-    return gemm(c, kind, a, b, out, m, k, n, 1.0f, acc != 0, to_stream(stream));
+    return gemm(c, kind, a, b, out, m, k, n, acc != 0, to_stream(stream));
 }
 
 int cfops_rmsnorm_forward(cfattn_ctx* c, const float* x, const float* w, float* y, float* rstd, size_t rows,
@@ -187,12 +264,12 @@ static int lm_head_ce_queue(cfattn_ctx* c, const float* hn, const float* head, c
     for (size_t r0 = 0; r0 < t; r0 += chunk) {
         const size_t nr = t - r0 < chunk ? t - r0 : chunk;
         // logits = hn . head^T (model.rs:438), then dlogits in place.
-        CF_TRY(gemm(c, CFOPS_NT, hn + r0 * d, head, logits, nr, d, vocab, 1.0f, false, st));
+        CF_TRY(gemm(c, CFOPS_NT, hn + r0 * d, head, logits, nr, d, vocab, false, st));
         CF_HIP(c, cfattn::launch_ce_rows(logits, targets, logits, row_loss, r0, nr, vocab, misc, st),
                "cross-entropy launch");
         // dhn = dlogits . head (model.rs:454, overwritten); dhead += dlogits^T . hn (:457).
-        CF_TRY(gemm(c, CFOPS_NN, logits, head, dhn + r0 * d, nr, vocab, d, 1.0f, false, st));
-        if (dhead) CF_TRY(gemm(c, CFOPS_TN, logits, hn + r0 * d, dhead, vocab, nr, d, 1.0f, true, st));
+        CF_TRY(gemm(c, CFOPS_NN, logits, head, dhn + r0 * d, nr, vocab, d, false, st));
+        if (dhead) CF_TRY(gemm(c, CFOPS_TN, logits, hn + r0 * d, dhead, vocab, nr, d, true, st));
     }
     CF_HIP(c, cfattn::launch_ce_finish(targets, row_loss, t, misc, st), "cross-entropy launch");
     return CFATTN_OK;
@@ -238,30 +315,11 @@ int cfops_linear_forward(cfattn_ctx* c, const float* x, const float* w, const fl
     if (t == 0 || out == 0) return CFATTN_OK;
     if (!x || !w || !y) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (lora_a && (!lora_b || !xs || rank == 0)) return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
-    const hipStream_t st = to_stream(stream);
-    // linear.rs:58-69.  With an adapter on the streaming kernels' shapes the
-    // adapter is folded into the weight, y = x (W + scale B A)^T in one GEMM
-    // (the same sum, rounded once per element instead of twice), and xs is
-    // formed beside it for the backward.
-    const void* ptrs[] = {x, lora_a, lora_b, xs, w};
-    if (lora_a && cfattn::lora_fused_applies(rank, t, in, out, ptrs, 5)) {
-        int rc = CFATTN_OK;
-        float* part = static_cast<float*>(
-            slot(c, cfattn_ctx::OPS_LORA, cfattn::lora_partial_floats(rank, t, in, out) * sizeof(float), &rc));
-        if (!part) return rc;
-        float* weff = static_cast<float*>(slot(c, cfattn_ctx::OPS_WEFF, out * in * sizeof(float), &rc));
-        if (!weff) return rc;
-        CF_HIP(c, cfattn::launch_lora_merge(rank, w, lora_a, lora_b, lora_scale, out, in, weff, st),
-               "lora merge launch");
-        CF_TRY(gemm(c, CFOPS_NT, x, weff, y, t, in, out, 1.0f, false, st));
-        CF_HIP(c, cfattn::launch_lora_fwd(rank, x, lora_a, lora_b, lora_scale, t, in, out, nullptr, xs, part, st),
-               "lora forward launch");
-        return CFATTN_OK;
-    }
-    CF_TRY(gemm(c, CFOPS_NT, x, w, y, t, in, out, 1.0f, false, st));
-    if (!lora_a) return CFATTN_OK;
-    CF_TRY(gemm(c, CFOPS_NT, x, lora_a, xs, t, in, rank, lora_scale, false, st));
-    return gemm(c, CFOPS_NT, xs, lora_b, y, t, rank, out, 1.0f, true, st);
+    cfops_linear l{};
+    l.w = w, l.lora_a = lora_a, l.lora_b = lora_b, l.lora_scale = lora_scale, l.out = out, l.rank = rank;
+    l.y = y, l.xs = xs;
+    CF_TRY(check_linears(c, t, in, &l, 1));
+    return linears_forward(c, x, t, in, &l, 1, to_stream(stream));
 }
 
 int cfops_linear_backward(cfattn_ctx* c, const float* x, const float* xs, const float* dy, const float* w,
@@ -271,39 +329,49 @@ int cfops_linear_backward(cfattn_ctx* c, const float* x, const float* xs, const 
     if (t == 0) return CFATTN_OK;
     if (!x || !dy || !w || !dx) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (lora_a && (!lora_b || !xs || rank == 0)) return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
-    const hipStream_t st = to_stream(stream);
-    // linear.rs:75-90.  With an adapter on the streaming kernels' shapes,
-    // dx += dy (W + scale B A) in one GEMM (the forward's folded weight),
-    // and the adapter kernels form dxa = scale dy B and the adapter's
-    // gradients only.
-    int rc = CFATTN_OK;
-    const void* ptrs[] = {x, xs, dy, lora_a, lora_b, w};
-    if (lora_a && cfattn::lora_fused_applies(rank, t, in, out, ptrs, 6)) {
-        float* weff = static_cast<float*>(slot(c, cfattn_ctx::OPS_WEFF, out * in * sizeof(float), &rc));
-        if (!weff) return rc;
-        CF_HIP(c, cfattn::launch_lora_merge(rank, w, lora_a, lora_b, lora_scale, out, in, weff, st),
-               "lora merge launch");
-        CF_TRY(gemm(c, CFOPS_NN, dy, weff, dx, t, out, in, 1.0f, true, st));
-        if (gw) CF_TRY(gemm(c, CFOPS_TN, dy, x, gw, out, t, in, 1.0f, true, st));
-        float* dxa = static_cast<float*>(slot(c, cfattn_ctx::OPS_DXA, t * rank * sizeof(float), &rc));
-        if (!dxa) return rc;
-        float* part = static_cast<float*>(
-            slot(c, cfattn_ctx::OPS_LORA, cfattn::lora_partial_floats(rank, t, in, out) * sizeof(float), &rc));
-        if (!part) return rc;
-        CF_HIP(c, cfattn::launch_lora_bwd(rank, x, xs, dy, lora_a, lora_b, lora_scale, t, in, out, nullptr, ga, gb,
-                                          dxa, part, st),
-               "lora backward launch");
-        return CFATTN_OK;
+    cfops_linear l{};
+    l.w = w, l.lora_a = lora_a, l.lora_b = lora_b, l.lora_scale = lora_scale, l.out = out, l.rank = rank;
+    l.xs = const_cast<float*>(xs), l.dy = dy, l.gw = gw, l.ga = lora_a ? ga : nullptr, l.gb = lora_a ? gb : nullptr;
+    CF_TRY(check_linears(c, t, in, &l, 1));
+    return linears_backward(c, x, t, in, dx, &l, 1, true, true, to_stream(stream));
+}
+
+int cfops_linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, const cfops_linear* lin, size_t n,
+                          void* stream) {
+    CF_LOCK(c);
+    if (t == 0 || n == 0) return CFATTN_OK;
+    if (!x || !lin) return fail(c, CFATTN_ERR_ARG, "null buffer");
+    for (size_t i = 0; i < n; i++) {
+        const cfops_linear& l = lin[i];
+        if (l.out && (!l.w || !l.y)) return fail(c, CFATTN_ERR_ARG, "null buffer");
+        if (l.lora_a && (!l.lora_b || !l.xs || l.rank == 0))
+            return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
     }
-    CF_TRY(gemm(c, CFOPS_NN, dy, w, dx, t, out, in, 1.0f, true, st));
-    if (gw) CF_TRY(gemm(c, CFOPS_TN, dy, x, gw, out, t, in, 1.0f, true, st));
-    if (!lora_a) return CFATTN_OK;
-    if (gb) CF_TRY(gemm(c, CFOPS_TN, dy, xs, gb, out, t, rank, 1.0f, true, st));
-    float* dxa = static_cast<float*>(slot(c, cfattn_ctx::OPS_DXA, t * rank * sizeof(float), &rc));
-    if (!dxa) return rc;
-    CF_TRY(gemm(c, CFOPS_NN, dy, lora_b, dxa, t, out, rank, lora_scale, false, st));
-    if (ga) CF_TRY(gemm(c, CFOPS_TN, dxa, x, ga, rank, t, in, 1.0f, true, st));
-    return gemm(c, CFOPS_NN, dxa, lora_a, dx, t, rank, in, 1.0f, true, st);
+    CF_TRY(check_linears(c, t, in, lin, n));
+    for (size_t i = 0; i < n; i += cfattn::kGemmProblems) {
+        const size_t m = n - i < (size_t)cfattn::kGemmProblems ? n - i : (size_t)cfattn::kGemmProblems;
+        CF_TRY(linears_forward(c, x, t, in, lin + i, m, to_stream(stream)));
+    }
+    return CFATTN_OK;
+}
+
+int cfops_linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin,
+                           size_t n, int acc, void* stream) {
+    CF_LOCK(c);
+    if (t == 0 || n == 0) return CFATTN_OK;
+    if (!x || !lin) return fail(c, CFATTN_ERR_ARG, "null buffer");
+    for (size_t i = 0; i < n; i++) {
+        const cfops_linear& l = lin[i];
+        if (!l.dy || !l.w) return fail(c, CFATTN_ERR_ARG, "null buffer");
+        if (l.lora_a && (!l.lora_b || !l.xs || l.rank == 0))
+            return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
+    }
+    CF_TRY(check_linears(c, t, in, lin, n));
+    for (size_t i = 0; i < n; i += cfattn::kGemmProblems) {
+        const size_t m = n - i < (size_t)cfattn::kGemmProblems ? n - i : (size_t)cfattn::kGemmProblems;
+        CF_TRY(linears_backward(c, x, t, in, dx, lin + i, m, acc || i > 0, acc != 0, to_stream(stream)));
+    }
+    return CFATTN_OK;
 }
 
 int cfops_adamw_update(cfattn_ctx* c, float* p, const float* g, float* m, float* v, size_t n, uint64_t t, float lr,

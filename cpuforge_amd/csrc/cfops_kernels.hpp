@@ -49,7 +49,7 @@ hipError_t launch_adamw(float* p, const float* g, float* m, float* v, size_t n, 
                         float eps, float weight_decay, float bc1, float bc2, hipStream_t st);
 
 // f32 GEMMs over a common row count m (gemm_f32.hip).  Problem i is
-//   C_i[m, n_i] (+)= alpha * (sum over its segments s of A_s B_s),
+//   C_i[m, n_i] (+)= sum over its segments s of A_s B_s,
 // the segments being runs of one long contraction (a base product and an
 // adapter's, or the products of several linears into one gradient).  A
 // element (row, k) is at a[row * lda + k], or a[k * lda + row] with
@@ -71,30 +71,42 @@ struct GemmF32 {
     GemmProblem pr[kGemmProblems];
     int npr = 0, m = 0;
     int acc = 0;  // 1: add to C, 0: overwrite it
-    float alpha = 1.0f;
     bool a_strided = false, b_strided = false;
 };
 // `ws` is scratch for the partial sums of a split contraction.
 hipError_t launch_gemm_f32(const GemmF32& g, float* ws, size_t ws_floats, hipStream_t st);
 
-// LoRA adapter products of Linear::forward / backward (linear.rs:56-91) as
-// streaming kernels (lora.hip), for ranks 4, 8 and 16 with 16-byte aligned
-// rows; `part` is scratch of lora_partial_floats floats for the per-chunk
-// partial sums, which are added in chunk order:
-//   forward:  xs = scale * x A^T (overwritten), y += xs B^T (y non-null);
-//   backward: dxa = scale * dy B (into `dxa`, t x rank), dx += dxa A (dx
-//             non-null), and when non-null gb += dy^T xs, ga += dxa^T x;
-//   merge:    weff = w + scale * B A ([out x in], w's layout), the base
-//             weight with the adapter folded in.
-constexpr int kLoraChunk = 64;  // tokens per partial sum of the gradients
-bool lora_fused_applies(size_t rank, size_t t, size_t in, size_t out, const void* const* ptrs, int nptr);
-size_t lora_partial_floats(size_t rank, size_t t, size_t in, size_t out);
-hipError_t launch_lora_fwd(size_t rank, const float* x, const float* a, const float* b, float scale, size_t t,
-                           size_t in, size_t out, float* y, float* xs, float* part, hipStream_t st);
-hipError_t launch_lora_merge(size_t rank, const float* w, const float* a, const float* b, float scale, size_t out,
-                             size_t in, float* weff, hipStream_t st);
-hipError_t launch_lora_bwd(size_t rank, const float* x, const float* xs, const float* dy, const float* a,
-                           const float* b, float scale, size_t t, size_t in, size_t out, float* dx, float* ga,
-                           float* gb, float* dxa, float* part, hipStream_t st);
+// LoRA adapter products of Linear::forward / backward (linear.rs:56-91) with
+// the rank as a dimension of the result (lora.hip), for up to kGemmProblems
+// linears over the same t tokens in one launch:
+//   down:  out = scale * src m^T (m [r x k], m_rows: xs = scale x A^T) or
+//          scale * src m (m [k x r]: dxa = scale dy B), out [t x r];
+//   grad:  out (+)= big^T small, [ncol x r] (gb from dy and xs), or its
+//          transpose [r x ncol] (ga from x and dxa).
+struct LoraDownJob {
+    const float *src, *m;
+    float* out;
+    float scale;
+    int k, r;
+};
+struct LoraDown {
+    LoraDownJob job[kGemmProblems];
+    int njobs = 0, t = 0;
+};
+hipError_t launch_lora_down(const LoraDown& g, bool m_rows, hipStream_t st);
+struct LoraGradJob {
+    const float *big, *small;
+    float* out;
+    int ncol, r, transposed;
+    long off;  // of its partial sums (set by lora_grad_plan)
+};
+struct LoraGrad {
+    LoraGradJob job[2 * kGemmProblems];
+    int njobs = 0, t = 0, acc = 1;
+    int chunks, tokens;     // set by lora_grad_plan
+    float* part = nullptr;  // scratch of as many floats as lora_grad_plan returns
+};
+size_t lora_grad_plan(LoraGrad& g);
+hipError_t launch_lora_grad(const LoraGrad& g, hipStream_t st);
 
 }  // namespace cfattn

@@ -49,7 +49,6 @@ struct GemmArgs {
     int mt, nt;          // tiles over m, and over all problems' n
     int per;             // k steps per split
     int n_inner;
-    float alpha;
     float* part;         // partial products of the splits, or null
 };
 
@@ -352,7 +351,6 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
         out = g.part + (split * cols + part_off) * g.m;
     }
     const bool add = g.acc && !g.part;
-    const float alpha = g.part ? 1.0f : g.alpha;
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
@@ -364,13 +362,12 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
                 const int row = mw + 32 * i + 8 * (r >> 2) + (r & 3);
                 if (row >= g.m) continue;
                 float* o = out + (long)row * p.n + col;
-                const float v = alpha * acc[i][j][r];
-                *o = add ? *o + v : v;
+                *o = add ? *o + acc[i][j][r] : acc[i][j][r];
             }
         }
 }
 
-// C (+)= alpha * (the splits' partial products, added in split order).
+// C (+)= the splits' partial products, added in split order.
 __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmArgs g, int splits, long cols) {
     const GemmProblem& p = g.pr[blockIdx.y];
     long off = 0;
@@ -380,7 +377,6 @@ __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmArgs g, 
     for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < mn; e += (long)gridDim.x * 256) {
         float s = part[e];
         for (int i = 1; i < splits; i++) s += part[i * stride + e];
-        s *= g.alpha;
         p.c[e] = g.acc ? p.c[e] + s : s;
     }
 }
@@ -438,7 +434,7 @@ hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipSt
             far |= (lda > ldb ? lda : ldb) >= 1L << 22;  // 256 rows of 4 bytes below 2^32
         }
     }
-    g.npr = in.npr, g.m = in.m, g.acc = in.acc, g.alpha = in.alpha;
+    g.npr = in.npr, g.m = in.m, g.acc = in.acc;
     // The tile and split of the least modelled time.  A split's partial sums
     // cost their pass through memory (4 bytes written and read, at 4 TB/s)
     // and a launch; a split is at least four steps.

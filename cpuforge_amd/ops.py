@@ -11,6 +11,7 @@ the holder of device memory and the current HIP stream:
     lm_head_ce                          crates/model/src/model.rs:436-457
       (lm_head_ce_dev: the same, its loss left in device memory)
     linear_forward / linear_backward    crates/model/src/linear.rs:56-91
+      (linears_forward / linears_backward: several linears of one input)
     adamw_update                        crates/train/src/optim.rs:9-30
 
 Misuse the reference would panic on raises `ShapeError` (an AssertionError);
@@ -204,6 +205,44 @@ def linear_backward(x, xs, dy, w, t, inn, out, dx, gw=None, ga=None, gb=None, lo
           _f32(w, "w", out * inn), _opt(lora_a, "lora_a", r * inn), _opt(lora_b, "lora_b", out * r),
           float(lora_scale), t, inn, out, r, _f32(dx, "dx", t * inn), _opt(gw, "gw", out * inn),
           _opt(ga, "ga", r * inn), _opt(gb, "gb", out * r), _stream())
+
+
+def _linears(lins, t, inn, forward):
+    """The cfops_linear array of `lins` (dicts; see linears_forward / _backward)."""
+    arr = (_lib.LinearC * len(lins))()
+    for c, li in zip(arr, lins):
+        w, a, b = li["w"], li.get("lora_a"), li.get("lora_b")
+        out = w.shape[0]
+        r = 0 if a is None else a.shape[0]
+        c.w, c.out, c.rank, c.lora_scale = _f32(w, "w", out * inn), out, r, float(li.get("scale", 1.0))
+        c.lora_a, c.lora_b = _opt(a, "lora_a", r * inn), _opt(b, "lora_b", out * r)
+        c.xs = _opt(li.get("xs"), "xs", t * r)
+        if forward:
+            c.y = _f32(li["y"], "y", t * out)
+        else:
+            c.dy = _f32(li["dy"], "dy", t * out)
+            c.gw = _opt(li.get("gw"), "gw", out * inn)
+            c.ga, c.gb = _opt(li.get("ga"), "ga", r * inn), _opt(li.get("gb"), "gb", out * r)
+    return arr
+
+
+def linears_forward(x, t, inn, lins, ctx: Context | None = None):
+    """linear_forward of several linears of one input x [t, inn] in the
+    launches of one.  Each is a dict of w [out, inn], y [t, out] (overwritten)
+    and, with an adapter, lora_a, lora_b, scale and xs [t, rank] (overwritten)."""
+    ctx = ctx or default_context()
+    _call(ctx, "cfops_linears_forward", _f32(x, "x", t * inn), t, inn, _linears(lins, t, inn, True), len(lins),
+          _stream())
+
+
+def linears_backward(x, t, inn, dx, lins, acc=True, ctx: Context | None = None):
+    """linear_backward of several linears of one input: dicts of w, dy, gw and,
+    with an adapter, lora_a, lora_b, scale, xs, ga and gb (None or absent:
+    frozen; dx None: x needs no gradient).  Adds to dx and the gradients, or
+    overwrites them with acc=False."""
+    ctx = ctx or default_context()
+    _call(ctx, "cfops_linears_backward", _f32(x, "x", t * inn), t, inn, _opt(dx, "dx", t * inn),
+          _linears(lins, t, inn, False), len(lins), int(acc), _stream())
 
 
 # ---------------------------------------------------------------- AdamW

@@ -99,21 +99,45 @@ int cfops_lm_head_ce_dev(cfattn_ctx* ctx, const float* hn, const float* head, co
 
 /* Linear::forward (linear.rs:56-71): y [t,out] = x [t,in] . W^T (overwritten),
  * W [out,in].  With an adapter (lora_a non-null; A [rank,in], B [out,rank]):
- * xs [t,rank] = scale * x . A^T (overwritten) and y += xs . B^T.  For ranks
- * 4, 8 and 16 with in and out multiples of 4 and 16-byte aligned operands,
- * y is formed as x . (W + scale * B . A)^T in one GEMM: the same sum,
- * rounded differently (within f32 rounding of the reference's). */
+ * xs [t,rank] = scale * x . A^T (overwritten) and y += xs . B^T, as more terms
+ * of the same sums (rounded once where the reference rounds twice). */
 int cfops_linear_forward(cfattn_ctx* ctx, const float* x, const float* w, const float* lora_a, const float* lora_b,
                          float lora_scale, size_t t, size_t in, size_t out, size_t rank, float* y, float* xs,
                          void* stream);
 /* Linear::backward (linear.rs:73-91): dx += dy . W; gw += dy^T . x when gw is
  * non-null; with an adapter gb += dy^T . xs (gb non-null), and with
- * dxa = scale * dy . B: ga += dxa^T . x (ga non-null) and dx += dxa . A
- * (on the forward's fast shapes: dx += dy . (W + scale * B . A) in one GEMM).
+ * dxa = scale * dy . B: ga += dxa^T . x (ga non-null) and dx += dxa . A.
  * NULL gradients are frozen tensors (the reference's empty LinGrad vectors). */
 int cfops_linear_backward(cfattn_ctx* ctx, const float* x, const float* xs, const float* dy, const float* w,
                           const float* lora_a, const float* lora_b, float lora_scale, size_t t, size_t in, size_t out,
                           size_t rank, float* dx, float* gw, float* ga, float* gb, void* stream);
+
+/* No reference counterpart: the linears of one input (a layer's q, k and v
+ * projections, its gate and up projections; layer.rs:98-102, 133-134) in the
+ * launches of one.  Fields of a linear the direction does not name are not
+ * read.  Forward: w, out, y and, with an adapter, lora_a, lora_b, lora_scale,
+ * rank, xs.  Backward: w, out, dy, gw and, with an adapter, lora_a, lora_b,
+ * lora_scale, rank, xs, ga, gb; dx NULL: x needs no gradient.  acc != 0 adds to
+ * dx and the gradients, as cfops_linear_backward does linear by linear; acc
+ * == 0 overwrites them. */
+typedef struct cfops_linear {
+    const float* w;
+    const float* lora_a;
+    const float* lora_b;
+    float lora_scale;
+    size_t out;
+    size_t rank;
+    float* y;
+    float* xs;
+    const float* dy;
+    float* gw;
+    float* ga;
+    float* gb;
+} cfops_linear;
+int cfops_linears_forward(cfattn_ctx* ctx, const float* x, size_t t, size_t in, const cfops_linear* lin, size_t n,
+                          void* stream);
+int cfops_linears_backward(cfattn_ctx* ctx, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin,
+                           size_t n, int acc, void* stream);
 
 /* adamw_update (optim.rs:9-30): one AdamW step of one tensor of n values,
  * t the 1-based step count; p, m, v updated in place.  Every product and sum
