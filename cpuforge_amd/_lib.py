@@ -95,6 +95,8 @@ SIGNATURES = {
     "cfops_linears_forward": (C.c_int, [_vp, _vp, _sz, _sz, C.POINTER(LinearC), _sz, _vp]),
     "cfops_linears_backward": (C.c_int, [_vp, _vp, _sz, _sz, _vp, C.POINTER(LinearC), _sz, C.c_int, _vp]),
     "cfops_adamw_update": (C.c_int, [_vp] * 5 + [_sz, C.c_uint64] + [C.c_float] * 5 + [_vp]),
+    "cfops_adamw_update_multi": (C.c_int, [_vp, _sz] + [C.POINTER(_vp)] * 4 + [C.POINTER(_sz), _fp, C.c_uint64]
+                                 + [C.c_float] * 4 + [_vp]),
     # include/cfio.h
     "cfio_bf16_to_f32": (C.c_int, [_vp, _vp, _vp, _sz, _vp]),
     "cfio_f16_to_f32": (C.c_int, [_vp, _vp, _vp, _sz, _vp]),

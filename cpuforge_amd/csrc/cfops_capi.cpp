@@ -376,14 +376,28 @@ int cfops_linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, f
 
 int cfops_adamw_update(cfattn_ctx* c, float* p, const float* g, float* m, float* v, size_t n, uint64_t t, float lr,
                        float beta1, float beta2, float eps, float weight_decay, void* stream) {
+    return cfops_adamw_update_multi(c, 1, &p, &g, &m, &v, &n, &weight_decay, t, lr, beta1, beta2, eps, stream);
+}
+
+int cfops_adamw_update_multi(cfattn_ctx* c, size_t count, float* const* p, const float* const* g, float* const* m,
+                             float* const* v, const size_t* n, const float* weight_decay, uint64_t t, float lr,
+                             float beta1, float beta2, float eps, void* stream) {
     CF_LOCK(c);
-    if (n == 0) return CFATTN_OK;
-    if (!p || !g || !m || !v) return fail(c, CFATTN_ERR_ARG, "null buffer");
+    if (count && (!p || !g || !m || !v || !n || !weight_decay)) return fail(c, CFATTN_ERR_ARG, "null array");
+    for (size_t i = 0; i < count; i++)
+        if (n[i] && (!p[i] || !g[i] || !m[i] || !v[i])) return fail(c, CFATTN_ERR_ARG, "null buffer");
+    cfattn::AdamwArgs a;
+    a.count = 0, a.lr = lr, a.beta1 = beta1, a.beta2 = beta2, a.eps = eps;
     // optim.rs:21-22: the bias corrections, `t as i32` as in the reference.
-    const float bc1 = 1.0f - powi_f32(beta1, (int)(int32_t)t);
-    const float bc2 = 1.0f - powi_f32(beta2, (int)(int32_t)t);
-    CF_HIP(c, cfattn::launch_adamw(p, g, m, v, n, lr, beta1, beta2, eps, weight_decay, bc1, bc2, to_stream(stream)),
-           "adamw launch");
+    a.bc1 = 1.0f - powi_f32(beta1, (int)(int32_t)t);
+    a.bc2 = 1.0f - powi_f32(beta2, (int)(int32_t)t);
+    for (size_t i = 0; i < count; i++) {
+        if (n[i]) a.t[a.count++] = {p[i], g[i], m[i], v[i], (long)n[i], weight_decay[i], 0, 0};
+        if (a.count == cfattn::kAdamwBatch || (i + 1 == count && a.count)) {
+            CF_HIP(c, cfattn::launch_adamw(a, to_stream(stream)), "adamw launch");
+            a.count = 0;
+        }
+    }
     return CFATTN_OK;
 }
 

@@ -43,10 +43,24 @@ hipError_t launch_ce_rows(const float* logits, const int64_t* targets, float* dl
                           size_t nrows, size_t vocab, void* misc, hipStream_t st);
 hipError_t launch_ce_finish(const int64_t* targets, const float* row_loss, size_t rows, void* misc, hipStream_t st);
 
-// One AdamW update (crates/train/src/optim.rs:9-30); bc1, bc2 are the bias
-// corrections 1 - beta^t, computed by the caller.
-hipError_t launch_adamw(float* p, const float* g, float* m, float* v, size_t n, float lr, float beta1, float beta2,
-                        float eps, float weight_decay, float bc1, float bc2, hipStream_t st);
+// One AdamW update (crates/train/src/optim.rs:9-30) of `count` tensors, none
+// empty; bc1, bc2 are the bias corrections 1 - beta^t, computed by the caller.
+constexpr int kAdamwBatch = 64;
+struct AdamwTensor {
+    float* p;
+    const float* g;
+    float *m, *v;
+    long n;
+    float weight_decay;
+    int vec;      // set by launch_adamw, as block0
+    long block0;
+};
+struct AdamwArgs {
+    AdamwTensor t[kAdamwBatch];
+    int count;
+    float lr, beta1, beta2, eps, bc1, bc2;
+};
+hipError_t launch_adamw(AdamwArgs a, hipStream_t st);
 
 // f32 GEMMs over a common row count m (gemm_f32.hip).  Problem i is
 //   C_i[m, n_i] (+)= sum over its segments s of A_s B_s,

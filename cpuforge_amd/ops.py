@@ -13,6 +13,7 @@ the holder of device memory and the current HIP stream:
     linear_forward / linear_backward    crates/model/src/linear.rs:56-91
       (linears_forward / linears_backward: several linears of one input)
     adamw_update                        crates/train/src/optim.rs:9-30
+      (adamw_update_multi: many tensors, optim.rs:48-61)
 
 Misuse the reference would panic on raises `ShapeError` (an AssertionError);
 library failures raise `CfattnError`.
@@ -252,3 +253,20 @@ def adamw_update(p, g, m, v, t, lr, beta1, beta2, eps, weight_decay, ctx: Contex
     n = p.numel()
     _call(ctx, "cfops_adamw_update", _f32(p, "p"), _f32(g, "g", n), _f32(m, "m", n), _f32(v, "v", n), n, int(t),
           float(lr), float(beta1), float(beta2), float(eps), float(weight_decay), _stream())
+
+
+def adamw_update_multi(ps, gs, ms, vs, t, lr, beta1, beta2, eps, weight_decays, ctx: Context | None = None):
+    """adamw_update of many tensors (no two overlapping), each with its own
+    weight decay, in few launches."""
+    ctx = ctx or default_context()
+    k = len(ps)
+    sizes = [x.numel() for x in ps]
+    arrs = []
+    for name, ts in (("p", ps), ("g", gs), ("m", ms), ("v", vs)):
+        for x, n in zip(ts, sizes):
+            # _f32's checks, spelled out once for the common case.
+            if not (x.is_cuda and x.dtype is torch.float32 and x.is_contiguous() and x.numel() == n):
+                _f32(x, name, n)
+        arrs.append((C.c_void_p * k)(*[x.data_ptr() for x in ts]))
+    _call(ctx, "cfops_adamw_update_multi", k, *arrs, (C.c_size_t * k)(*sizes), (C.c_float * k)(*weight_decays),
+          int(t), float(lr), float(beta1), float(beta2), float(eps), _stream())

@@ -30,12 +30,26 @@ class AdamW:
     @torch.no_grad()
     def update(self, model, lr: float) -> None:
         self.step += 1
+        ps, gs, ms, vs, decays = [], [], [], [], []
         for name, p in model.named_params():
             if not p.requires_grad:
                 continue
-            g = p.grad if p.grad is not None else torch.zeros_like(p)
-            if name not in self.state:
-                self.state[name] = (torch.zeros_like(p), torch.zeros_like(p))
-            m, v = self.state[name]
-            decay = 0.0 if "norm" in name else self.weight_decay
-            P.adamw_update(p, g.contiguous(), m, v, self.step, lr, self.beta1, self.beta2, self.eps, decay)
+            g = p.grad
+            if g is None:
+                g = torch.zeros_like(p)
+            elif not g.is_contiguous():
+                g = g.contiguous()
+            s = self.state.get(name)
+            if s is None:
+                s = self.state[name] = (torch.zeros_like(p), torch.zeros_like(p))
+            ps.append(p)
+            gs.append(g)
+            ms.append(s[0])
+            vs.append(s[1])
+            decays.append(0.0 if "norm" in name else self.weight_decay)
+        hyper = (self.step, lr, self.beta1, self.beta2, self.eps)
+        if len({p.data_ptr() for p in ps}) == len(ps):
+            P.adamw_update_multi(ps, gs, ms, vs, *hyper, decays)
+        else:  # a tensor under two names is updated once for each, in turn
+            for p, g, m, v, d in zip(ps, gs, ms, vs, decays):
+                P.adamw_update(p, g, m, v, *hyper, d)

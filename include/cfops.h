@@ -146,6 +146,13 @@ int cfops_linears_backward(cfattn_ctx* ctx, const float* x, size_t t, size_t in,
 int cfops_adamw_update(cfattn_ctx* ctx, float* p, const float* g, float* m, float* v, size_t n, uint64_t t, float lr,
                        float beta1, float beta2, float eps, float weight_decay, void* stream);
 
+/* AdamW::step's loop over the parameters (optim.rs:48-61) in few launches:
+ * adamw_update of `count` tensors, tensor i of n[i] values with its own weight
+ * decay.  No two may overlap in memory. */
+int cfops_adamw_update_multi(cfattn_ctx* ctx, size_t count, float* const* p, const float* const* g, float* const* m,
+                             float* const* v, const size_t* n, const float* weight_decay, uint64_t t, float lr,
+                             float beta1, float beta2, float eps, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
