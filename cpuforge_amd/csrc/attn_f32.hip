@@ -1,6 +1,8 @@
 // fp32 parity mode on gfx950: causal GQA attention forward, dQ and dK/dV with
 // f32 inputs and v_mfma_f32_32x32x2_f32 (exact f32 products, f32
-// accumulation), for head_dim 64 and 128 with 16-byte aligned rows.
+// accumulation), for head_dim 64 and 128 with 16-byte aligned rows.  The
+// forward's units run on the bf16 matrix cores (attn_f32x3.hpp), the f32 one
+// below where a result is not finite.
 //
 // An f32 MFMA takes one value per lane and operand (lane l: A[l%32][l/32],
 // B[l/32][l%32]), so every operand is read row-major:
@@ -128,6 +130,11 @@ __device__ __forceinline__ F32Unit f32_unit(int u, int n_ttiles, int tt, int seq
 }
 
 }  // namespace
+}  // namespace cfattn
+
+#include "attn_f32x3.hpp"
+
+namespace cfattn {
 
 // ------------------------------------------------------------------ forward
 // A wave owns 32 queries of one head; a workgroup of four waves covers hpw
@@ -297,25 +304,33 @@ __device__ __forceinline__ void fwd_f32_unit(const FwdParams& p, const F32Unit u
     if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = (m2 + __log2f(ltot)) * kLn2;
 }
 
+// One unit: on the bf16 matrix cores, or where a result is not finite with
+// f32 MFMAs (after the workgroup's vote every LDS read is done; the loads still
+// in flight are waited for, as fwd_f32_unit counts its own).
 template <int DP>
-__global__ __launch_bounds__(256) void attn_fwd_f32_kernel(const FwdParams p) {
-    constexpr int BN = 32;
-    __shared__ __attribute__((aligned(16))) float sK0[BN * DP];
-    __shared__ __attribute__((aligned(16))) float sK1[BN * DP];
-    __shared__ __attribute__((aligned(16))) float sK2[BN * DP];
-    __shared__ __attribute__((aligned(16))) float sV0[BN * DP];
-    __shared__ __attribute__((aligned(16))) float sV1[BN * DP];
-    __shared__ __attribute__((aligned(16))) float sV2[BN * DP];
+__device__ __forceinline__ void fwd_unit(const FwdParams& p, const F32Unit un, int rest, uint4* sm) {
+    if (fwd_x3_unit<DP>(p, un, rest, sm)) return;
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    float* s = reinterpret_cast<float*>(sm);
+    constexpr int N = 32 * DP;
+    fwd_f32_unit<DP>(p, un, rest, s, s + N, s + 2 * N, s + 3 * N, s + 4 * N, s + 5 * N);
+}
+
+template <int DP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 64 ? 2 : 1, DP == 64 ? 2 : 1))) void
+attn_fwd_f32_kernel(const FwdParams p) {
+    __shared__ uint4 sm[FwdX3<DP>::LDS];
+    static_assert(sizeof(sm) >= 6 * 32 * DP * sizeof(float), "the f32 unit's buffers");
     if (p.xcd_wgs > 0) {
         const int n_groups = p.n_items / p.n_ttiles;
         int tile, grp;
         for (int it = 0; persistent_item(it, n_groups, p.n_ttiles, p.xcd_wgs, p.walk_gm, tile, grp); it++)
-            fwd_f32_unit<DP>(p, F32Unit{tile, 0, 1}, grp, sK0, sK1, sK2, sV0, sV1, sV2);
+            fwd_unit<DP>(p, F32Unit{tile, 0, 1}, grp, sm);
         return;
     }
     const int id = xcd_remap(blockIdx.x, p.n_wg, p.xcd);
     const F32Unit un = f32_unit(id % p.units, p.n_ttiles, 32 * p.tpw, p.seq, p.ksplit);  // longest tiles first
-    fwd_f32_unit<DP>(p, un, id / p.units, sK0, sK1, sK2, sV0, sV1, sV2);
+    fwd_unit<DP>(p, un, id / p.units, sm);
 }
 
 // -------------------------------------------------------------------- dQ

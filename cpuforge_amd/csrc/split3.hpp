@@ -28,12 +28,18 @@
 
 namespace cfattn {
 
-// Two f32 rounded to bf16, packed.  Written as assembly: from the plain casts
-// the compiler converts the low value a second time on its own for lo_f32.
+// Two f32 rounded to bf16, packed (v_cvt_pk_bf16_f32).  The empty assembly makes
+// the pair opaque: from the plain casts the compiler converts the low value a second
+// time on its own for lo_f32.  (The conversion itself is not written as
+// assembly: the compiler would not see a VALU write before an MFMA that reads the
+// pair, and would leave out the wait states between them.)
 __device__ __forceinline__ uint32_t cvt2_bf16(float a, float b) {
-    uint32_t r;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    bf16x2 r;
+    r[0] = (__bf16)a;
+    r[1] = (__bf16)b;
+    uint32_t u = __builtin_bit_cast(uint32_t, r);
+    asm("" : "+v"(u));
+    return u;
 }
 __device__ __forceinline__ float lo_f32(uint32_t u) { return __builtin_bit_cast(float, u << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
@@ -42,7 +48,10 @@ __device__ __forceinline__ float hi_f32(uint32_t u) { return __builtin_bit_cast(
 struct Split8 {
     uint4 p[3];
 };
+// (Contraction is off: fused with a product that forms a value, the subtraction
+// would take the pieces of the unrounded product.)
 __device__ __forceinline__ void split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
+#pragma clang fp contract(off)
     p0 = cvt2_bf16(a, b);
     a -= lo_f32(p0);
     b -= hi_f32(p0);

@@ -1,0 +1,72 @@
+"""GPU tests of the fp32 attention forward on split operands
+(cpuforge_amd/csrc/attn_f32x3.hpp): accuracy against float64 at the edges of
+its 32-key tiles and key splits, and inputs whose bf16 pieces are not finite,
+which the f32 unit computes."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def reference(q, k, v):
+    """o, lse in float64."""
+    B, S, H, d = q.shape
+    G = H // k.shape[2]
+    q, k, v = (x.double() for x in (q, k, v))
+    s = torch.einsum("bshd,bthd->bhst", q, k.repeat_interleave(G, 2)) / math.sqrt(d)
+    s.masked_fill_(torch.ones(S, S, device=DEV, dtype=torch.bool).triu(1), -math.inf)
+    return (torch.einsum("bhst,bthd->bshd", torch.softmax(s, -1), v.repeat_interleave(G, 2)),
+            torch.logsumexp(s, -1))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("shape", [(1, 1, 2, 1), (2, 31, 3, 3), (1, 32, 4, 1), (1, 33, 9, 3), (3, 127, 8, 2),
+                                   (1, 129, 4, 4), (2, 300, 6, 2), (1, 1025, 8, 1)])
+def test_forward_is_f32_accurate(shape, d):
+    from cpuforge_amd import device as D
+    B, S, H, K = shape
+    print(shape, d, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(S + d)
+    q, k, v = (torch.randn(B, S, h, d, generator=g, device=DEV) for h in (H, K, K))
+    o, lse = D.fwd(q, k, v)
+    want, wlse = reference(q, k, v)
+    # A score's error is below (d + 8) 2^-24 sum |q k| / sqrt(d) (about d std-1 products), a probability's
+    # relative error that and exp2's few ulp; o is a convex mean of v's.
+    smax = 4.0 * math.sqrt(d) * (d + 8) * 2.0 ** -24
+    assert (o.double() - want).abs().max() <= (2 * smax + 64 * 2.0 ** -24) * v.abs().max()
+    assert (lse.double() - wlse).abs().max() <= smax + 2.0 ** -20
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_forward_of_infinite_and_huge_inputs_is_f32s(d):
+    """Infinite values give infinities, NaN scores NaN, in the rows that see
+    them only.  A large value stays finite up to 2^119: the unnormalised
+    probabilities go to 2^8 (the running max moves lazily), so that f32 itself
+    overflows on sums past 2^120."""
+    from cpuforge_amd import device as D
+    S, H = 200, 2
+    g = torch.Generator(device=DEV).manual_seed(d)
+    q, k, v = (torch.randn(1, S, H, d, generator=g, device=DEV) for _ in range(3))
+    base, _ = D.fwd(q, k, v)
+    w = v.clone()
+    w[0, 40, 0, 3] = 2.0 ** 119
+    o, _ = D.fwd(q, k, w)
+    want, _ = reference(q, k, w)
+    assert torch.isfinite(o).all()
+    assert (o.double() - want).abs().max() <= 1e-5 * want.abs().max()
+    w[0, 40, 0, 3] = math.inf
+    o, _ = D.fwd(q, k, w)
+    assert (o[0, 40:, 0, 3] == math.inf).all()
+    # (Queries 32..39 share key 40's tile: their masked zero times infinity is
+    # NaN in that head dim, in f32 as well.)
+    o[0, 32:, 0, 3] = base[0, 32:, 0, 3]
+    assert torch.allclose(o, base, rtol=1e-5, atol=1e-5)
+    x = k.clone()
+    x[0, 70, 1, 5] = math.nan
+    o, lse = D.fwd(q, x, v)
+    assert torch.isnan(o[0, 70:, 1]).all() and torch.isnan(lse[0, 1, 70:]).all()
+    assert torch.allclose(o[0, :70], base[0, :70], rtol=1e-5, atol=1e-5)
+    assert torch.allclose(o[0, :, 0], base[0, :, 0], rtol=1e-5, atol=1e-5)
