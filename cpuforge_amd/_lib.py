@@ -84,6 +84,8 @@ SIGNATURES = {
     "cfops_matmul": (C.c_int, [_vp, C.c_int, _vp, _vp, _vp, _sz, _sz, _sz, C.c_int, _vp]),
     "cfops_rmsnorm_forward": (C.c_int, [_vp] * 5 + [_sz, _sz, C.c_float, _vp]),
     "cfops_rmsnorm_backward": (C.c_int, [_vp] * 7 + [_sz, _sz, _vp]),
+    "cfops_rmsnorm_grad": (C.c_int, [_vp] * 7 + [_sz, _sz, C.c_int, _vp]),
+    "cfops_silu_mul_grad": (C.c_int, [_vp] * 6 + [_sz, C.c_int, _vp]),
     "cfops_silu_mul_forward": (C.c_int, [_vp] * 4 + [_sz, _vp]),
     "cfops_silu_mul_backward": (C.c_int, [_vp] * 6 + [_sz, _vp]),
     "cfops_cross_entropy_fwd_bwd": (C.c_int, [_vp] * 4 + [_sz, _sz, _fp, _vp]),

@@ -53,8 +53,8 @@ class RMSNormFn(torch.autograd.Function):
     def backward(ctx, dy):
         x2, w, rstd = ctx.saved_tensors
         rows, dim = x2.shape
-        dx, dw = _zeros(x2, w if ctx.needs_input_grad[1] else None)
-        P.rmsnorm_backward(_flat(dy, dim), x2, w, rstd, dx, dw, rows, dim)
+        dx, dw = _empty(x2, w if ctx.needs_input_grad[1] else None)
+        P.rmsnorm_backward(_flat(dy, dim), x2, w, rstd, dx, dw, rows, dim, acc=False)
         return dx.view(dy.shape), dw, None
 
 
@@ -72,8 +72,8 @@ class SiluMulFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dh):
         g, u = ctx.saved_tensors
-        dg, du = _zeros(g, u)
-        P.silu_mul_backward(dh.contiguous(), g, u, dg, du)
+        dg, du = _empty(g, u)
+        P.silu_mul_backward(dh.contiguous(), g, u, dg, du, acc=False)
         return dg, du
 
 

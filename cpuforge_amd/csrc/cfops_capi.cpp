@@ -186,6 +186,11 @@ int cfops_rmsnorm_forward(cfattn_ctx* c, const float* x, const float* w, float* 
 
 int cfops_rmsnorm_backward(cfattn_ctx* c, const float* dy, const float* x, const float* w, const float* rstd,
                            float* dx, float* dw, size_t rows, size_t dim, void* stream) {
+    return cfops_rmsnorm_grad(c, dy, x, w, rstd, dx, dw, rows, dim, 1, stream);
+}
+
+int cfops_rmsnorm_grad(cfattn_ctx* c, const float* dy, const float* x, const float* w, const float* rstd, float* dx,
+                       float* dw, size_t rows, size_t dim, int acc, void* stream) {
     CF_LOCK(c);
     if (rows == 0 || dim == 0) return CFATTN_OK;
     if (!dy || !x || !w || !rstd || !dx) return fail(c, CFATTN_ERR_ARG, "null buffer");
@@ -197,7 +202,7 @@ int cfops_rmsnorm_backward(cfattn_ctx* c, const float* dy, const float* x, const
             slot(c, cfattn_ctx::OPS_PARTIAL, cfattn::rmsnorm_bwd_partial_floats(rows, dim) * sizeof(float), &rc));
         if (!partial) return rc;
     }
-    CF_HIP(c, cfattn::launch_rmsnorm_bwd(dy, x, w, rstd, dx, dw, partial, rows, dim, to_stream(stream)),
+    CF_HIP(c, cfattn::launch_rmsnorm_bwd(dy, x, w, rstd, dx, dw, partial, rows, dim, acc != 0, to_stream(stream)),
            "rmsnorm backward launch");
     return CFATTN_OK;
 }
@@ -212,10 +217,15 @@ int cfops_silu_mul_forward(cfattn_ctx* c, const float* g, const float* u, float*
 
 int cfops_silu_mul_backward(cfattn_ctx* c, const float* dh, const float* g, const float* u, float* dg, float* du,
                             size_t n, void* stream) {
+    return cfops_silu_mul_grad(c, dh, g, u, dg, du, n, 1, stream);
+}
+
+int cfops_silu_mul_grad(cfattn_ctx* c, const float* dh, const float* g, const float* u, float* dg, float* du, size_t n,
+                        int acc, void* stream) {
     CF_LOCK(c);
     if (n == 0) return CFATTN_OK;
     if (!dh || !g || !u || !dg || !du) return fail(c, CFATTN_ERR_ARG, "null buffer");
-    CF_HIP(c, cfattn::launch_silu_mul_bwd(dh, g, u, dg, du, n, to_stream(stream)), "silu_mul backward launch");
+    CF_HIP(c, cfattn::launch_silu_mul_bwd(dh, g, u, dg, du, n, acc != 0, to_stream(stream)), "silu_mul backward launch");
     return CFATTN_OK;
 }
 

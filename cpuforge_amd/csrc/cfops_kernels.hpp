@@ -9,18 +9,18 @@
 namespace cfattn {
 
 // RMSNorm (crates/core/src/ops/rmsnorm.rs:4-67).  Forward overwrites y and
-// rstd.  Backward accumulates into dx and, when dw is non-null, into dw; it
+// rstd.  Backward adds to (acc) or overwrites dx and, when non-null, dw; it
 // needs `partial` scratch of rmsnorm_bwd_partial_floats(rows, dim) floats.
 hipError_t launch_rmsnorm_fwd(const float* x, const float* w, float* y, float* rstd, size_t rows, size_t dim, float eps,
                               hipStream_t st);
 size_t rmsnorm_bwd_partial_floats(size_t rows, size_t dim);
 hipError_t launch_rmsnorm_bwd(const float* dy, const float* x, const float* w, const float* rstd, float* dx, float* dw,
-                              float* partial, size_t rows, size_t dim, hipStream_t st);
+                              float* partial, size_t rows, size_t dim, int acc, hipStream_t st);
 
 // SwiGLU gate (crates/core/src/ops/swiglu.rs:10-30): forward overwrites h,
-// backward accumulates into dg and du.
+// backward adds to (acc) or overwrites dg and du.
 hipError_t launch_silu_mul_fwd(const float* g, const float* u, float* h, size_t n, hipStream_t st);
-hipError_t launch_silu_mul_bwd(const float* dh, const float* g, const float* u, float* dg, float* du, size_t n,
+hipError_t launch_silu_mul_bwd(const float* dh, const float* g, const float* u, float* dg, float* du, size_t n, int acc,
                                hipStream_t st);
 
 // Cross-entropy with its gradient (crates/core/src/ops/loss.rs:9-55), in three

@@ -11,6 +11,8 @@
 // order instead: deterministic, and within a few ulp of the sequential sum.
 #include <limits.h>
 
+#include <algorithm>
+
 #include "cfattn_common.hpp"
 #include "cfops_kernels.hpp"
 
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_bwd_kernel(const float* _
                                                                   const float* __restrict__ w,
                                                                   const float* __restrict__ rstd,
                                                                   float* __restrict__ dx, float* __restrict__ partial,
-                                                                  long rows, int dim, int rpb) {
+                                                                  long rows, int dim, int rpb, int acc_dx) {
     extern __shared__ float smem[];
     const int ld = dim | 1;
     float* sx = smem;
@@ -198,7 +200,7 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_bwd_kernel(const float* _
     if (VEC) {
         for (int i = threadIdx.x; i < n / 4; i += blockDim.x) {
             const int e = i * 4, rr = e / dim, c = e - rr * dim;
-            float4 d = reinterpret_cast<float4*>(dxb)[i];
+            float4 d = acc_dx ? reinterpret_cast<float4*>(dxb)[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             d.x = radd(d.x, grad(rr, c));
             d.y = radd(d.y, grad(rr, c + 1));
             d.z = radd(d.z, grad(rr, c + 2));
@@ -208,7 +210,7 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_bwd_kernel(const float* _
     } else {
         for (int i = threadIdx.x; i < n; i += blockDim.x) {
             const int rr = i / dim, c = i - rr * dim;
-            dxb[i] = radd(dxb[i], grad(rr, c));
+            dxb[i] = acc_dx ? radd(dxb[i], grad(rr, c)) : grad(rr, c);
         }
     }
     if (partial) {
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rowwise_kernel(const float* _
                                                                   const float* __restrict__ w,
                                                                   const float* __restrict__ rstd,
                                                                   float* __restrict__ dx, float* __restrict__ partial,
-                                                                  long rows, long dim) {
+                                                                  long rows, long dim, int acc_dx) {
     const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     const float* xr = x + r * dim;
@@ -239,9 +241,90 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rowwise_kernel(const float* _
     const float mean = rdiv(dot, (float)dim);
     for (long i = 0; i < dim; i++) {
         const float xh = rmul(xr[i], inv);
-        dx[r * dim + i] = radd(dx[r * dim + i], rmul(inv, rsub(rmul(gr[i], w[i]), rmul(xh, mean))));
+        const float d = rmul(inv, rsub(rmul(gr[i], w[i]), rmul(xh, mean)));
+        dx[r * dim + i] = acc_dx ? radd(dx[r * dim + i], d) : d;
         if (partial) partial[r * dim + i] = rmul(gr[i], xh);
     }
+}
+
+// The same for rows of at most 256 V floats (whole, aligned float4): a wave holds a
+// row in registers, V float4 a lane, so x and dy are read once and the dot is
+// a wave's tree instead of a 576-add chain in one lane; two rows to a wave, eight
+// to a workgroup, whose waves' gain partials are added in wave order.  HBM-bound:
+// 4096 x 576 24.5 -> 7.5 us (28 MB without the read of dx, which was 5 us of fill more).
+constexpr int kRmsWaveRows = 2, kRmsBlockRows = 4 * kRmsWaveRows;
+template <int V>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const float* __restrict__ dy, const float* __restrict__ x,
+                                                               const float* __restrict__ w,
+                                                               const float* __restrict__ rstd, float* __restrict__ dx,
+                                                               float* __restrict__ partial, long rows, int dim,
+                                                               int acc_dx) {
+    extern __shared__ float smem[];  // [4][dim] with `partial`
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n4 = dim / 4;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 wv[V], gain[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int c = lane + 64 * i;
+        wv[i] = c < n4 ? reinterpret_cast<const float4*>(w)[c] : zero;
+        gain[i] = zero;
+    }
+    const long r0 = (long)blockIdx.x * kRmsBlockRows + wave * kRmsWaveRows;
+    float4 xv[kRmsWaveRows][V], gv[kRmsWaveRows][V];
+    float inv[kRmsWaveRows];
+#pragma unroll
+    for (int k = 0; k < kRmsWaveRows; k++) {
+        const long r = r0 + k < rows ? r0 + k : rows - 1;
+        inv[k] = rstd[r];
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const int c = lane + 64 * i;
+            xv[k][i] = c < n4 ? reinterpret_cast<const float4*>(x + r * dim)[c] : zero;
+            gv[k][i] = c < n4 ? reinterpret_cast<const float4*>(dy + r * dim)[c] : zero;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kRmsWaveRows; k++) {
+        if (r0 + k >= rows) break;
+        float dot = 0.0f;
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const float4 a = gv[k][i], b = xv[k][i], c = wv[i];
+            dot = radd(dot, radd(radd(rmul(rmul(a.x, c.x), b.x), rmul(rmul(a.y, c.y), b.y)),
+                                 radd(rmul(rmul(a.z, c.z), b.z), rmul(rmul(a.w, c.w), b.w))));
+        }
+#pragma unroll
+        for (int m = 1; m < 64; m *= 2) dot = radd(dot, __shfl_xor(dot, m));
+        const float mean = rdiv(rmul(dot, inv[k]), (float)dim);
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const int c = lane + 64 * i;
+            if (c >= n4) continue;
+            const float4 a = gv[k][i], b = xv[k][i], ww = wv[i];
+            const float4 h = make_float4(rmul(b.x, inv[k]), rmul(b.y, inv[k]), rmul(b.z, inv[k]), rmul(b.w, inv[k]));
+            float4 d = make_float4(rmul(inv[k], rsub(rmul(a.x, ww.x), rmul(h.x, mean))),
+                                   rmul(inv[k], rsub(rmul(a.y, ww.y), rmul(h.y, mean))),
+                                   rmul(inv[k], rsub(rmul(a.z, ww.z), rmul(h.z, mean))),
+                                   rmul(inv[k], rsub(rmul(a.w, ww.w), rmul(h.w, mean))));
+            float4* o = reinterpret_cast<float4*>(dx + (r0 + k) * dim) + c;
+            if (acc_dx) {
+                const float4 p = *o;
+                d = make_float4(radd(p.x, d.x), radd(p.y, d.y), radd(p.z, d.z), radd(p.w, d.w));
+            }
+            *o = d;
+            gain[i] = make_float4(radd(gain[i].x, rmul(a.x, h.x)), radd(gain[i].y, rmul(a.y, h.y)),
+                                  radd(gain[i].z, rmul(a.z, h.z)), radd(gain[i].w, rmul(a.w, h.w)));
+        }
+    }
+    if (!partial) return;
+#pragma unroll
+    for (int i = 0; i < V; i++)
+        if (lane + 64 * i < n4) reinterpret_cast<float4*>(smem + wave * dim)[lane + 64 * i] = gain[i];
+    __syncthreads();
+    for (int c = threadIdx.x; c < dim; c += 256)
+        partial[(long)blockIdx.x * dim + c] =
+            radd(radd(smem[c], smem[dim + c]), radd(smem[2 * dim + c], smem[3 * dim + c]));
 }
 
 // dw[i] += the partial rows, in a fixed two-level order: a workgroup covers
@@ -250,7 +333,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rowwise_kernel(const float* _
 // in j order.  Deterministic, and the loads of one thread are independent
 // of its adds, so they stay in flight together.
 __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial,
-                                                                float* __restrict__ dw, long nblk, long dim) {
+                                                                float* __restrict__ dw, long nblk, long dim, int acc) {
     __shared__ float ssum[8][32];
     const int cl = threadIdx.x & 31, j = threadIdx.x >> 5;
     const long c = (long)blockIdx.x * 32 + cl;
@@ -264,7 +347,7 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(const float* __r
     ssum[j][cl] = s;
     __syncthreads();
     if (j == 0 && c < dim) {
-        float t = dw[c];
+        float t = acc ? dw[c] : 0.0f;
         for (int i = 0; i < 8; i++) t = radd(t, ssum[i][cl]);
         dw[c] = t;
     }
@@ -273,7 +356,8 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(const float* __r
 size_t rmsnorm_bwd_partial_floats(size_t rows, size_t dim) {
     if (rows == 0 || dim == 0) return 0;
     if (!rms_staged(dim)) return rows * dim;
-    const size_t rpb = (size_t)rms_rows(dim);
+    // The wave kernel's blocks are the smaller.
+    const size_t rpb = std::min((size_t)rms_rows(dim), (size_t)kRmsBlockRows);
     return (rows + rpb - 1) / rpb * dim;
 }
 
@@ -300,13 +384,24 @@ hipError_t launch_rmsnorm_fwd(const float* x, const float* w, float* y, float* r
 }
 
 hipError_t launch_rmsnorm_bwd(const float* dy, const float* x, const float* w, const float* rstd, float* dx, float* dw,
-                              float* partial, size_t rows, size_t dim, hipStream_t st) {
+                              float* partial, size_t rows, size_t dim, int acc, hipStream_t st) {
     if (rows == 0 || dim == 0) return hipSuccess;
     float* part = dw ? partial : nullptr;
     size_t nblk;
-    if (!rms_staged(dim)) {
+    if (dim % 4 == 0 && dim <= 2048 && aligned16(dy) && aligned16(x) && aligned16(dx) && aligned16(w)) {
+        nblk = (rows + kRmsBlockRows - 1) / kRmsBlockRows;
+        if (nblk > 0x7fffffffu) return hipErrorInvalidConfiguration;
+        const size_t lds = part ? 4 * dim * sizeof(float) : 0;
+        const auto kernel = dim <= 256   ? rmsnorm_bwd_wave_kernel<1>
+                            : dim <= 512 ? rmsnorm_bwd_wave_kernel<2>
+                            : dim <= 768 ? rmsnorm_bwd_wave_kernel<3>
+                            : dim <= 1024 ? rmsnorm_bwd_wave_kernel<4>
+                                          : rmsnorm_bwd_wave_kernel<8>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(256), lds, st, dy, x, w, rstd, dx, part, (long)rows,
+                           (int)dim, acc);
+    } else if (!rms_staged(dim)) {
         hipLaunchKernelGGL(rmsnorm_bwd_rowwise_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, dy, x,
-                           w, rstd, dx, part, (long)rows, (long)dim);
+                           w, rstd, dx, part, (long)rows, (long)dim, acc);
         nblk = rows;
     } else {
         const int rpb = rms_rows(dim);
@@ -316,15 +411,15 @@ hipError_t launch_rmsnorm_bwd(const float* dy, const float* x, const float* w, c
         const bool vec = dim % 4 == 0 && aligned16(dy) && aligned16(x) && aligned16(dx);
         if (vec)
             hipLaunchKernelGGL(rmsnorm_bwd_kernel<true>, dim3((unsigned)nblk), dim3(kRmsThreads), lds, st, dy, x, w,
-                               rstd, dx, part, (long)rows, (int)dim, rpb);
+                               rstd, dx, part, (long)rows, (int)dim, rpb, acc);
         else
             hipLaunchKernelGGL(rmsnorm_bwd_kernel<false>, dim3((unsigned)nblk), dim3(kRmsThreads), lds, st, dy, x, w,
-                               rstd, dx, part, (long)rows, (int)dim, rpb);
+                               rstd, dx, part, (long)rows, (int)dim, rpb, acc);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !dw) return e;
     hipLaunchKernelGGL(rmsnorm_dw_reduce_kernel, dim3((unsigned)((dim + 31) / 32)), dim3(256), 0, st, part, dw,
-                       (long)nblk, (long)dim);
+                       (long)nblk, (long)dim, acc);
     return hipGetLastError();
 }
 
@@ -364,7 +459,7 @@ __global__ __launch_bounds__(256) void silu_mul_fwd_kernel(const float* __restri
 template <bool VEC>
 __global__ __launch_bounds__(256) void silu_mul_bwd_kernel(const float* __restrict__ dh, const float* __restrict__ g,
                                                            const float* __restrict__ u, float* __restrict__ dg,
-                                                           float* __restrict__ du, long n) {
+                                                           float* __restrict__ du, long n, int acc) {
     const long stride = (long)gridDim.x * blockDim.x;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (VEC) {
@@ -372,8 +467,8 @@ __global__ __launch_bounds__(256) void silu_mul_bwd_kernel(const float* __restri
             const float4 d = reinterpret_cast<const float4*>(dh)[i];
             const float4 a = reinterpret_cast<const float4*>(g)[i];
             const float4 b = reinterpret_cast<const float4*>(u)[i];
-            float4 x = reinterpret_cast<float4*>(dg)[i];
-            float4 y = reinterpret_cast<float4*>(du)[i];
+            float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f), y = x;
+            if (acc) x = reinterpret_cast<float4*>(dg)[i], y = reinterpret_cast<float4*>(du)[i];
             silu_mul_grad(d.x, a.x, b.x, x.x, y.x);
             silu_mul_grad(d.y, a.y, b.y, x.y, y.y);
             silu_mul_grad(d.z, a.z, b.z, x.z, y.z);
@@ -382,7 +477,12 @@ __global__ __launch_bounds__(256) void silu_mul_bwd_kernel(const float* __restri
             reinterpret_cast<float4*>(du)[i] = y;
         }
     } else {
-        for (; i < n; i += stride) silu_mul_grad(dh[i], g[i], u[i], dg[i], du[i]);
+        for (; i < n; i += stride) {
+            float x = acc ? dg[i] : 0.0f, y = acc ? du[i] : 0.0f;
+            silu_mul_grad(dh[i], g[i], u[i], x, y);
+            dg[i] = x;
+            du[i] = y;
+        }
     }
 }
 
@@ -401,15 +501,15 @@ hipError_t launch_silu_mul_fwd(const float* g, const float* u, float* h, size_t 
     return hipGetLastError();
 }
 
-hipError_t launch_silu_mul_bwd(const float* dh, const float* g, const float* u, float* dg, float* du, size_t n,
+hipError_t launch_silu_mul_bwd(const float* dh, const float* g, const float* u, float* dg, float* du, size_t n, int acc,
                                hipStream_t st) {
     if (n == 0) return hipSuccess;
     if (n % 4 == 0 && aligned16(dh) && aligned16(g) && aligned16(u) && aligned16(dg) && aligned16(du))
         hipLaunchKernelGGL(silu_mul_bwd_kernel<true>, dim3(ew_blocks(n / 4)), dim3(256), 0, st, dh, g, u, dg, du,
-                           (long)n);
+                           (long)n, acc);
     else
         hipLaunchKernelGGL(silu_mul_bwd_kernel<false>, dim3(ew_blocks(n)), dim3(256), 0, st, dh, g, u, dg, du,
-                           (long)n);
+                           (long)n, acc);
     return hipGetLastError();
 }
 

@@ -96,11 +96,12 @@ def rmsnorm_forward(x, w, y, rstd, rows, dim, eps, ctx: Context | None = None):
           _f32(rstd, "rstd", rows), rows, dim, float(eps), _stream())
 
 
-def rmsnorm_backward(dy, x, w, rstd, dx, dw, rows, dim, ctx: Context | None = None):
-    """rmsnorm.rs:33-67: accumulates into dx and dw (dw None: frozen gain)."""
+def rmsnorm_backward(dy, x, w, rstd, dx, dw, rows, dim, ctx: Context | None = None, acc: bool = True):
+    """rmsnorm.rs:33-67: accumulates into dx and dw (dw None: frozen gain), or
+    overwrites them with acc=False."""
     ctx = ctx or default_context()
-    _call(ctx, "cfops_rmsnorm_backward", _f32(dy, "dy", rows * dim), _f32(x, "x", rows * dim), _f32(w, "w", dim),
-          _f32(rstd, "rstd", rows), _f32(dx, "dx", rows * dim), _opt(dw, "dw", dim), rows, dim, _stream())
+    _call(ctx, "cfops_rmsnorm_grad", _f32(dy, "dy", rows * dim), _f32(x, "x", rows * dim), _f32(w, "w", dim),
+          _f32(rstd, "rstd", rows), _f32(dx, "dx", rows * dim), _opt(dw, "dw", dim), rows, dim, int(acc), _stream())
 
 
 # --------------------------------------------------------------- SwiGLU
@@ -111,12 +112,12 @@ def silu_mul_forward(g, u, h, ctx: Context | None = None):
     _call(ctx, "cfops_silu_mul_forward", _f32(g, "g"), _f32(u, "u", n), _f32(h, "h", n), n, _stream())
 
 
-def silu_mul_backward(dh, g, u, dg, du, ctx: Context | None = None):
-    """swiglu.rs:18-30: accumulates into dg and du."""
+def silu_mul_backward(dh, g, u, dg, du, ctx: Context | None = None, acc: bool = True):
+    """swiglu.rs:18-30: accumulates into dg and du, or overwrites them with acc=False."""
     ctx = ctx or default_context()
     n = g.numel()
-    _call(ctx, "cfops_silu_mul_backward", _f32(dh, "dh", n), _f32(g, "g"), _f32(u, "u", n), _f32(dg, "dg", n),
-          _f32(du, "du", n), n, _stream())
+    _call(ctx, "cfops_silu_mul_grad", _f32(dh, "dh", n), _f32(g, "g"), _f32(u, "u", n), _f32(dg, "dg", n),
+          _f32(du, "du", n), n, int(acc), _stream())
 
 
 # -------------------------------------------------------- cross-entropy

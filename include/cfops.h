@@ -53,11 +53,20 @@ int cfops_rmsnorm_forward(cfattn_ctx* ctx, const float* x, const float* w, float
 int cfops_rmsnorm_backward(cfattn_ctx* ctx, const float* dy, const float* x, const float* w, const float* rstd,
                            float* dx, float* dw, size_t rows, size_t dim, void* stream);
 
+/* No reference counterpart: the same with acc == 0 overwriting dx and dw
+ * (for callers whose buffers hold nothing yet), acc != 0 adding to them. */
+int cfops_rmsnorm_grad(cfattn_ctx* ctx, const float* dy, const float* x, const float* w, const float* rstd, float* dx,
+                       float* dw, size_t rows, size_t dim, int acc, void* stream);
+
 /* silu_mul_forward / _backward (swiglu.rs:10-30): h = silu(g) * u
  * (overwritten); the backward accumulates into dg and du. */
 int cfops_silu_mul_forward(cfattn_ctx* ctx, const float* g, const float* u, float* h, size_t n, void* stream);
 int cfops_silu_mul_backward(cfattn_ctx* ctx, const float* dh, const float* g, const float* u, float* dg, float* du,
                             size_t n, void* stream);
+
+/* The same with acc == 0 overwriting dg and du, acc != 0 adding to them. */
+int cfops_silu_mul_grad(cfattn_ctx* ctx, const float* dh, const float* g, const float* u, float* dg, float* du,
+                        size_t n, int acc, void* stream);
 
 /* cross_entropy_fwd_bwd (loss.rs:9-55): mean cross-entropy over the rows
  * whose target is not CFOPS_IGNORE_INDEX; dlogits [rows, vocab] is

@@ -1,0 +1,49 @@
+"""GPU tests of the overwriting gradients (rmsnorm_backward, silu_mul_backward
+with acc=False) and of the one-wave-per-row RMSNorm backward at the edges of
+its widths (256 floats to a register step) and row blocks (8), against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 1000])
+@pytest.mark.parametrize("dim", [4, 252, 256, 260, 512, 576, 768, 772, 1024, 1028, 2048, 2052, 577])
+def test_rmsnorm_backward_edges(rows, dim):
+    from cpuforge_amd import ops as P
+    print(rows, dim, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows * 10000 + dim)
+    R = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    dy, x, w, dx0, dw0 = R(rows, dim), R(rows, dim), R(dim), R(rows, dim), R(dim)
+    y, rstd = torch.empty_like(x), torch.empty(rows, device=DEV)
+    P.rmsnorm_forward(x, w, y, rstd, rows, dim, 1e-5)
+    xd, wd, dyd, inv = x.double(), w.double(), dy.double(), rstd.double()[:, None]
+    xh = xd * inv
+    gx = inv * (dyd * wd - xh * (dyd * wd * xh).mean(-1, keepdim=True))
+    gw = (dyd * xh).sum(0)
+    mag = inv * ((dyd * wd).abs() + xh.abs() * (dyd * wd * xh).abs().mean(-1, keepdim=True))
+    wmag = (dyd * xh).abs().sum(0)
+    for acc in (True, False):
+        for frozen in (True, False):
+            dx = dx0.clone() if acc else torch.full_like(x, float("nan"))
+            dw = None if frozen else dw0.clone() if acc else torch.full_like(w, float("nan"))
+            P.rmsnorm_backward(dy, x, w, rstd, dx, dw, rows, dim, acc=acc)
+            # A rounding per term of each sum, and a few per element.
+            base = dx0.double() if acc else 0.0
+            assert bool(((dx - (gx + base)).abs() <= 2.0 ** -24 * ((dim + 16) * mag + 2 * dx0.abs())).all())
+            if not frozen:
+                base = dw0.double() if acc else 0.0
+                assert bool(((dw - (gw + base)).abs() <= 2.0 ** -24 * ((rows + 16) * wmag + 2 * dw0.abs())).all())
+
+
+@pytest.mark.parametrize("n", [1, 4, 1001, 4096])
+def test_silu_mul_backward_overwrites(n):
+    from cpuforge_amd import ops as P
+    g = torch.Generator(device=DEV).manual_seed(n)
+    dh, a, u = (torch.randn(n, generator=g, device=DEV) for _ in range(3))
+    zeros = [torch.zeros(n, device=DEV) for _ in range(2)]
+    P.silu_mul_backward(dh, a, u, *zeros)
+    out = [torch.full((n,), float("nan"), device=DEV) for _ in range(2)]
+    P.silu_mul_backward(dh, a, u, *out, acc=False)
+    assert all(torch.equal(x, z) for x, z in zip(out, zeros))
