@@ -31,20 +31,23 @@ IGNORE_INDEX = _lib.IGNORE_INDEX
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """torch.cuda.current_stream().cuda_stream without the Stream object, which
+    takes 5 us a call to make, half of what a small op's whole call takes."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _f32(t: torch.Tensor, name: str, numel: int | None = None) -> int:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32 and t.is_contiguous() \
+            and (numel is None or t.numel() == numel):
+        return t.data_ptr()
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != torch.float32:
         raise TypeError(f"{name} must be float32, got {t.dtype}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    if numel is not None and t.numel() != numel:
-        raise _lib.ShapeError(_lib.ERR_SHAPE,
-                              f"assertion `left == right` failed: {name}.len() = {t.numel()}, expected {numel}")
-    return t.data_ptr()
+    raise _lib.ShapeError(_lib.ERR_SHAPE,
+                          f"assertion `left == right` failed: {name}.len() = {t.numel()}, expected {numel}")
 
 
 def _opt(t, name, numel=None):
