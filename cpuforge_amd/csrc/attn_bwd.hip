@@ -256,8 +256,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const BwdParams p) {
     float* dvrow = p.dv + (long)b * p.kv_bs + (long)kw * kvrs + (long)g * p.hd;
 #pragma unroll
     for (int db = 0; db < NDB; db++) {
-        add_row_block(dkrow, dkt[db], db * 32, hh, p.hd, p.g_vec_ok);
-        add_row_block(dvrow, dvt[db], db * 32, hh, p.hd, p.g_vec_ok);
+        add_row_block(dkrow, dkt[db], db * 32, hh, p.hd, p.g_vec_ok, p.acc & kAccDk);
+        add_row_block(dvrow, dvt[db], db * 32, hh, p.hd, p.g_vec_ok, p.acc & kAccDv);
     }
 }
 
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(const BwdParams p) {
     if (!wave_active || !row_ok) return;
     float* dqrow = p.dq + qoff;
 #pragma unroll
-    for (int db = 0; db < NDB; db++) add_row_block(dqrow, dqt[db], db * 32, hh, p.hd, p.g_vec_ok);
+    for (int db = 0; db < NDB; db++) add_row_block(dqrow, dqt[db], db * 32, hh, p.hd, p.g_vec_ok, p.acc & kAccDq);
 }
 
 // ---------------------------------------------------------------------------
@@ -633,7 +633,7 @@ __device__ __forceinline__ void dq_bf16_unit(const BwdParams& p, const int tile,
         for (int db = 0; db < NDB; db++) dqt[db] *= p.scale;
         const float inv = ok ? p.norm_qr[r] : 0.0f;
         float4 cur[NDB][4];
-        load_grad_row<NDB>(cur, p.dq + qoff, hh, ok);
+        load_grad_row<NDB>(cur, p.dq + qoff, hh, ok && (p.acc & kAccDq));
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         write_grad_row_norm<NDB>(p.dq + qoff, xs, inv, p.norm_qw, dqt, lane, tq, ok, p, cur);
         const int slot = blockIdx.x * NW + wave;
@@ -643,7 +643,7 @@ __device__ __forceinline__ void dq_bf16_unit(const BwdParams& p, const int tile,
     if (!wave_active || !row_ok) return;
 #pragma unroll
     for (int db = 0; db < NDB; db++) dqt[db] *= p.scale;  // dS was accumulated without the softmax scale
-    write_grad_row<NDB>(p.dq + qoff, dqt, hh, tq, p);
+    write_grad_row<NDB>(p.dq + qoff, dqt, hh, tq, p, p.acc & kAccDq);
 }
 
 template <int DP, int BN, int NW, bool NORM>
@@ -794,7 +794,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_ds_kernel(const BwdParams
     // tiles stream in, instead of as a dependent read at the end.
     float* const dq_row = p.dq + (long)b * p.q_bs + (long)tq * qrs + (long)head * DP;
     float4 dq_pre[NDB][4];
-    const bool pre = row_ok && grad_row_prefetch<NDB, NORM>(dq_pre, dq_row, hh, p);
+    const bool pre = row_ok && grad_row_prefetch<NDB, NORM>(dq_pre, dq_row, hh, p, p.acc & kAccDq);
 
     // Step kt reads buffer kt % 3 and fills buffer (kt + 2) % 3, which the
     // barrier closing step kt - 1 has freed.
@@ -876,9 +876,9 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_ds_kernel(const BwdParams
 #pragma unroll
     for (int db = 0; db < NDB; db++) dqt[db] *= p.scale;  // dS was stored without the softmax scale
     if (pre)
-        write_grad_row<NDB, true>(dq_row, dqt, hh, tq, p, dq_pre);
+        write_grad_row<NDB, true>(dq_row, dqt, hh, tq, p, true, dq_pre);
     else
-        write_grad_row<NDB>(dq_row, dqt, hh, tq, p);
+        write_grad_row<NDB>(dq_row, dqt, hh, tq, p, p.acc & kAccDq);
 }
 
 // dK/dV with two specialised waves per 32-key slice: eight waves, 128 keys per
@@ -1281,7 +1281,7 @@ __device__ __forceinline__ void dkdv_ws_unit(const BwdParams& p, const int kvt, 
                 for (int db = 0; db < NDB; db++) acc[db] *= p.scale;
                 const float inv = ok ? p.norm_kr[r] : 0.0f;
                 float4 cur[NDB][4];
-                load_grad_row<NDB>(cur, p.dk + r * DP, hh, ok);
+                load_grad_row<NDB>(cur, p.dk + r * DP, hh, ok && (p.acc & kAccDk));
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 write_grad_row_norm<NDB>(p.dk + r * DP, xs, inv, p.norm_kw, acc, lane, kw, ok, p, cur);
                 const int slot = blockIdx.x * 4 + slice;
@@ -1293,11 +1293,11 @@ __device__ __forceinline__ void dkdv_ws_unit(const BwdParams& p, const int kvt, 
         float* row = (PW ? p.dv : p.dk) + (long)b * p.kv_bs + (long)kw * kvrs + (long)g * DP;
         if constexpr (PW) {
 #pragma unroll
-            for (int db = 0; db < NDB; db++) add_row_block(row, acc[db], db * 32, hh, DP, true);
+            for (int db = 0; db < NDB; db++) add_row_block(row, acc[db], db * 32, hh, DP, true, p.acc & kAccDv);
         } else {
 #pragma unroll
             for (int db = 0; db < NDB; db++) acc[db] *= p.scale;  // dS was accumulated without the softmax scale
-            write_grad_row<NDB>(row, acc, hh, kw, p);
+            write_grad_row<NDB>(row, acc, hh, kw, p, p.acc & kAccDk);
         }
     };
 
@@ -1433,7 +1433,7 @@ bool attn_bwd_epilogue_applies(Dtype dt, const Dims& d, const void* d_o, const v
 
 hipError_t launch_attn_bwd(Dtype dt, const Dims& d, const void* d_o, const void* q, const void* k, const void* v,
                            const float* o, const float* lse, float* delta, float* dq, float* dk, float* dv,
-                           hipStream_t st, const Tuning& tu, void* ds, size_t ds_bytes, const BwdEpilogue* epi) {
+                           hipStream_t st, const Tuning& tu, void* ds, size_t ds_bytes, const BwdEpilogue* epi, int acc) {
     if (d.batch == 0 || d.seq == 0 || d.nh == 0) return hipSuccess;
     const bool fast = fast_bf16_applies(dt, d, d_o, q, k, v, dq, dk, dv, tu);
     // The epilogue reads the cos/sin rows (and with the norm the pre-norm
@@ -1465,6 +1465,7 @@ hipError_t launch_attn_bwd(Dtype dt, const Dims& d, const void* d_o, const void*
     p.dq = dq;
     p.dk = dk;
     p.dv = dv;
+    p.acc = acc;
     p.batch = d.batch;
     p.seq = d.seq;
     p.nh = d.nh;
@@ -1653,7 +1654,8 @@ hipError_t launch_attn_bwd(Dtype dt, const Dims& d, const void* d_o, const void*
             e = hipGetLastError();
         }
         if (e != hipSuccess || p.epi != kEpiUnrotNorm) return e;
-        return launch_norm_gain_reduce(p.norm_part, p.norm_nq, p.norm_nk, d.hd, epi->norm.dqw, epi->norm.dkw, st);
+        return launch_norm_gain_reduce(p.norm_part, p.norm_nq, p.norm_nk, d.hd, epi->norm.dqw, epi->norm.dkw,
+                                       (acc & kAccDq) != 0, st);
     }
     if (dt == kF32 && attn_f32_fast_applies(d, p.vec_ok, p.g_vec_ok) && tu.bwd_kv_waves == 0 && ds != nullptr &&
         ds_bytes >= attn_f32_scratch_bytes(d)) {

@@ -24,14 +24,16 @@ __device__ __forceinline__ bool dkdv_walks_down(unsigned hw_id, int xcd_cus) {
     return ((hw_id / 8u / (unsigned)xcd_cus) & 1u) == 0u;
 }
 
-// Accumulate one lane's 4 x (4 consecutive head dims) of a transposed
-// accumulator block into a global row: dst[d0 + 8*rq + 4*hh + i] += acc[4*rq + i].
-__device__ __forceinline__ void add_row_block(float* row, const f32x16& acc, int dbase, int hh, int hd, bool vec_ok) {
+// One lane's 4 x (4 consecutive head dims) of a transposed accumulator block
+// to a global row: dst[d0 + 8*rq + 4*hh + i] += acc[4*rq + i], or = without
+// `add` (the row is then not read).
+__device__ __forceinline__ void add_row_block(float* row, const f32x16& acc, int dbase, int hh, int hd, bool vec_ok,
+                                              bool add) {
 #pragma unroll
     for (int rq = 0; rq < 4; rq++) {
         const int d0 = dbase + rq * 8 + hh * 4;
         if (vec_ok && d0 + 4 <= hd) {
-            float4 v = *reinterpret_cast<float4*>(row + d0);
+            float4 v = add ? *reinterpret_cast<float4*>(row + d0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             v.x += acc[rq * 4 + 0];
             v.y += acc[rq * 4 + 1];
             v.z += acc[rq * 4 + 2];
@@ -40,7 +42,7 @@ __device__ __forceinline__ void add_row_block(float* row, const f32x16& acc, int
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                if (d0 + i < hd) row[d0 + i] += acc[rq * 4 + i];
+                if (d0 + i < hd) row[d0 + i] = (add ? row[d0 + i] : 0.0f) + acc[rq * 4 + i];
         }
     }
 }
@@ -57,10 +59,11 @@ __device__ __forceinline__ void add_row_block(float* row, const f32x16& acc, int
 // With PRE (the += modes), the row's current values come from `pre` instead
 // of memory: grad_row_prefetch read them earlier, so that the read is not a
 // dependent round trip at the end of the kernel.
-// `mode` is p.epi unless given (>= 0).
+// Without `add` the row is written in the += modes too, and not read; `pre` is
+// then not given.  `mode` is p.epi unless given (>= 0).
 template <int NDB, bool PRE = false>
 __device__ __forceinline__ void write_grad_row(float* row, const f32x16 (&acc)[NDB], int hh, int t,
-                                               const BwdParams& p, const float4 (*pre)[4] = nullptr,
+                                               const BwdParams& p, bool add, const float4 (*pre)[4] = nullptr,
                                                int mode = -1) {
 #pragma clang fp contract(off)
     constexpr int DP = NDB * 32, HALF = DP / 2;
@@ -81,7 +84,7 @@ __device__ __forceinline__ void write_grad_row(float* row, const f32x16 (&acc)[N
             return;
         }
 #pragma unroll
-        for (int db = 0; db < NDB; db++) add_row_block(row, acc[db], db * 32, hh, DP, true);
+        for (int db = 0; db < NDB; db++) add_row_block(row, acc[db], db * 32, hh, DP, true, add);
         return;
     }
     const float* cs = p.rope_cos + (long)(p.rope_pos0 + t) * HALF;
@@ -115,7 +118,7 @@ __device__ __forceinline__ void write_grad_row(float* row, const f32x16 (&acc)[N
             }
             float4* r1 = reinterpret_cast<float4*>(row + d0);
             float4* r2 = reinterpret_cast<float4*>(row + d0 + HALF);
-            if (mode == kEpiUnrotAdd) {
+            if (mode == kEpiUnrotAdd && (PRE || add)) {
                 float4 a, b;
                 if constexpr (PRE) {
                     a = pre[db][rq];
@@ -313,12 +316,14 @@ __device__ __forceinline__ void load_grad_row(float4 (&v)[NDB][4], const float* 
 }
 
 // The lane's part of a gradient row, read ahead for the += epilogue modes
-// (kEpiUnrotNorm too with NORM); false (nothing read) for the others.
+// (kEpiUnrotNorm too with NORM, zeros where it is not added to); false
+// (nothing read) for the others and for a row that is overwritten.
 template <int NDB, bool NORM = false>
 __device__ __forceinline__ bool grad_row_prefetch(float4 (&pre)[NDB][4], const float* row, int hh,
-                                                  const BwdParams& p) {
-    if (p.epi != kEpiAdd && p.epi != kEpiUnrotAdd && !(NORM && p.epi == kEpiUnrotNorm)) return false;
-    load_grad_row<NDB>(pre, row, hh, true);
+                                                  const BwdParams& p, bool add) {
+    const bool norm = NORM && p.epi == kEpiUnrotNorm;
+    if (!norm && (!add || (p.epi != kEpiAdd && p.epi != kEpiUnrotAdd))) return false;
+    load_grad_row<NDB>(pre, row, hh, add);
     return true;
 }
 

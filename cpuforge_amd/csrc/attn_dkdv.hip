@@ -328,13 +328,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     auto acc_settle = [&](f32x16 (&acc)[NDB][NKB]) {
         acc_wait8(acc[0][0], acc[0][1], acc[1][0], acc[1][1], acc[2][0], acc[2][1], acc[3][0], acc[3][1]);
     };
-    // dV rows are added; dK rows (scaled: dS was accumulated without the
+    // dV rows are added or written (p.acc); dK rows (scaled: dS was accumulated without the
     // softmax scale) go through the epilogue mode.  The current values of
     // the lane's rows (both key blocks) are read before any is written, so
     // that the wave waits for one round of reads rather than one per block.
     auto store_rows = [&](float* dst, f32x16 (&acc)[NDB][NKB], bool dk_rows) {
         if (!pair_live) return;
         const int mode = dk_rows ? p.epi : kEpiAdd;
+        const bool add = p.acc & (dk_rows ? kAccDk : kAccDv);
+        const bool pre = add && (mode == kEpiAdd || mode == kEpiUnrotAdd);
         float* row[NKB];
         bool ok[NKB];
 #pragma unroll
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             row[kb] = dst + (long)b * p.kv_bs + (long)kw * kvrs + (long)g * DP;
         }
         float4 cur[NKB][NDB][4];
-        if (mode == kEpiAdd || mode == kEpiUnrotAdd) {
+        if (pre) {
 #pragma unroll
             for (int kb = 0; kb < NKB; kb++) load_grad_row<NDB>(cur[kb], row[kb], hh, ok[kb]);
         }
@@ -355,10 +357,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             f32x16 r[NDB];
 #pragma unroll
             for (int db = 0; db < NDB; db++) r[db] = dk_rows ? acc[db][kb] * p.scale : acc[db][kb];
-            if (mode == kEpiAdd || mode == kEpiUnrotAdd)
-                write_grad_row<NDB, true>(row[kb], r, hh, kw, p, cur[kb], mode);
+            if (pre)
+                write_grad_row<NDB, true>(row[kb], r, hh, kw, p, true, cur[kb], mode);
             else
-                write_grad_row<NDB>(row[kb], r, hh, kw, p, nullptr, mode);
+                write_grad_row<NDB>(row[kb], r, hh, kw, p, add, nullptr, mode);
         }
     };
     // Per-row values (lse or delta) of MFMA rows 8*g4 + 4*hh + [0, 4) of

@@ -461,7 +461,7 @@ __device__ __forceinline__ void dq_f32_unit(const BwdParams& p, const F32Unit un
 #pragma unroll
         for (int rq = 0; rq < 4; rq++) {
             float4* dst = reinterpret_cast<float4*>(row + db * 32 + rq * 8 + hh * 4);
-            float4 v = *dst;
+            float4 v = p.acc & kAccDq ? *dst : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             v.x += acc[db][rq * 4] * p.scale;
             v.y += acc[db][rq * 4 + 1] * p.scale;
             v.z += acc[db][rq * 4 + 2] * p.scale;
@@ -581,7 +581,7 @@ __device__ __forceinline__ void dq_f32_ds_unit(const BwdParams& p, const int til
 #pragma unroll
         for (int rq = 0; rq < 4; rq++) {
             float4* dst = reinterpret_cast<float4*>(row + db * 32 + rq * 8 + hh * 4);
-            float4 v = *dst;
+            float4 v = p.acc & kAccDq ? *dst : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             v.x += acc[db][rq * 4] * p.scale;
             v.y += acc[db][rq * 4 + 1] * p.scale;
             v.z += acc[db][rq * 4 + 2] * p.scale;
@@ -839,13 +839,13 @@ attn_bwd_dkdv_f32_kernel(const BwdParams p, const F32DkdvArgs a) {
     dkdv_f32_unit<DP>(p, a, id % a.units, id / a.units, sQ0, sQ1, sQ2, sO0, sO1, sO2, sLD);
 }
 
-// dk += sum over slots (query head of the group, then query split) of the
+// dk += (or =, `acc`) sum over slots (query head of the group, then query split) of the
 // dK slots, dv likewise; four floats per thread.  The workgroups of a key
 // tile's splits write their slots for all of its keys (zeros where they saw
 // no query), so the slots read here are defined; the splits beyond the key
 // tile's count are neither written nor read.
 __global__ __launch_bounds__(256) void attn_f32_reduce_kernel(const float* __restrict__ part, const F32DkdvArgs a,
-                                                              int seq, int row_floats, int group,
+                                                              int seq, int row_floats, int group, int acc,
                                                               float* __restrict__ dk, float* __restrict__ dv) {
     const long i4 = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long half = a.part_half;
@@ -865,7 +865,8 @@ __global__ __launch_bounds__(256) void attn_f32_reduce_kernel(const float* __res
         }
     float4* dk4 = reinterpret_cast<float4*>(dk) + i4;
     float4* dv4 = reinterpret_cast<float4*>(dv) + i4;
-    float4 x = *dk4, y = *dv4;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 x = acc & kAccDk ? *dk4 : zero, y = acc & kAccDv ? *dv4 : zero;
     x.x += sk.x, x.y += sk.y, x.z += sk.z, x.w += sk.w;
     y.x += sv.x, y.y += sv.y, y.z += sv.z, y.w += sv.w;
     *dk4 = x;
@@ -915,7 +916,7 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_merge_kernel(const FwdParams
     if (c == 0) p.lse[row] = (m + __log2f(l)) * kLn2;
 }
 
-// dq += sum over the splits of a row, in split order.
+// dq += (or =, p.acc) sum over the splits of a row, in split order.
 template <int DP>
 __global__ __launch_bounds__(256) void attn_f32_dq_merge_kernel(const BwdParams p) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(256) void attn_f32_dq_merge_kernel(const BwdParams 
     const long bh = row / p.seq;
     const long b = bh / p.nh, head = bh % p.nh;
     float4* dst = reinterpret_cast<float4*>(p.dq + b * p.q_bs + (long)tq * p.nh * DP + head * DP) + c;
-    float4 v = *dst;
+    float4 v = p.acc & kAccDq ? *dst : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     v.x += sum.x, v.y += sum.y, v.z += sum.z, v.w += sum.w;
     *dst = v;
 }
@@ -1193,7 +1194,7 @@ hipError_t launch_attn_bwd_f32(const Dims& d, BwdParams p, void* scratch, size_t
         if (e != hipSuccess) return e;
         const long n4 = a.part_half / 4;
         hipLaunchKernelGGL(attn_f32_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, a.part, a,
-                           d.seq, d.nkv * d.hd, p.group, p.dk, p.dv);
+                           d.seq, d.nkv * d.hd, p.group, p.acc, p.dk, p.dv);
         e = hipGetLastError();
     }
     if (e != hipSuccess) return e;

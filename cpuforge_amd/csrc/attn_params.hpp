@@ -51,6 +51,7 @@ struct BwdParams {
     float* dq;
     float* dk;
     float* dv;
+    int acc;  // kAccDq | kAccDk | kAccDv: the gradients added to; the others are overwritten
     int batch, seq, nh, nkv, hd, group;
     // dK/dV grid; xcd_cus: compute units per XCD, that is the workgroups of
     // one XCD's dispatch round for the one-workgroup-per-CU dK/dV kernels

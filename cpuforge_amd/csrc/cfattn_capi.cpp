@@ -11,8 +11,10 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "cfattn.h"
@@ -372,7 +374,7 @@ int cfattn_fwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const voi
 
 static int cfattn_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const void* d_o, const void* q, const void* k,
                const void* v, const float* o, const float* lse, float* dq, float* dk, float* dv, void* stream,
-               const cfattn::BwdEpilogue* epi = nullptr) {
+               const cfattn::BwdEpilogue* epi = nullptr, int acc = cfattn::kAccAll) {
     CF_TRY(check_dtype(c, dtype));
     if (batch == 0 || s.seq == 0) return CFATTN_OK;
     CF_TRY(check_shape(c, s));
@@ -386,7 +388,7 @@ static int cfattn_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batch, int dt
     size_t ds_bytes = 0;
     void* ds = ds_scratch(c, (Dtype)dtype, dims_of(s, batch), &ds_bytes);
     CF_HIP(c, cfattn::launch_attn_bwd((Dtype)dtype, dims_of(s, batch), d_o, q, k, v, o, lse, delta, dq, dk, dv,
-                                      pick_stream(c, stream), c->tuning(), ds, ds_bytes, epi),
+                                      pick_stream(c, stream), c->tuning(), ds, ds_bytes, epi, acc),
            "attention backward launch");
     return CFATTN_OK;
 }
@@ -398,6 +400,27 @@ int cfattn_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const voi
     c->err.clear();
     DeviceCallMark mark(c, pick_stream(c, stream));
     return cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq, dk, dv, stream);
+}
+
+// Zeros for the gradients of a call that has no rows to write them.
+static int zero_grads(cfattn_ctx* c, std::initializer_list<std::pair<float*, size_t>> grads, void* stream) {
+    DeviceGuard dg(c->device);
+    for (const auto& g : grads)
+        if (g.first) CF_HIP(c, cfattn::launch_fill_zero(g.first, g.second, pick_stream(c, stream)), "zero gradients");
+    return CFATTN_OK;
+}
+
+int cfattn_bwd_grad(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const void* d_o, const void* q,
+                    const void* k, const void* v, const float* o, const float* lse, float* dq, float* dk, float* dv,
+                    void* stream) {
+    if (!c) return CFATTN_ERR_ARG;
+    std::lock_guard<std::mutex> lk(c->mu);
+    c->err.clear();
+    DeviceCallMark mark(c, pick_stream(c, stream));
+    CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq, dk, dv, stream, nullptr, 0));
+    if (s.n_heads) return CFATTN_OK;
+    const size_t nk = batch * s.seq * s.n_kv * s.head_dim;
+    return zero_grads(c, {{dk, nk}, {dv, nk}}, stream);
 }
 
 int cfattn_bwd_noalloc(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const void* d_o, const void* q,
@@ -462,7 +485,7 @@ int cfattn_prologue_fwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, 
 static int cfattn_prologue_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batch, const cfattn_prologue* pr, const float* dq,
                         const float* dk, const float* q_pre, const float* k_pre, const float* q_rstd,
                         const float* k_rstd, float* dq_pre, float* dk_pre, float* dq_norm, float* dk_norm,
-                        void* stream, bool unrotated = false) {
+                        void* stream, bool unrotated = false, bool acc = true) {
     if (batch == 0 || s.seq == 0) return CFATTN_OK;
     CF_TRY(check_shape(c, s));
     CF_TRY(check_prologue(c, s, pr));
@@ -478,7 +501,8 @@ static int cfattn_prologue_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batc
         if (!partial) return rc;
     }
     CF_HIP(c, cfattn::launch_prologue_bwd(d, to_prologue(pr), dq, dk, q_pre, k_pre, q_rstd, k_rstd, dq_pre, dk_pre,
-                                          dq_norm, dk_norm, partial, pick_stream(c, stream), c->timer, unrotated),
+                                          dq_norm, dk_norm, partial, pick_stream(c, stream), c->timer, unrotated,
+                                          /*k_only=*/false, acc),
            "prologue backward launch");
     return CFATTN_OK;
 }
@@ -504,14 +528,11 @@ int cfattn_fused_fwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, con
     return cfattn_fwd_locked(c, s, batch, dtype, q_out, k_out, v, o, lse, stream);
 }
 
-int cfattn_fused_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const cfattn_prologue* pr,
+// `acc`: kAccAll adds to every gradient, 0 overwrites them.
+static int cfattn_fused_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const cfattn_prologue* pr,
                      const void* d_o, const float* q_pre, const float* k_pre, const void* q, const void* k,
                      const void* v, const float* o, const float* lse, const float* q_rstd, const float* k_rstd,
-                     float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream) {
-    if (!c) return CFATTN_ERR_ARG;
-    std::lock_guard<std::mutex> lk(c->mu);
-    c->err.clear();
-    DeviceCallMark mark(c, pick_stream(c, stream));
+                     float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream, int acc) {
     CF_TRY(check_dtype(c, dtype));
     if (batch == 0 || s.seq == 0) return CFATTN_OK;
     CF_TRY(check_shape(c, s));
@@ -536,7 +557,8 @@ int cfattn_fused_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, con
         epi.pos0 = P.pos0;
         if (!pr->q_norm) {
             epi.mode = cfattn::kEpiUnrotAdd;
-            return cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_pre, dk_pre, dv, stream, &epi);
+            return cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_pre, dk_pre, dv, stream, &epi,
+                                     acc);
         }
         if (!q_pre || !k_pre || !q_rstd || !k_rstd || !dq_norm || !dk_norm)
             return fail(c, CFATTN_ERR_ARG, "q/k norm backward needs q_pre, k_pre, rstd and gain-gradient buffers");
@@ -573,12 +595,13 @@ int cfattn_fused_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, con
             epi.norm.dkw = dk_norm;
             epi.norm.part = part;
             epi.norm.part_floats = nf;
-            CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_pre, dk_dst, dv, stream, &epi));
+            CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_pre, dk_dst, dv, stream, &epi,
+                                     acc));
             if (kfused) return CFATTN_OK;
             CF_HIP(c,
                    cfattn::launch_prologue_bwd(dd, P, nullptr, dk_dst, nullptr, k_pre, nullptr, k_rstd, nullptr, dk_pre,
                                                nullptr, dk_norm, part, pick_stream(c, stream), c->timer,
-                                               /*unrotated=*/true, /*k_only=*/true),
+                                               /*unrotated=*/true, /*k_only=*/true, acc != 0),
                    "prologue backward launch");
             return CFATTN_OK;
         }
@@ -587,21 +610,47 @@ int cfattn_fused_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, con
         if (!dy_q) return rc;
         float* dy_k = static_cast<float*>(slot(c, cfattn_ctx::DKROT, nk * 4, &rc));
         if (!dy_k) return rc;
-        CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dy_q, dy_k, dv, stream, &epi));
+        CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dy_q, dy_k, dv, stream, &epi,
+                                 acc));
         return cfattn_prologue_bwd_locked(c, s, batch, pr, dy_q, dy_k, q_pre, k_pre, q_rstd, k_rstd, dq_pre, dk_pre,
-                                          dq_norm, dk_norm, stream, /*unrotated=*/true);
+                                          dq_norm, dk_norm, stream, /*unrotated=*/true, acc != 0);
     }
     float* dq_rot = static_cast<float*>(slot(c, cfattn_ctx::DQROT, nq * 4, &rc));
     if (!dq_rot) return rc;
     float* dk_rot = static_cast<float*>(slot(c, cfattn_ctx::DKROT, nk * 4, &rc));
     if (!dk_rot) return rc;
-    hipStream_t st = pick_stream(c, stream);
-    // Layer::backward starts from zeroed dq/dk (layer.rs:183-185).
-    CF_HIP(c, cfattn::launch_fill_zero(dq_rot, nq, st), "zero dq");
-    CF_HIP(c, cfattn::launch_fill_zero(dk_rot, nk, st), "zero dk");
-    CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_rot, dk_rot, dv, stream));
+    // Layer::backward starts from zeroed dq/dk (layer.rs:183-185): written, not added to.
+    CF_TRY(cfattn_bwd_locked(c, s, batch, dtype, d_o, q, k, v, o, lse, dq_rot, dk_rot, dv, stream, nullptr,
+                             acc & cfattn::kAccDv));
     return cfattn_prologue_bwd_locked(c, s, batch, pr, dq_rot, dk_rot, q_pre, k_pre, q_rstd, k_rstd, dq_pre, dk_pre,
-                                      dq_norm, dk_norm, stream);
+                                      dq_norm, dk_norm, stream, /*unrotated=*/false, acc != 0);
+}
+
+int cfattn_fused_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const cfattn_prologue* pr,
+                     const void* d_o, const float* q_pre, const float* k_pre, const void* q, const void* k,
+                     const void* v, const float* o, const float* lse, const float* q_rstd, const float* k_rstd,
+                     float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream) {
+    if (!c) return CFATTN_ERR_ARG;
+    std::lock_guard<std::mutex> lk(c->mu);
+    c->err.clear();
+    DeviceCallMark mark(c, pick_stream(c, stream));
+    return cfattn_fused_bwd_locked(c, s, batch, dtype, pr, d_o, q_pre, k_pre, q, k, v, o, lse, q_rstd, k_rstd, dq_pre,
+                                   dk_pre, dv, dq_norm, dk_norm, stream, cfattn::kAccAll);
+}
+
+int cfattn_fused_bwd_grad(cfattn_ctx* c, cfattn_shape s, size_t batch, int dtype, const cfattn_prologue* pr,
+                          const void* d_o, const float* q_pre, const float* k_pre, const void* q, const void* k,
+                          const void* v, const float* o, const float* lse, const float* q_rstd, const float* k_rstd,
+                          float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream) {
+    if (!c) return CFATTN_ERR_ARG;
+    std::lock_guard<std::mutex> lk(c->mu);
+    c->err.clear();
+    DeviceCallMark mark(c, pick_stream(c, stream));
+    CF_TRY(cfattn_fused_bwd_locked(c, s, batch, dtype, pr, d_o, q_pre, k_pre, q, k, v, o, lse, q_rstd, k_rstd, dq_pre,
+                                   dk_pre, dv, dq_norm, dk_norm, stream, 0));
+    if (batch && s.seq && s.n_heads) return CFATTN_OK;
+    const size_t nk = batch * s.seq * s.n_kv * s.head_dim;
+    return zero_grads(c, {{dk_pre, nk}, {dv, nk}, {dq_norm, s.head_dim}, {dk_norm, s.head_dim}}, stream);
 }
 
 double cfattn_llama3_scale(const cfattn_llama3_scaling* sc, double inv_freq) {

@@ -121,7 +121,7 @@ hipError_t launch_attn_fwd(Dtype dt, const Dims& d, const void* q, const void* k
                            size_t scratch_bytes = 0);
 
 // Backward.  `delta` is caller-provided scratch of batch*n_heads*seq floats.
-// dq, dk, dv are accumulated (+=).
+// dq, dk, dv are accumulated (+=) or overwritten (`acc` below).
 //
 // `ds` is optional scratch for the stored-dS dQ path: when it is non-null
 // and `ds_bytes` >= attn_bwd_ds_bytes(dt, d), and the fast bf16 kernels run,
@@ -134,11 +134,14 @@ hipError_t launch_attn_fwd(Dtype dt, const Dims& d, const void* q, const void* k
 // recomputing it (the same bits).
 size_t attn_bwd_ds_bytes(Dtype dt, const Dims& d);
 size_t attn_f32_scratch_bytes(const Dims& d);
-// How the fast bf16 kernels write the dQ and dK rows (dV rows are always
+// How the fast bf16 kernels write the dQ and dK rows (dV rows are
 // added).  The inverse-RoPE modes fold the prologue backward's rotation
 // (RopeCache::apply with inverse = true, rope.rs:71-89) into the kernels:
 // row t of a sequence is unrotated with cos/sin row pos0 + t of the
 // [max_pos][head_dim/2] tables, elementwise as the prologue backward does.
+// A += below, and dV's, is = for a gradient that `acc` of launch_attn_bwd does
+// not name.
+enum Accumulate { kAccDq = 1, kAccDk = 2, kAccDv = 4, kAccAll = 7 };
 enum EpilogueMode {
     kEpiAdd = 0,          // dq/dk += rows
     kEpiUnrotAdd = 1,     // dq/dk += inverse-RoPE(rows)
@@ -187,10 +190,17 @@ bool attn_bwd_norm_dk_epilogue(const Dims& d, const Tuning& tu);
 size_t attn_bwd_norm_part_floats(const Dims& d, const Tuning& tu);
 // The fixed-order reduction of the partials (prologue.hip): dqw[i] += the sum
 // over rows [0, nq) of part[.][i], dkw[i] over rows [nq, nq + nk).
-hipError_t launch_norm_gain_reduce(float* part, int nq, int nk, int hd, float* dqw, float* dkw, hipStream_t st);
+hipError_t launch_norm_gain_reduce(float* part, int nq, int nk, int hd, float* dqw, float* dkw, bool acc,
+                                   hipStream_t st);
 // With f32 inputs the same scratch (when large enough) holds the per-head
 // dK/dV contributions of the fp32 fast path (attn_f32.hip), which
 // attn_bwd_ds_bytes reports for kF32.
+// The gradients named in `acc` are added to, the others overwritten: every
+// element is written and none read, so the caller needs no fill.  With
+// kEpiUnrotNorm the gain gradients follow kAccDq.  What the fill and the reads
+// cost, forward and backward together: bf16 B1 S8192 32/8 D128 2.05 ms with
+// zeroed buffers, 1.99 overwritten; B4 S4096 32/8 D64 with RoPE 1.68, 1.62;
+// 16/8 D128 with q/k norm 1.54, 1.41; fp32 B8 S2048 9/3 D64 1.156, 1.126.
 // A non-default `epi` needs attn_bwd_epilogue_applies and 16-byte aligned
 // cos/sin tables; kEpiUnrotNorm also 16-byte aligned pre-norm rows and gains
 // and part_floats >= attn_bwd_norm_part_floats (hipErrorInvalidValue
@@ -199,7 +209,7 @@ hipError_t launch_norm_gain_reduce(float* part, int nq, int nk, int hd, float* d
 hipError_t launch_attn_bwd(Dtype dt, const Dims& d, const void* d_o, const void* q, const void* k, const void* v,
                            const float* o, const float* lse, float* delta, float* dq, float* dk, float* dv,
                            hipStream_t st, const Tuning& tu, void* ds = nullptr, size_t ds_bytes = 0,
-                           const BwdEpilogue* epi = nullptr);
+                           const BwdEpilogue* epi = nullptr, int acc = kAccAll);
 
 // Attention prologue: optional per-head RMSNorm of q_pre/k_pre (when qw/kw
 // are non-null) followed by rotate-half RoPE at positions pos0+t, written in
@@ -227,7 +237,8 @@ size_t prologue_bwd_scratch_floats(const Dims& d);
 hipError_t launch_prologue_bwd(const Dims& d, const Prologue& pr, const float* dq, const float* dk,
                                const float* q_pre, const float* k_pre, const float* q_rstd, const float* k_rstd,
                                float* dq_pre, float* dk_pre, float* dqw, float* dkw, float* partial, hipStream_t st,
-                               KernelTimer* timer = nullptr, bool unrotated = false, bool k_only = false);
+                               KernelTimer* timer = nullptr, bool unrotated = false, bool k_only = false,
+                               bool acc = true);
 
 // Elementwise helpers.
 hipError_t launch_f32_to_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t st);

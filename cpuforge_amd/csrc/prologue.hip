@@ -252,6 +252,7 @@ struct ProBwdParams {
     long rows_q, rows_k;
     int chunk_rows, n_chunks_q, n_chunks_k;
     int srows;  // rows per block of the staged kernel
+    int acc;    // 0: dq_pre, dk_pre, dqw and dkw are overwritten (not read) instead of added to
     int unrot;  // 0: dq/dk are already unrotated (the backward's kEpiUnrotStore epilogue)
 };
 
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(256) void prologue_bwd_rows_kernel(const ProBwdPara
     const float* sn = p.sin + (long)(p.pos0 + t) * p.half;
     auto dyv = [&](int i) { return p.unrot ? unrotate(g, cs, sn, i, p.half) : g[i]; };
     if (!w) {
-        for (int i = 0; i < p.hd; i++) dx[i] += dyv(i);
+        for (int i = 0; i < p.hd; i++) dx[i] = (p.acc ? dx[i] : 0.0f) + dyv(i);
         return;
     }
     const float* x = (isq ? p.q_pre : p.k_pre) + r * p.hd;
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(256) void prologue_bwd_rows_kernel(const ProBwdPara
     for (int i = 0; i < p.hd; i++) {
         const float dy = dyv(i);
         const float xhat = x[i] * inv;
-        dx[i] += inv * (dy * w[i] - xhat * mean);
+        dx[i] = (p.acc ? dx[i] : 0.0f) + inv * (dy * w[i] - xhat * mean);
     }
 }
 
@@ -326,6 +327,10 @@ __global__ __launch_bounds__(256) void prologue_bwd_rows_staged_kernel(const Pro
     float* smean = stage + 2 * p.srows * LD;
     float* sw = smean + p.srows;
     float* dx = (isq ? p.dq_pre : p.dk_pre) + r0 * D;
+    auto put = [&](int row, int i, float v) {
+        float* dst = dx + (long)row * D + i;
+        *dst = (p.acc ? *dst : 0.0f) + v;
+    };
     auto dy_pair = [&](int row, int i, float& dy1, float& dy2) {
         const int t = (int)(((r0 + row) / heads) % p.seq);
         const float* cs = p.cos + (long)(p.pos0 + t) * half;
@@ -344,8 +349,8 @@ __global__ __launch_bounds__(256) void prologue_bwd_rows_staged_kernel(const Pro
             const int row = j / half, i = j % half;
             float dy1, dy2;
             dy_pair(row, i, dy1, dy2);
-            dx[(long)row * D + i] += dy1;
-            dx[(long)row * D + i + half] += dy2;
+            put(row, i, dy1);
+            put(row, i + half, dy2);
         }
         return;
     }
@@ -381,8 +386,8 @@ __global__ __launch_bounds__(256) void prologue_bwd_rows_staged_kernel(const Pro
         const float inv = rstd[row], mean = smean[row];
         const float dy1 = sdy[row * LD + i], dy2 = sdy[row * LD + i + half];
         const float xh1 = sx[row * LD + i] * inv, xh2 = sx[row * LD + i + half] * inv;
-        dx[(long)row * D + i] += inv * (dy1 * sw[i] - xh1 * mean);
-        dx[(long)row * D + i + half] += inv * (dy2 * sw[i + half] - xh2 * mean);
+        put(row, i, inv * (dy1 * sw[i] - xh1 * mean));
+        put(row, i + half, inv * (dy2 * sw[i + half] - xh2 * mean));
     }
 }
 
@@ -469,8 +474,8 @@ __global__ __launch_bounds__(256) void prologue_bwd_norm_vec_kernel(const ProBwd
         if (ok) {
             const float mean = dot / (float)D;
             float* dx = dxbase + r * D + d0;
-            float o[8];
-            load8(dx, o);
+            float o[8] = {};
+            if (p.acc) load8(dx, o);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float xh = x[i] * inv;
@@ -541,7 +546,10 @@ __global__ __launch_bounds__(256) void prologue_bwd_dw_reduce_kernel(const ProBw
         if (tid < w) red[tid] = red[tid] + red[tid + w];
         __syncthreads();
     }
-    if (tid == 0) (isq ? p.dqw : p.dkw)[i] += red[0];
+    if (tid == 0) {
+        float* dw = (isq ? p.dqw : p.dkw) + i;
+        *dw = (p.acc ? *dw : 0.0f) + red[0];
+    }
 }
 
 __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restrict__ src, uint16_t* __restrict__ dst,
@@ -639,8 +647,9 @@ size_t prologue_bwd_scratch_floats(const Dims& d) {
 hipError_t launch_prologue_bwd(const Dims& d, const Prologue& pr, const float* dq, const float* dk,
                                const float* q_pre, const float* k_pre, const float* q_rstd, const float* k_rstd,
                                float* dq_pre, float* dk_pre, float* dqw, float* dkw, float* partial, hipStream_t st,
-                               KernelTimer* timer, bool unrotated, bool k_only) {
+                               KernelTimer* timer, bool unrotated, bool k_only, bool acc) {
     ProBwdParams p{};
+    p.acc = acc;
     p.unrot = unrotated ? 0 : 1;
     p.dq = dq;
     p.dk = dk;
@@ -709,9 +718,11 @@ hipError_t launch_prologue_bwd(const Dims& d, const Prologue& pr, const float* d
     return hipGetLastError();
 }
 
-hipError_t launch_norm_gain_reduce(float* part, int nq, int nk, int hd, float* dqw, float* dkw, hipStream_t st) {
+hipError_t launch_norm_gain_reduce(float* part, int nq, int nk, int hd, float* dqw, float* dkw, bool acc,
+                                   hipStream_t st) {
     if (hd <= 0) return hipSuccess;
     ProBwdParams p{};
+    p.acc = acc;
     p.partial = part;
     p.n_chunks_q = nq;
     p.n_chunks_k = nk;

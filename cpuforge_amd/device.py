@@ -11,7 +11,6 @@ and lse; backward accumulates into dq, dk, dv (crates/core/src/ops/mod.rs:1-6).
 from __future__ import annotations
 
 import ctypes as C
-import math
 
 import torch
 
@@ -56,14 +55,6 @@ def _stream() -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def _zeros(device, *shapes):
-    """Zero float32 tensors of the given shapes (None entries stay None) from
-    one allocation, filled in one launch; each starts 256 bytes aligned."""
-    sizes = [0 if sh is None else (math.prod(sh) + 63) // 64 * 64 for sh in shapes]
-    flat = torch.zeros(sum(sizes), dtype=torch.float32, device=device)
-    return [None if sh is None else part[:math.prod(sh)].view(sh) for sh, part in zip(shapes, flat.split(sizes))]
-
-
 def fwd(q, k, v, o=None, lse=None, ctx: Context | None = None):
     """Causal GQA attention forward; returns (o, lse)."""
     ctx = ctx or default_context()
@@ -88,7 +79,8 @@ def fwd(q, k, v, o=None, lse=None, ctx: Context | None = None):
 
 
 def bwd(d_o, q, k, v, o, lse, dq=None, dk=None, dv=None, ctx: Context | None = None):
-    """Backward; accumulates into dq, dk, dv (zero-initialised if None)."""
+    """Backward; accumulates into dq, dk, dv.  A None is a new tensor (written
+    without a fill when all three are None, zeros otherwise)."""
     ctx = ctx or default_context()
     B, s = _batched(q, k)
     dt = _code(q)
@@ -97,15 +89,16 @@ def bwd(d_o, q, k, v, o, lse, dq=None, dk=None, dv=None, ctx: Context | None = N
     _need(d_o, "d_o", q.shape)
     _need(o, "o", q.shape, torch.float32)
     _need(lse, "lse", (B, s.n_heads, s.seq) if q.dim() == 4 else (s.n_heads, s.seq), torch.float32)
-    if dq is None or dk is None or dv is None:
-        z = _zeros(q.device, None if dq is not None else q.shape, None if dk is not None else k.shape,
-                   None if dv is not None else k.shape)
-        dq, dk, dv = (g if g is not None else n for g, n in zip((dq, dk, dv), z))
+    fresh = dq is None and dk is None and dv is None
+    new = torch.empty if fresh else torch.zeros
+    dq, dk, dv = (new(sh, dtype=torch.float32, device=q.device) if g is None else g
+                  for g, sh in ((dq, q.shape), (dk, k.shape), (dv, k.shape)))
     _need(dq, "dq", q.shape, torch.float32)
     _need(dk, "dk", k.shape, torch.float32)
     _need(dv, "dv", k.shape, torch.float32)
-    rc = ctx._lib.cfattn_bwd(ctx.handle, s.c(), B, dt, d_o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                             o.data_ptr(), lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), _stream())
+    call = ctx._lib.cfattn_bwd_grad if fresh else ctx._lib.cfattn_bwd
+    rc = call(ctx.handle, s.c(), B, dt, d_o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+              lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), _stream())
     _lib.check(rc, ctx.handle)
     return dq, dk, dv
 
@@ -201,22 +194,24 @@ def fused_fwd(q_pre, k_pre, v, pr: DeviceRope, ctx: Context | None = None):
 def fused_bwd(d_o, q_pre, k_pre, q, k, v, o, lse, q_rstd, k_rstd, pr: DeviceRope, dq_pre=None, dk_pre=None, dv=None,
               dq_norm=None, dk_norm=None, ctx: Context | None = None):
     """Attention backward + prologue backward; accumulates and returns
-    (dq_pre, dk_pre, dv, dq_norm, dk_norm)."""
+    (dq_pre, dk_pre, dv, dq_norm, dk_norm); a None is a new tensor (as in bwd)."""
     ctx = ctx or default_context()
     B, s = _batched(q_pre, k_pre)
     dev = q_pre.device
     norm = (s.head_dim,) if pr.q_norm is not None else None
     given = (dq_pre, dk_pre, dv, dq_norm, dk_norm)
     shapes = (q_pre.shape, k_pre.shape, k_pre.shape, norm, norm)
-    if any(g is None and sh is not None for g, sh in zip(given, shapes)):
-        z = _zeros(dev, *(None if g is not None else sh for g, sh in zip(given, shapes)))
-        dq_pre, dk_pre, dv, dq_norm, dk_norm = (g if g is not None else n for g, n in zip(given, z))
+    fresh = all(g is None for g in given)
+    new = torch.empty if fresh else torch.zeros
+    dq_pre, dk_pre, dv, dq_norm, dk_norm = (
+        new(sh, dtype=torch.float32, device=dev) if g is None and sh is not None else g
+        for g, sh in zip(given, shapes))
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
     prc = pr.c()
-    rc = ctx._lib.cfattn_fused_bwd(ctx.handle, s.c(), B, _code(q), C.byref(prc), d_o.data_ptr(), q_pre.data_ptr(),
-                                   k_pre.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                   lse.data_ptr(), ptr(q_rstd), ptr(k_rstd), dq_pre.data_ptr(), dk_pre.data_ptr(),
-                                   dv.data_ptr(), ptr(dq_norm), ptr(dk_norm), _stream())
+    call = ctx._lib.cfattn_fused_bwd_grad if fresh else ctx._lib.cfattn_fused_bwd
+    rc = call(ctx.handle, s.c(), B, _code(q), C.byref(prc), d_o.data_ptr(), q_pre.data_ptr(), k_pre.data_ptr(),
+              q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), ptr(q_rstd), ptr(k_rstd),
+              dq_pre.data_ptr(), dk_pre.data_ptr(), dv.data_ptr(), ptr(dq_norm), ptr(dk_norm), _stream())
     _lib.check(rc, ctx.handle)
     return dq_pre, dk_pre, dv, dq_norm, dk_norm
 

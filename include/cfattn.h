@@ -137,6 +137,13 @@ int cfattn_bwd(cfattn_ctx* ctx, cfattn_shape s, size_t batch, int dtype, const v
                const void* k, const void* v, const float* o, const float* lse, float* dq, float* dk, float* dv,
                void* stream);
 
+/* cfattn_bwd into gradients that hold nothing yet: writes every element of
+ * dq, dk and dv and reads none (the results of zeroed buffers without the
+ * fill and the read). */
+int cfattn_bwd_grad(cfattn_ctx* ctx, cfattn_shape s, size_t batch, int dtype, const void* d_o, const void* q,
+                    const void* k, const void* v, const float* o, const float* lse, float* dq, float* dk, float* dv,
+                    void* stream);
+
 /* No reference counterpart.  cfattn_bwd that allocates nothing, for callers
  * that cannot call hipMalloc (code under HIP graph capture, tight serving
  * loops, harnesses that forbid allocation).  The same arguments, results and
@@ -180,6 +187,11 @@ int cfattn_fused_bwd(cfattn_ctx* ctx, cfattn_shape s, size_t batch, int dtype, c
                      const void* d_o, const float* q_pre, const float* k_pre, const void* q, const void* k,
                      const void* v, const float* o, const float* lse, const float* q_rstd, const float* k_rstd,
                      float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream);
+/* cfattn_fused_bwd that overwrites its gradients (cfattn_bwd_grad). */
+int cfattn_fused_bwd_grad(cfattn_ctx* ctx, cfattn_shape s, size_t batch, int dtype, const cfattn_prologue* pr,
+                          const void* d_o, const float* q_pre, const float* k_pre, const void* q, const void* k,
+                          const void* v, const float* o, const float* lse, const float* q_rstd, const float* k_rstd,
+                          float* dq_pre, float* dk_pre, float* dv, float* dq_norm, float* dk_norm, void* stream);
 
 /* ---- host helpers ---------------------------------------------------------- */
 /* RopeCache::with_scaling (core/src/ops/rope.rs:46-63): cos/sin tables
