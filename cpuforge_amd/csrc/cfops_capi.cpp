@@ -32,6 +32,12 @@ int launch_gemm(cfattn_ctx* c, const cfattn::GemmF32& g, hipStream_t st) {
     return CFATTN_OK;
 }
 
+// An overwritten gradient of a call without rows: the empty sum.
+int zero_grad(cfattn_ctx* c, float* g, size_t n, hipStream_t st) {
+    if (g && n) CF_HIP(c, cfattn::launch_fill_zero(g, n, st), "zero-fill launch");
+    return CFATTN_OK;
+}
+
 // Row-major C[m,n] = op(A) op(B) (+ C when acc), as matmul.rs's
 // matmul_nn / matmul_nt / matmul_tn (core/src/matmul.rs:127-147).
 int gemm(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, size_t m, size_t k, size_t n, bool acc,
@@ -192,6 +198,7 @@ int cfops_rmsnorm_backward(cfattn_ctx* c, const float* dy, const float* x, const
 int cfops_rmsnorm_grad(cfattn_ctx* c, const float* dy, const float* x, const float* w, const float* rstd, float* dx,
                        float* dw, size_t rows, size_t dim, int acc, void* stream) {
     CF_LOCK(c);
+    if (rows == 0 && !acc) return zero_grad(c, dw, dim, to_stream(stream));
     if (rows == 0 || dim == 0) return CFATTN_OK;
     if (!dy || !x || !w || !rstd || !dx) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (!fits_int(dim)) return fail(c, CFATTN_ERR_UNSUPPORTED, "dim=%zu above 2^31", dim);
@@ -368,6 +375,13 @@ int cfops_linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, co
 int cfops_linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin,
                            size_t n, int acc, void* stream) {
     CF_LOCK(c);
+    if (t == 0 && !acc)
+        for (size_t i = 0; lin && i < n; i++) {
+            const cfops_linear& l = lin[i];
+            CF_TRY(zero_grad(c, l.gw, l.out * in, to_stream(stream)));
+            CF_TRY(zero_grad(c, l.ga, l.rank * in, to_stream(stream)));
+            CF_TRY(zero_grad(c, l.gb, l.out * l.rank, to_stream(stream)));
+        }
     if (t == 0 || n == 0) return CFATTN_OK;
     if (!x || !lin) return fail(c, CFATTN_ERR_ARG, "null buffer");
     for (size_t i = 0; i < n; i++) {

@@ -47,3 +47,23 @@ def test_silu_mul_backward_overwrites(n):
     out = [torch.full((n,), float("nan"), device=DEV) for _ in range(2)]
     P.silu_mul_backward(dh, a, u, *out, acc=False)
     assert all(torch.equal(x, z) for x, z in zip(out, zeros))
+
+
+def test_gradients_of_no_rows_are_zero():
+    """A sum over no rows overwrites its gradient with zeros, as a zeroed buffer left it."""
+    from cpuforge_amd import autograd as A
+    from cpuforge_amd import ops as P
+    nan = lambda *s: torch.full(s, float("nan"), device=DEV)  # noqa: E731
+    x = torch.empty(0, 24, device=DEV)
+    dw = nan(24)
+    P.rmsnorm_backward(x, x, torch.ones(24, device=DEV), torch.empty(0, device=DEV), torch.empty_like(x), dw, 0, 24,
+                       acc=False)
+    assert bool((dw == 0).all())
+    w, a, b = (torch.randn(*s, device=DEV) for s in ((40, 24), (4, 24), (40, 4)))
+    li = dict(w=w, lora_a=a, lora_b=b, scale=2.0, xs=torch.empty(0, 4, device=DEV), dy=torch.empty(0, 40, device=DEV),
+              gw=nan(40, 24), ga=nan(4, 24), gb=nan(40, 4))
+    P.linears_backward(x, 0, 24, torch.empty_like(x), [li], acc=False)
+    assert all(bool((li[n] == 0).all()) for n in ("gw", "ga", "gb"))
+    leaves = [t.requires_grad_() for t in (w, a, b)]
+    grads = torch.autograd.grad(A.linear(x, w, a, b, 2.0).sum(), leaves)
+    assert all(bool((g == 0).all()) for g in grads)
