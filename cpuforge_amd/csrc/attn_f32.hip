@@ -1,8 +1,8 @@
 // fp32 parity mode on gfx950: causal GQA attention forward, dQ and dK/dV with
 // f32 inputs and v_mfma_f32_32x32x2_f32 (exact f32 products, f32
 // accumulation), for head_dim 64 and 128 with 16-byte aligned rows.  The
-// forward's units run on the bf16 matrix cores (attn_f32x3.hpp), the f32 one
-// below where a result is not finite.
+// forward's units from kX3MinSeq positions on run on the bf16 matrix cores (attn_f32x3.hpp), the f32 one
+// below for shorter sequences and where a result is not finite.
 //
 // An f32 MFMA takes one value per lane and operand (lane l: A[l%32][l/32],
 // B[l/32][l%32]), so every operand is read row-major:
@@ -101,6 +101,25 @@ __device__ __forceinline__ void f32_step_end(bool newer) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// lse in the exponent's units, lse log2(e) = hi + lo: rounded to one float, a
+// row's P are all off by up to 2^-24 lse log2(e). With it, and lse rounded once
+// (lse_of), attention at S512 9/3 D64 is 4.3e-7 off where it was 4.6e-7. (The
+// forward's scores on split operands do not carry the rounding of the f32 products
+// that the backward forms again, which cancelled in P: see kX3MinSeq.) Costs
+// 2% of the step at B8 S2048 (1134 -> 1158 us). Infinite and NaN lse stay what they are.
+struct LseLog2 {
+    float hi, lo;
+};
+__device__ __forceinline__ LseLog2 lse_log2(float lse) {
+    constexpr float kLog2eLo = (float)(1.4426950408889634 - (double)kLog2e);
+    const float hi = lse * kLog2e;
+    const float lo = __builtin_fmaf(lse, kLog2eLo, __builtin_fmaf(lse, kLog2e, -hi));
+    return {hi, fabsf(hi) < INFINITY ? lo : 0.0f};
+}
+__device__ __forceinline__ float prob_f32(float score, float sl2, const LseLog2& l) {
+    return __builtin_amdgcn_exp2f(__builtin_fmaf(score, sl2, -l.hi) - l.lo);
 }
 
 // Stored fp32 dS block (32 queries x 32 keys): the value of query row q and
@@ -301,15 +320,23 @@ __device__ __forceinline__ void fwd_f32_unit(const FwdParams& p, const F32Unit u
             *reinterpret_cast<float4*>(orow + db * 32 + rq * 8 + hh * 4) =
                 make_float4(oacc[db][rq * 4] * inv, oacc[db][rq * 4 + 1] * inv, oacc[db][rq * 4 + 2] * inv,
                             oacc[db][rq * 4 + 3] * inv);
-    if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = (m2 + __log2f(ltot)) * kLn2;
+    if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = lse_of(m2, ltot);
 }
+
+// Shortest sequence on split operands. The rounding of the backward's f32 scores
+// cancels in P = exp(S - lse) where the forward's lse has the same scores in it, the
+// more the fewer keys a row has. Split against f32 forward: o 0.07 / 0.13, 0.10 /
+// 0.20, 0.11 / 0.23, 0.13 / 0.28 parts in 10^6 off at S 20, 100, 300, 1500; dq
+// 0.32 / 0.30, 0.36 / 0.35, 0.40 / 0.40, 0.52 / 0.51. Below it a call is a launch and
+// a few tiles, and neither is faster.
+constexpr int kX3MinSeq = 128;
 
 // One unit: on the bf16 matrix cores, or where a result is not finite with
 // f32 MFMAs (after the workgroup's vote every LDS read is done; the loads still
 // in flight are waited for, as fwd_f32_unit counts its own).
 template <int DP>
 __device__ __forceinline__ void fwd_unit(const FwdParams& p, const F32Unit un, int rest, uint4* sm) {
-    if (fwd_x3_unit<DP>(p, un, rest, sm)) return;
+    if (p.seq >= kX3MinSeq && fwd_x3_unit<DP>(p, un, rest, sm)) return;
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     float* s = reinterpret_cast<float*>(sm);
     constexpr int N = 32 * DP;
@@ -384,7 +411,7 @@ __device__ __forceinline__ void dq_f32_unit(const BwdParams& p, const F32Unit un
         of[4 * i] = c.x, of[4 * i + 1] = c.y, of[4 * i + 2] = c.z, of[4 * i + 3] = c.w;
     }
     const long lrow = ((long)b * p.nh + head) * p.seq + min(tq, p.seq - 1);
-    const float lq = p.lse[lrow] * kLog2e;
+    const LseLog2 lq = lse_log2(p.lse[lrow]);
     const float dlq = p.delta[lrow];
     // The rows above and tile kt0 have landed; a wait the compiler sees (see
     // the forward).
@@ -417,7 +444,7 @@ __device__ __forceinline__ void dq_f32_unit(const BwdParams& p, const F32Unit un
             float ds[16];
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], p.sl2, -lq));
+                float pv = prob_f32(sc[r], p.sl2, lq);
                 if (masked && k0 + acc_row(r, hh) > tq) pv = 0.0f;
                 ds[r] = pv * (dp[r] - dlq);
             }
@@ -747,13 +774,13 @@ __device__ __forceinline__ void dkdv_f32_unit(const BwdParams& p, const F32DkdvA
             for (int g4 = 0; g4 < 4; g4++) {
                 const float4 l4 = *reinterpret_cast<const float4*>(LDs + g4 * 8 + hh * 4);
                 const float4 d4 = *reinterpret_cast<const float4*>(LDs + BM + g4 * 8 + hh * 4);
-                const float lv[4] = {l4.x * kLog2e, l4.y * kLog2e, l4.z * kLog2e, l4.w * kLog2e};
+                const LseLog2 lv[4] = {lse_log2(l4.x), lse_log2(l4.y), lse_log2(l4.z), lse_log2(l4.w)};
                 const float dv[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int r = g4 * 4 + i;
                     const int qr = q0 + acc_row(r, hh);
-                    float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], p.sl2, -lv[i]));
+                    float pv = prob_f32(sc[r], p.sl2, lv[i]);
                     if (masked && (kw > qr || qr >= p.seq)) pv = 0.0f;
                     pr[r] = pv;
                     ds[r] = pv * (dp[r] - dv[i]);
@@ -913,7 +940,7 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_merge_kernel(const FwdParams
     const long b = bh / p.nh, head = bh % p.nh;
     float* orow = p.o + b * p.q_bs + (long)tq * p.nh * DP + head * DP;
     reinterpret_cast<float4*>(orow)[c] = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
-    if (c == 0) p.lse[row] = (m + __log2f(l)) * kLn2;
+    if (c == 0) p.lse[row] = lse_of(m, l);
 }
 
 // dq += (or =, p.acc) sum over the splits of a row, in split order.

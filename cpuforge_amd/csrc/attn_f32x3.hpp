@@ -133,6 +133,9 @@ __device__ __forceinline__ void row_ops(const float* __restrict__ row, int hh, O
     }
 }
 
+// (m + log2(l)) ln 2, the larger sum rounded once.
+__device__ __forceinline__ float lse_of(float m, float l) { return __builtin_fmaf(m, kLn2, __log2f(l) * kLn2); }
+
 // LDS of a step is written and read; loads to registers stay in flight.
 __device__ __forceinline__ void x3_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -289,7 +292,7 @@ __device__ __forceinline__ bool fwd_x3_unit(const FwdParams& p, const F32Unit un
             *reinterpret_cast<float4*>(orow + db * 32 + rq * 8 + hh * 4) =
                 make_float4(oacc[db][rq * 4] * inv, oacc[db][rq * 4 + 1] * inv, oacc[db][rq * 4 + 2] * inv,
                             oacc[db][rq * 4 + 3] * inv);
-    if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = (m2 + __log2f(ltot)) * kLn2;
+    if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = lse_of(m2, ltot);
     return true;
 }
 
