@@ -515,10 +515,10 @@ hipError_t launch_silu_mul_bwd(const float* dh, const float* g, const float* u, 
 
 // ----------------------------------------------------------- cross-entropy
 constexpr long kIgnoreIndex = -100;  // crates/core/src/ops/loss.rs:4
-constexpr int kCeThreads = 512;
 
-// Block-wide max / sum over kCeThreads threads in a fixed order: within each
-// wave by xor shuffles, then the eight wave results in wave order.
+// Block-wide max / sum over NT threads in a fixed order: within each wave by
+// xor shuffles, then the wave results the same way.
+template <int NT>
 __device__ __forceinline__ float block_reduce(float v, bool is_max, float* sred) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
@@ -528,8 +528,13 @@ __device__ __forceinline__ float block_reduce(float v, bool is_max, float* sred)
     __syncthreads();  // sred is free (an earlier reduction's readers are done)
     if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = v;
     __syncthreads();
-    float r = sred[0];
-    for (int i = 1; i < kCeThreads / 64; i++) r = is_max ? fmaxf(r, sred[i]) : radd(r, sred[i]);
+    // (All NT / 64 results in one lane's registers would be a wave less in flight.)
+    float r = sred[threadIdx.x % (NT / 64)];
+#pragma unroll
+    for (int o = NT / 128; o >= 1; o >>= 1) {
+        const float w = __shfl_xor(r, o);
+        r = is_max ? fmaxf(r, w) : radd(r, w);
+    }
     return r;
 }
 
@@ -552,11 +557,15 @@ __global__ __launch_bounds__(256) void ce_begin_kernel(const int64_t* __restrict
 // One row per workgroup (loss.rs:27-53).  With NV4 > 0 the row stays in
 // registers (NV4 float4 per thread) between the max, the exp sum and the
 // write, so it is read from memory once; NV4 == 0 streams it three times.
-template <int NV4>
-__global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(const float* logits, const int64_t* __restrict__ targets,
+// A CU must have the reads of one row beside the writes of another: with the
+// 64 registers of eight waves to a SIMD, two rows of 1024 threads are at work,
+// where 512 threads of 32 float4 left room for one and memory idle in its
+// reductions (2048 x 49152 on average, 805 MB: 232 -> 154 us, 3.5 -> 5.2 TB/s).
+template <int NV4, int NT>
+__global__ __launch_bounds__(NT, NV4 == 12 || NV4 == 8 ? 8 : 1) void ce_rows_kernel(const float* logits, const int64_t* __restrict__ targets,
                                                              float* dlogits, float* __restrict__ row_loss, long row0,
                                                              long vocab, CeMisc* __restrict__ m) {
-    __shared__ float sred[kCeThreads / 64];
+    __shared__ float sred[NT / 64];
     const long r = row0 + blockIdx.x;
     const int64_t t = targets[r];
     const float* lr = logits + (long)blockIdx.x * vocab;
@@ -564,7 +573,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(const float* logits
     const int tid = threadIdx.x;
     if (t == kIgnoreIndex || t < 0 || t >= vocab) {
         if (t != kIgnoreIndex && tid == 0) atomicMin(&m->bad_row, (int)r);
-        for (long i = tid; i < vocab; i += kCeThreads) dr[i] = 0.0f;
+        for (long i = tid; i < vocab; i += NT) dr[i] = 0.0f;
         if (tid == 0) row_loss[r] = 0.0f;
         return;
     }
@@ -572,60 +581,49 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(const float* logits
     const float lt = lr[t];
     float mx = -INFINITY;
     if constexpr (NV4 > 0) {
-        const long nv = vocab / 4;
+        const int nv = (int)(vocab / 4);
+        const unsigned at = 16u * (unsigned)tid;  // beside uniform addresses: one register for all
+        auto in = [&](int i) { return tid < nv - i * NT; };
         float4 v[NV4];
 #pragma unroll
-        for (int i = 0; i < NV4; i++) {
-            const long idx = (long)i * kCeThreads + tid;
-            if (idx < nv) {
-                v[i] = reinterpret_cast<const float4*>(lr)[idx];
+        for (int i = 0; i < NV4; i++)
+            if (in(i)) {
+                v[i] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(lr + (long)i * NT * 4) + at);
                 mx = fmaxf(mx, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
             }
-        }
-        mx = block_reduce(mx, true, sred);
+        mx = block_reduce<NT>(mx, true, sred);
         float sum = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NV4; i++) {
-            const long idx = (long)i * kCeThreads + tid;
-            if (idx < nv) {
+        for (int i = 0; i < NV4; i++)
+            if (in(i)) {
                 v[i].x = expf(rsub(v[i].x, mx));
                 v[i].y = expf(rsub(v[i].y, mx));
                 v[i].z = expf(rsub(v[i].z, mx));
                 v[i].w = expf(rsub(v[i].w, mx));
                 sum = radd(sum, radd(radd(v[i].x, v[i].y), radd(v[i].z, v[i].w)));
+                __builtin_amdgcn_sched_barrier(0);  // (several expf at once take more registers than there are)
             }
-        }
-        sum = block_reduce(sum, false, sred);
+        sum = block_reduce<NT>(sum, false, sred);
         const float sc = rmul(rdiv(1.0f, sum), inv_n);
 #pragma unroll
-        for (int i = 0; i < NV4; i++) {
-            const long idx = (long)i * kCeThreads + tid;
-            if (idx < nv) {
-                float4 d = make_float4(rmul(v[i].x, sc), rmul(v[i].y, sc), rmul(v[i].z, sc),
-                                       rmul(v[i].w, sc));
-                const long e = idx * 4;
-                if (t >= e && t < e + 4) {
-                    const int k = (int)(t - e);
-                    if (k == 0) d.x = rsub(d.x, inv_n);
-                    if (k == 1) d.y = rsub(d.y, inv_n);
-                    if (k == 2) d.z = rsub(d.z, inv_n);
-                    if (k == 3) d.w = rsub(d.w, inv_n);
-                }
-                reinterpret_cast<float4*>(dr)[idx] = d;
-            }
-        }
+        for (int i = 0; i < NV4; i++)
+            if (in(i))
+                *reinterpret_cast<float4*>(reinterpret_cast<char*>(dr + (long)i * NT * 4) + at) =
+                    make_float4(rmul(v[i].x, sc), rmul(v[i].y, sc), rmul(v[i].z, sc), rmul(v[i].w, sc));
+        // The target's element again, by the thread that has just written it.
+        if (tid == (int)(t / 4 % NT)) dr[t] = rsub(rmul(expf(rsub(lt, mx)), sc), inv_n);
         if (tid == 0) row_loss[r] = rsub(radd(logf(sum), mx), lt);
     } else {
-        for (long i = tid; i < vocab; i += kCeThreads) mx = fmaxf(mx, lr[i]);
-        mx = block_reduce(mx, true, sred);
+        for (long i = tid; i < vocab; i += NT) mx = fmaxf(mx, lr[i]);
+        mx = block_reduce<NT>(mx, true, sred);
         float sum = 0.0f;
-        for (long i = tid; i < vocab; i += kCeThreads) sum = radd(sum, expf(rsub(lr[i], mx)));
-        sum = block_reduce(sum, false, sred);
+        for (long i = tid; i < vocab; i += NT) sum = radd(sum, expf(rsub(lr[i], mx)));
+        sum = block_reduce<NT>(sum, false, sred);
         const float sc = rmul(rdiv(1.0f, sum), inv_n);
         // Every thread has read all of its elements before any is written,
         // and each element is read and written by the same thread, so dr
         // may alias lr.
-        for (long i = tid; i < vocab; i += kCeThreads) {
+        for (long i = tid; i < vocab; i += NT) {
             float d = rmul(expf(rsub(lr[i], mx)), sc);
             if (i == t) d = rsub(d, inv_n);
             dr[i] = d;
@@ -665,21 +663,28 @@ hipError_t launch_ce_rows(const float* logits, const int64_t* targets, float* dl
     if (nrows == 0 || vocab == 0) return hipSuccess;
     if (nrows > 0x7fffffffu) return hipErrorInvalidConfiguration;
     CeMisc* m = static_cast<CeMisc*>(misc);
-    const dim3 grid((unsigned)nrows), block(kCeThreads);
     const bool vec = vocab % 4 == 0 && aligned16(logits) && aligned16(dlogits);
-    const size_t v4 = (vocab / 4 + kCeThreads - 1) / kCeThreads;  // float4 per thread
-    if (vec && v4 <= 8)
-        hipLaunchKernelGGL(ce_rows_kernel<8>, grid, block, 0, st, logits, targets, dlogits, row_loss, (long)row0,
+    const size_t v4 = vocab / 4;
+    auto rows = [&](auto nv4, auto nt) {
+        hipLaunchKernelGGL((ce_rows_kernel<decltype(nv4)::value, decltype(nt)::value>), dim3((unsigned)nrows),
+                           dim3(decltype(nt)::value), 0, st, logits, targets, dlogits, row_loss, (long)row0,
                            (long)vocab, m);
-    else if (vec && v4 <= 16)
-        hipLaunchKernelGGL(ce_rows_kernel<16>, grid, block, 0, st, logits, targets, dlogits, row_loss, (long)row0,
-                           (long)vocab, m);
-    else if (vec && v4 <= 32)
-        hipLaunchKernelGGL(ce_rows_kernel<32>, grid, block, 0, st, logits, targets, dlogits, row_loss, (long)row0,
-                           (long)vocab, m);
+    };
+    using std::integral_constant;
+    using T512 = integral_constant<int, 512>;
+    using T1024 = integral_constant<int, 1024>;
+    // The fewest float4 a thread that hold the row: registers not used for it
+    // are waves in flight.
+    if (vec && v4 <= 8 * 512)
+        rows(integral_constant<int, 8>{}, T512{});
+    else if (vec && v4 <= 8 * 1024)
+        rows(integral_constant<int, 8>{}, T1024{});
+    else if (vec && v4 <= 12 * 1024)
+        rows(integral_constant<int, 12>{}, T1024{});
+    else if (vec && v4 <= 16 * 1024)
+        rows(integral_constant<int, 16>{}, T1024{});
     else
-        hipLaunchKernelGGL(ce_rows_kernel<0>, grid, block, 0, st, logits, targets, dlogits, row_loss, (long)row0,
-                           (long)vocab, m);
+        rows(integral_constant<int, 0>{}, T512{});
     return hipGetLastError();
 }
 
