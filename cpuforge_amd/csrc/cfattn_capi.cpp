@@ -541,6 +541,15 @@ static int cfattn_fused_bwd_locked(cfattn_ctx* c, cfattn_shape s, size_t batch, 
     int rc = CFATTN_OK;
     const size_t nq = batch * s.seq * s.n_heads * s.head_dim, nk = batch * s.seq * s.n_kv * s.head_dim;
     if (!d_o || !q || !k || !v || !dq_pre || !dk_pre || !dv) return fail(c, CFATTN_ERR_ARG, "null buffer");
+    // Without query heads nothing is added (an overwriting caller zeroes the
+    // gradients itself): the attention below launches nothing, so the
+    // scratch that the prologue backward reads would not be written.
+    if (s.n_heads == 0) {
+        if (!o || !lse) return fail(c, CFATTN_ERR_ARG, "null buffer");
+        if (pr->q_norm && (!q_pre || !k_pre || !q_rstd || !k_rstd || !dq_norm || !dk_norm))
+            return fail(c, CFATTN_ERR_ARG, "q/k norm backward needs q_pre, k_pre, rstd and gain-gradient buffers");
+        return CFATTN_OK;
+    }
     // The epilogue reads the cos/sin rows 16 bytes at a time: tables not
     // 16-byte aligned take the separate prologue backward instead.
     const bool tables16 = (reinterpret_cast<uintptr_t>(pr->cos) | reinterpret_cast<uintptr_t>(pr->sin)) % 16 == 0;

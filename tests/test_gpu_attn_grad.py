@@ -92,3 +92,40 @@ def test_no_rows_gives_zero_gain_gradients():
     rstd = torch.empty(0, device=DEV)
     out = D.fused_bwd(e(4), e(4), e(2), e(4), e(2), e(2), e(4), torch.empty(0, 4, 4, device=DEV), rstd, rstd, pr)
     assert bool((out[3] == 0).all()) and bool((out[4] == 0).all())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("dim", [6, 64, 128])
+@pytest.mark.parametrize("qk_norm", [True, False])
+def test_fused_bwd_without_query_heads_adds_nothing(dtype, dim, qk_norm):
+    """With n_heads = 0 the accumulating call leaves every gradient as it was
+    (and the overwriting one gives zeros), whatever an earlier call left in
+    the context's scratch."""
+    import ctypes
+
+    from cpuforge_amd import RopeCache, _lib
+    from cpuforge_amd import device as D
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    R = lambda *sh: torch.randn(*sh, generator=g, device=DEV)  # noqa: E731
+    seq, heads, kv = 40, 4, 2
+    q_pre, k_pre, v, d_o = R(1, seq, heads, dim), R(1, seq, kv, dim), R(1, seq, kv, dim).to(dt), R(1, seq, heads, dim)
+    gains = dict(q_norm=1 + 0.1 * R(dim), k_norm=1 + 0.1 * R(dim)) if qk_norm else {}
+    pr = D.DeviceRope(RopeCache(dim, seq, 1e4), DEV, **gains)
+    ctx = D.Context()
+    o, lse, q, k, q_rstd, k_rstd = D.fused_fwd(q_pre, k_pre, v, pr, ctx=ctx)
+    D.fused_bwd(d_o.to(dt), q_pre, k_pre, q, k, v, o, lse, q_rstd, k_rstd, pr, ctx=ctx)  # fills the scratch
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    for acc in (True, False):
+        grads = [R(q.numel()), R(k.numel()), R(k.numel())] + ([R(dim), R(dim)] if qk_norm else [None, None])
+        before = [None if t is None else t.clone() for t in grads]
+        fn = ctx._lib.cfattn_fused_bwd if acc else ctx._lib.cfattn_fused_bwd_grad
+        prc = pr.c()
+        shape = _lib.Shape(seq, 0, kv, dim)
+        _lib.check(fn(ctx.handle, shape, 1, D._code(q), ctypes.byref(prc), d_o.data_ptr(), q_pre.data_ptr(),
+                      k_pre.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
+                      ptr(q_rstd), ptr(k_rstd), *map(ptr, grads), D._stream()), ctx.handle)
+        torch.cuda.synchronize()
+        assert torch.equal(grads[0], before[0])  # no rows: not touched
+        for a, b in zip(grads[1:], before[1:]):
+            assert a is None or torch.equal(a, b if acc else torch.zeros_like(b))
