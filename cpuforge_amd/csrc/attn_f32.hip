@@ -103,12 +103,24 @@ __device__ __forceinline__ void f32_step_end(bool newer) {
     asm volatile("" ::: "memory");
 }
 
+// S of the f32 units (the forward's for short sequences, dQ, dK/dV) is summed
+// in two chains, one per half of each lane's head dims, added at the end: a
+// chain's roundings grow with its partial sum, two half as long round 0.7 times
+// as much.  The split forward's lse does not carry the rounding of the f32
+// scores that the backward forms again, which cancels in P = exp(S - lse) where
+// it does; with one chain the gradients were further off for that than with an
+// f32 forward (dv 3.79e-7 against 3.39e-7 at B2 S128 16/8 D128, 4.67 against
+// 4.45 at S700), with two they are nearer than with either (2.89, 3.80; dq, dk,
+// dv 0.84 to 0.97 of the f32 forward's with one chain from S20 to S3000).  Costs
+// 0.6% of the step at B8 S2048 9/3 D64 (1148 -> 1155 us).  dP in two chains as
+// well spills at head_dim 64 (1201 us); an f32 S in the forward, where the f32
+// MFMA leaves the VALU no time beside it, takes 1232.
+//
 // lse in the exponent's units, lse log2(e) = hi + lo: rounded to one float, a
-// row's P are all off by up to 2^-24 lse log2(e). With it, and lse rounded once
-// (lse_of), attention at S512 9/3 D64 is 4.3e-7 off where it was 4.6e-7. (The
-// forward's scores on split operands do not carry the rounding of the f32 products
-// that the backward forms again, which cancelled in P: see kX3MinSeq.) Costs
-// 2% of the step at B8 S2048 (1134 -> 1158 us). Infinite and NaN lse stay what they are.
+// row's P are all off by up to 2^-24 lse log2(e).  With it dv at S128 16/8 D128
+// is 2.89e-7 off, without 3.08; at S1500 9/3 D64 0.93 and 0.99 of the f32
+// forward's.  Costs 1.4% of the step at B8 S2048 (1138 -> 1155 us).  Infinite and
+// NaN lse stay what they are.
 struct LseLog2 {
     float hi, lo;
 };
@@ -235,20 +247,22 @@ __device__ __forceinline__ void fwd_f32_unit(const FwdParams& p, const F32Unit u
             // Each group's K row operands are read before the previous
             // group's MFMAs issue (pinned: the compiler otherwise reads them
             // after, and the products wait for the read).
-            f32x16 sc = zero16();
+            f32x16 sc = zero16(), s2 = zero16();
             float4 an = *reinterpret_cast<const float4*>(Ks + f32_at<DP>(l32, hh * HALF));
 #pragma unroll
             for (int c = 0; c < HALF / 4; c++) {
                 const float4 a = an;
                 if (c + 1 < HALF / 4) an = *reinterpret_cast<const float4*>(Ks + f32_at<DP>(l32, hh * HALF + 4 * c + 4));
                 __builtin_amdgcn_sched_barrier(0);
-                sc = mfma_f32(a.x, qf[4 * c], sc);
-                sc = mfma_f32(a.y, qf[4 * c + 1], sc);
-                sc = mfma_f32(a.z, qf[4 * c + 2], sc);
-                sc = mfma_f32(a.w, qf[4 * c + 3], sc);
+                f32x16& h = c < HALF / 8 ? sc : s2;
+                h = mfma_f32(a.x, qf[4 * c], h);
+                h = mfma_f32(a.y, qf[4 * c + 1], h);
+                h = mfma_f32(a.z, qf[4 * c + 2], h);
+                h = mfma_f32(a.w, qf[4 * c + 3], h);
                 __builtin_amdgcn_sched_barrier(0);
                 if (c == 0 && ahead) dma(kt + 2, Kn, Vn);
             }
+            sc += s2;
             float mx = -INFINITY;
             const bool masked = k0 + 31 > t_wave;
 #pragma unroll
@@ -323,17 +337,17 @@ __device__ __forceinline__ void fwd_f32_unit(const FwdParams& p, const F32Unit u
     if (hh == 0) p.lse[((long)b * p.nh + head) * p.seq + tq] = lse_of(m2, ltot);
 }
 
-// Shortest sequence on split operands. The rounding of the backward's f32 scores
-// cancels in P = exp(S - lse) where the forward's lse has the same scores in it, the
-// more the fewer keys a row has. Split against f32 forward: o 0.07 / 0.13, 0.10 /
-// 0.20, 0.11 / 0.23, 0.13 / 0.28 parts in 10^6 off at S 20, 100, 300, 1500; dq
-// 0.32 / 0.30, 0.36 / 0.35, 0.40 / 0.40, 0.52 / 0.51. Below it a call is a launch and
-// a few tiles, and neither is faster.
+// Shortest sequence on split operands.  Below it a call is a launch and a few
+// tiles, and neither unit is the faster (the layer's forward on the f32 unit and
+// on the split one: S20 9/3 D64 25 and 26 us, 8 x S100 30 and 31, 8 x S120 16/8
+// D128 34.9 and 34.7; 2 x S512 9/3 D64 34 and 32).
 constexpr int kX3MinSeq = 128;
 
 // One unit: on the bf16 matrix cores, or where a result is not finite with
 // f32 MFMAs (after the workgroup's vote every LDS read is done; the loads still
-// in flight are waited for, as fwd_f32_unit counts its own).
+// in flight are waited for, as fwd_f32_unit counts its own).  At head_dim 128
+// the persistent walk's invariants of both units do not fit the registers: 43
+// spill, stored before the walk and read back between units, none in a step.
 template <int DP>
 __device__ __forceinline__ void fwd_unit(const FwdParams& p, const F32Unit un, int rest, uint4* sm) {
     if (p.seq >= kX3MinSeq && fwd_x3_unit<DP>(p, un, rest, sm)) return;
@@ -425,21 +439,23 @@ __device__ __forceinline__ void dq_f32_unit(const BwdParams& p, const F32Unit un
         const bool ahead = kt + 2 < n_kt;
         const int k0 = kt * BN;
         if (wave_active && k0 <= wave_last) {
-            f32x16 sc = zero16(), dp = zero16();
+            f32x16 sc = zero16(), s2 = zero16(), dp = zero16();
 #pragma unroll
             for (int c = 0; c < HALF / 4; c++) {
                 const float4 a = *reinterpret_cast<const float4*>(Ks + f32_at<DP>(l32, hh * HALF + 4 * c));
                 const float4 v = *reinterpret_cast<const float4*>(Vs + f32_at<DP>(l32, hh * HALF + 4 * c));
-                sc = mfma_f32(a.x, qf[4 * c], sc);
+                f32x16& h = c < HALF / 8 ? sc : s2;
+                h = mfma_f32(a.x, qf[4 * c], h);
                 dp = mfma_f32(v.x, of[4 * c], dp);
-                sc = mfma_f32(a.y, qf[4 * c + 1], sc);
+                h = mfma_f32(a.y, qf[4 * c + 1], h);
                 dp = mfma_f32(v.y, of[4 * c + 1], dp);
-                sc = mfma_f32(a.z, qf[4 * c + 2], sc);
+                h = mfma_f32(a.z, qf[4 * c + 2], h);
                 dp = mfma_f32(v.z, of[4 * c + 2], dp);
-                sc = mfma_f32(a.w, qf[4 * c + 3], sc);
+                h = mfma_f32(a.w, qf[4 * c + 3], h);
                 dp = mfma_f32(v.w, of[4 * c + 3], dp);
                 if (c == 0 && ahead) dma(kt + 2, Kn, Vn);  // behind the first MFMAs, as the forward
             }
+            sc += s2;
             const bool masked = k0 + 31 > t_wave;
             float ds[16];
 #pragma unroll
@@ -744,7 +760,7 @@ __device__ __forceinline__ void dkdv_f32_unit(const BwdParams& p, const F32DkdvA
         if (wave_active && q0 + BM - 1 >= key0 && q0 < p.seq) {
             // S and dP: rows = queries q0 + [0, 32), columns = this wave's keys.
             // Q / dO row operands read a group ahead, as the forward's K rows.
-            f32x16 sc = zero16(), dp = zero16();
+            f32x16 sc = zero16(), s2 = zero16(), dp = zero16();
             float4 xn = *reinterpret_cast<const float4*>(Qs + f32_at<DP>(l32, hh * HALF));
             float4 yn = *reinterpret_cast<const float4*>(Os + f32_at<DP>(l32, hh * HALF));
 #pragma unroll
@@ -755,17 +771,19 @@ __device__ __forceinline__ void dkdv_f32_unit(const BwdParams& p, const F32DkdvA
                     yn = *reinterpret_cast<const float4*>(Os + f32_at<DP>(l32, hh * HALF + 4 * c + 4));
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                sc = mfma_f32(x.x, kf[4 * c], sc);
+                f32x16& hs = c < HALF / 8 ? sc : s2;
+                hs = mfma_f32(x.x, kf[4 * c], hs);
                 dp = mfma_f32(y.x, vf[4 * c], dp);
-                sc = mfma_f32(x.y, kf[4 * c + 1], sc);
+                hs = mfma_f32(x.y, kf[4 * c + 1], hs);
                 dp = mfma_f32(y.y, vf[4 * c + 1], dp);
-                sc = mfma_f32(x.z, kf[4 * c + 2], sc);
+                hs = mfma_f32(x.z, kf[4 * c + 2], hs);
                 dp = mfma_f32(y.z, vf[4 * c + 2], dp);
-                sc = mfma_f32(x.w, kf[4 * c + 3], sc);
+                hs = mfma_f32(x.w, kf[4 * c + 3], hs);
                 dp = mfma_f32(y.w, vf[4 * c + 3], dp);
                 __builtin_amdgcn_sched_barrier(0);
                 if (c == 0 && ahead) dma(s + 2, Qn, On, LDn);  // behind the first MFMAs, as the forward
             }
+            sc += s2;
             // Masked: the diagonal steps and the one past the sequence end
             // (P = 0 for keys after the query and for queries >= seq).
             const bool masked = q0 < key0 + 31 || q0 + BM > p.seq;
