@@ -32,8 +32,7 @@ namespace {
 struct Op3 {
     bf16x8 p[3];
 };
-__device__ __forceinline__ Op3 op3(const float* v) {
-    const Split8 s = split8(v);
+__device__ __forceinline__ Op3 op3(const Split8& s) {
     Op3 o;
 #pragma unroll
     for (int i = 0; i < 3; i++) o.p[i] = __builtin_bit_cast(bf16x8, s.p[i]);
@@ -69,7 +68,7 @@ struct RowsX3 {
     __device__ __forceinline__ void store(uint4* s, int tid) const {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const Split8 sp = split8(v[u]);
+            const Split8 sp = split8_scaled(v[u]);
             uint4* d = s + tid % OCT * PITCH + tid / OCT + STEP * u;
 #pragma unroll
             for (int i = 0; i < 3; i++) d[i * PLANE] = sp.p[i];
@@ -104,7 +103,7 @@ struct ColsX3 {
     __device__ __forceinline__ void store(uint4* s, int tid) const {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const Split8 sp = split8(v[u]);
+            const Split8 sp = split8_scaled(v[u]);
             uint4* d = s + (tid >> 6) * PITCH + (tid & 63) + 64 * u;
 #pragma unroll
             for (int i = 0; i < 3; i++) d[i * PLANE] = sp.p[i];
@@ -129,7 +128,7 @@ __device__ __forceinline__ void row_ops(const float* __restrict__ row, int hh, O
         const float4 a = *reinterpret_cast<const float4*>(row + 16 * c + 8 * hh);
         const float4 b = *reinterpret_cast<const float4*>(row + 16 * c + 8 * hh + 4);
         v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-        o[c] = op3(v);
+        o[c] = op3(split8_scaled(v));
     }
 }
 
@@ -161,6 +160,9 @@ template <int DP>
 __device__ __forceinline__ bool fwd_x3_unit(const FwdParams& p, const F32Unit un, int rest, uint4* sm) {
     constexpr int BN = 32, NDB = DP / 32, NC = DP / 16, STAGE = FwdX3<DP>::STAGE;
     constexpr float kLazy = 8.0f;
+    // K, Q and V are split scaled, P is not: a P below 2^-110 keeps an absolute
+    // error of 2^-134, beside a sum of 2^-8 and more.
+    const float sl2 = p.sl2 * (kSplitUnscale * kSplitUnscale);
     using Rows = RowsX3<DP>;
     using Cols = ColsX3<DP>;
 
@@ -230,7 +232,7 @@ __device__ __forceinline__ bool fwd_x3_unit(const FwdParams& p, const F32Unit un
                 if (masked && k0 + acc_row(r, hh) > tq) sc[r] = -INFINITY;
                 mx = fmaxf(mx, sc[r]);
             }
-            mx = max_halves(mx) * p.sl2;
+            mx = max_halves(mx) * sl2;
             const float mnew = mx > m2 + kLazy ? mx : m2;
             if (__any(mnew != m2)) {
                 const float alpha = __builtin_amdgcn_exp2f(m2 - mnew);
@@ -242,12 +244,12 @@ __device__ __forceinline__ bool fwd_x3_unit(const FwdParams& p, const F32Unit un
             float pr[16];
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], p.sl2, -m2));
+                pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], sl2, -m2));
                 lsum += pr[r];
             }
 #pragma unroll
             for (int s = 0; s < 2; s++) {
-                const Op3 pf = op3(pr + 8 * s);
+                const Op3 pf = op3(split8(pr + 8 * s));
 #pragma unroll
                 for (int db = 0; db < NDB; db++) mul3(Cols::read(Vs, s, db, l32, hh), pf, oacc[db], olow[db]);
             }
@@ -266,6 +268,7 @@ __device__ __forceinline__ bool fwd_x3_unit(const FwdParams& p, const F32Unit un
         for (int i = 0; i < NDB; i++) {
             oacc[i] += olow[i];
             odd |= any_odd(oacc[i]);
+            oacc[i] *= kSplitUnscale;
         }
     }
     if (__syncthreads_or(odd)) return false;

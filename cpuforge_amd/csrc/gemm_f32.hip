@@ -142,7 +142,7 @@ struct TileLoad {
         constexpr int P = kOct * PITCH;
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const Split8 sp = split8(v[u]);
+            const Split8 sp = split8_scaled(v[u]);
             uint4* d = s + oct(tid) * PITCH + row(tid, u);
             d[0] = sp.p[0];
             d[P] = sp.p[1];
@@ -314,6 +314,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
             acc[i][j] += low[i][j];
 #pragma unroll
             for (int r = 0; r < 16; r++) odd |= !(fabsf(acc[i][j][r]) < INFINITY);
+            acc[i][j] *= kSplitUnscale * kSplitUnscale;
         }
     const int mw = m0 + (wave >> 1) * (BM / WR) + 4 * hh, nw = n0 + br;
     if (__any(odd)) {

@@ -18,11 +18,15 @@
 // are kept in sums of their own (a0 b0 in one, the other five in the second), added
 // once at the end.
 //
-// What differs from f32 arithmetic: an infinite or NaN input, or one that
-// rounds to infinity in bf16 (within 2^-9 of the f32 maximum), gives a
-// non-finite sum also where f32 gives a finite or infinite one; callers
-// recompute such sums in f32.  Pieces below 2^-133, the smallest bf16
-// subnormal, round away: inputs below 2^-110 keep an absolute error of 2^-134.
+// The values are split times 2^16 (kSplitScale): bf16 has f32's exponents, so
+// the low pieces of a value below 2^-110 would lie below bf16's smallest
+// subnormal, 2^-133, and round away; scaled, all 24 bits of every normal f32 and
+// every subnormal are held.  The sums are scaled back at the end.
+//
+// What differs from f32 arithmetic: an infinite or NaN input, one of 2^111 and
+// above, and a sum whose scaled value overflows (2^96 and above with both
+// operands scaled) give a non-finite sum also where f32 gives a finite or
+// infinite one; callers recompute such sums in f32.
 #pragma once
 #include "cfattn_common.hpp"
 
@@ -43,6 +47,8 @@ __device__ __forceinline__ uint32_t cvt2_bf16(float a, float b) {
 }
 __device__ __forceinline__ float lo_f32(uint32_t u) { return __builtin_bit_cast(float, u << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
+
+constexpr float kSplitScale = 65536.0f, kSplitUnscale = 1.0f / 65536.0f;
 
 // The pieces of eight values, as three MFMA operands.
 struct Split8 {
@@ -67,6 +73,13 @@ __device__ __forceinline__ Split8 split8(const float* v) {
     split2(v[4], v[5], s.p[0].z, s.p[1].z, s.p[2].z);
     split2(v[6], v[7], s.p[0].w, s.p[1].w, s.p[2].w);
     return s;
+}
+__device__ __forceinline__ Split8 split8_scaled(const float* v) {
+#pragma clang fp contract(off)
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) w[i] = v[i] * kSplitScale;
+    return split8(w);
 }
 
 }  // namespace cfattn

@@ -72,6 +72,27 @@ def test_forward_of_infinite_and_huge_inputs_is_f32s(d):
     assert torch.allclose(o[0, :, 0], base[0, :, 0], rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("exp", [-114, -124, -140])
+def test_forward_of_the_smallest_values(d, exp):
+    """Inputs down to f32's subnormals keep all their bits: v as o's scale, and
+    k beside a q that makes the scores ordinary numbers."""
+    from cpuforge_amd import device as D
+    g = torch.Generator(device=DEV).manual_seed(d - exp)
+    q, k, v = (torch.randn(1, 200, h, d, generator=g, device=DEV) for h in (4, 2, 2))
+    w = v * 2.0 ** exp
+    o, _ = D.fwd(q, k, w)
+    want, _ = reference(q, k, w)
+    # Results below f32's smallest normal are rounded to its subnormals, 2^-149 apart.
+    assert float((o.double() - want).norm()) <= 5e-7 * float(want.norm()) + 2.0 ** -149 * want.numel() ** 0.5
+    kk, qq = k * 2.0 ** max(exp, -124), q * 2.0 ** min(-exp, 124)
+    o, lse = D.fwd(qq, kk, v)
+    want, wlse = reference(qq, kk, v)
+    assert bool(torch.isfinite(o).all())
+    assert float((o.double() - want).norm()) <= 5e-7 * float(want.norm())
+    assert float((lse.double() - wlse).abs().max()) <= 4e-6
+
+
 # Relative 2-norm errors (dq, dk, dv) of unit-variance inputs where the forward
 # and the backward form the same f32 scores in one chain of sums.
 @pytest.mark.parametrize("shape,limits", [((2, 128, 16, 8, 128), (4.42e-7, 4.43e-7, 3.39e-7)),

@@ -69,6 +69,22 @@ def test_gemm_small_and_large_magnitudes(kind):
 
 
 @pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("exp", [-112, -118, -124, -130, -140])
+def test_gemm_of_the_smallest_values(kind, exp):
+    """Inputs down to f32's subnormals keep all their bits (their low pieces
+    would lie below bf16's smallest subnormal): against large ones on the other
+    side, the products are ordinary numbers."""
+    g = torch.Generator(device=DEV).manual_seed(-exp)
+    a = torch.randn(70, 96, generator=g, device=DEV) * 2.0 ** exp
+    b = torch.randn(96, 66, generator=g, device=DEV) * 2.0 ** 90
+    assert bool((a[:, :8] != 0).any())
+    for x, y in ((a, b), (b.t().contiguous(), a.t().contiguous())):
+        c = product(kind, x, y, torch.empty(x.shape[0], y.shape[1], device=DEV), False)
+        bound = 2.0 ** -24 * 104 * (x.abs().double() @ y.abs().double())
+        assert bool(((c.double() - x.double() @ y.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
 def test_gemm_infinities_and_nan_are_f32s(kind):
     """What f32 arithmetic gives where an input is infinite or NaN: the same
     infinities and NaN, the other outputs untouched by them."""
