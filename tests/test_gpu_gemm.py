@@ -99,3 +99,23 @@ def test_gemm_infinities_and_nan_are_f32s(kind):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     assert np.array_equal(got[ok], want[ok])
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,k,n", [(70, 37, 66), (65, 4099, 63), (300, 1333, 501), (2048, 1000, 2050), (4096, 96, 2050)])
+def test_gemm_recomputed_tiles(kind, m, k, n):
+    """Every tile and split form with NaN, infinite and huge values in some
+    places: what f32 arithmetic gives there, and its accuracy everywhere else."""
+    g = torch.Generator(device=DEV).manual_seed(m + k + n)
+    a = torch.randn(m, k, generator=g, device=DEV)
+    b = torch.randn(k, n, generator=g, device=DEV)
+    a[m - 1, k // 2], a[m // 2, k - 1], a[3, 0], b[k - 1, n - 1] = float("nan"), float("inf"), 2.0 ** 120, -float("inf")
+    want = a.double() @ b.double()
+    c = product(kind, a, b, torch.empty(m, n, device=DEV), False)
+    assert torch.equal(c.isnan(), want.isnan())
+    assert torch.equal(c == float("inf"), want == float("inf"))
+    assert torch.equal(c == -float("inf"), want == -float("inf"))
+    ok = want.isfinite()
+    fin = lambda x: torch.where(x.isfinite(), x, 0.0).abs().double()  # noqa: E731
+    bound = 2.0 ** -24 * (k + 8) * (fin(a) @ fin(b)) + 2.0 ** -22 * want.abs()
+    assert bool(((c.double() - want).abs() <= bound)[ok].all())
