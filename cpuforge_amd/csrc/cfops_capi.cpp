@@ -5,8 +5,10 @@
 // layer_ops.hip.  There is no CPU compute path.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstddef>
+#include <cstdint>
 #include <cstring>
 
 #include "cfattn_ctx.hpp"
@@ -57,6 +59,32 @@ int gemm(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, si
     g.pr[0].nseg = 1, g.pr[0].c = out, g.pr[0].n = (int)n;
     g.pr[0].seg[0] = {a, b, (long)(kind == CFOPS_TN ? m : k), (long)(kind == CFOPS_NT ? k : n), (int)k};
     return launch_gemm(c, g, st);
+}
+
+// Whether a buffer that one tensor's update writes shares memory with any of
+// another's (a parameter under two names, or beside a view of itself).
+bool adamw_overlaps(const cfattn::AdamwArgs& a) {
+    struct Range {
+        uintptr_t lo, hi;
+        bool written;
+    } r[4 * cfattn::kAdamwBatch];
+    int n = 0;
+    for (int i = 0; i < a.count; i++) {
+        const cfattn::AdamwTensor& t = a.t[i];
+        const float* const ptr[4] = {t.p, t.m, t.v, t.g};
+        for (int j = 0; j < 4; j++) {
+            const uintptr_t lo = reinterpret_cast<uintptr_t>(ptr[j]);
+            r[n++] = {lo, lo + (size_t)t.n * sizeof(float), j < 3};
+        }
+    }
+    std::sort(r, r + n, [](const Range& x, const Range& y) { return x.lo < y.lo; });
+    uintptr_t end = 0, end_written = 0;
+    for (int i = 0; i < n; i++) {
+        if (r[i].lo < (r[i].written ? end : end_written)) return true;
+        end = std::max(end, r[i].hi);
+        if (r[i].written) end_written = std::max(end_written, r[i].hi);
+    }
+    return false;
 }
 
 int check_linears(cfattn_ctx* c, size_t t, size_t in, const cfops_linear* lin, size_t n) {
@@ -418,7 +446,14 @@ int cfops_adamw_update_multi(cfattn_ctx* c, size_t count, float* const* p, const
     for (size_t i = 0; i < count; i++) {
         if (n[i]) a.t[a.count++] = {p[i], g[i], m[i], v[i], (long)n[i], weight_decay[i], 0, 0};
         if (a.count == cfattn::kAdamwBatch || (i + 1 == count && a.count)) {
-            CF_HIP(c, cfattn::launch_adamw(a, to_stream(stream)), "adamw launch");
+            // Tensors of one launch are updated side by side.
+            const int step = adamw_overlaps(a) ? 1 : a.count;
+            for (int k = 0; k < a.count; k += step) {
+                cfattn::AdamwArgs b = a;
+                std::copy(a.t + k, a.t + k + step, b.t);
+                b.count = step;
+                CF_HIP(c, cfattn::launch_adamw(b, to_stream(stream)), "adamw launch");
+            }
             a.count = 0;
         }
     }

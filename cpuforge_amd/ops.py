@@ -260,10 +260,13 @@ def adamw_update(p, g, m, v, t, lr, beta1, beta2, eps, weight_decay, ctx: Contex
 
 
 def adamw_update_multi(ps, gs, ms, vs, t, lr, beta1, beta2, eps, weight_decays, ctx: Context | None = None):
-    """adamw_update of many tensors (no two overlapping), each with its own
-    weight decay, in few launches."""
+    """adamw_update of many tensors, each with its own weight decay, in few
+    launches (tensors that share memory are updated in order)."""
     ctx = ctx or default_context()
     k = len(ps)
+    for name, xs in (("g", gs), ("m", ms), ("v", vs), ("weight_decays", weight_decays)):
+        if len(xs) != k:
+            raise _lib.ShapeError(_lib.ERR_SHAPE, f"assertion `left == right` failed: {len(xs)} {name} for {k} tensors")
     sizes = [x.numel() for x in ps]
     arrs = []
     for name, ts in (("p", ps), ("g", gs), ("m", ms), ("v", vs)):

@@ -47,9 +47,4 @@ class AdamW:
             ms.append(s[0])
             vs.append(s[1])
             decays.append(0.0 if "norm" in name else self.weight_decay)
-        hyper = (self.step, lr, self.beta1, self.beta2, self.eps)
-        if len({p.data_ptr() for p in ps}) == len(ps):
-            P.adamw_update_multi(ps, gs, ms, vs, *hyper, decays)
-        else:  # a tensor under two names is updated once for each, in turn
-            for p, g, m, v, d in zip(ps, gs, ms, vs, decays):
-                P.adamw_update(p, g, m, v, *hyper, d)
+        P.adamw_update_multi(ps, gs, ms, vs, self.step, lr, self.beta1, self.beta2, self.eps, decays)

@@ -157,7 +157,8 @@ int cfops_adamw_update(cfattn_ctx* ctx, float* p, const float* g, float* m, floa
 
 /* AdamW::step's loop over the parameters (optim.rs:48-61) in few launches:
  * adamw_update of `count` tensors, tensor i of n[i] values with its own weight
- * decay.  No two may overlap in memory. */
+ * decay.  Where tensors share memory the result is that of updating one after
+ * the other. */
 int cfops_adamw_update_multi(cfattn_ctx* ctx, size_t count, float* const* p, const float* const* g, float* const* m,
                              float* const* v, const size_t* n, const float* weight_decay, uint64_t t, float lr,
                              float beta1, float beta2, float eps, void* stream);

@@ -57,3 +57,49 @@ def test_a_tensor_under_two_names_is_updated_twice():
         P.adamw_update(q, p.grad, z, torch.zeros(100, device=DEV), 1, 1e-2, 0.9, 0.999, 1e-8, 0.0)
     AdamW(0.9, 0.999, 1e-8, 0.0).update(Model([("a", p), ("b", p)]), 1e-2)
     assert torch.equal(p.detach(), q)
+
+
+@pytest.mark.parametrize("case", ["view", "inner view", "name", "moments"])
+def test_tensors_that_share_memory_are_updated_in_order(case):
+    """A parameter beside a view into it, two parameters under one name (and
+    so with one state), moments that overlap: as updated one after the other."""
+    from cpuforge_amd import ops as P
+    from cpuforge_amd.optim import AdamW
+
+    def build():
+        g = torch.Generator(device=DEV).manual_seed(5)
+        R = lambda n: torch.randn(n, generator=g, device=DEV)  # noqa: E731
+        base, n = R(100000), 60000
+        cut = {"view": (0, 40000), "inner view": (8, 1000)}.get(case)
+        named = [("a", base), ("b", base[cut[0]:cut[1]])] if cut else [("a", base[:n]), ("b", R(n))]
+        if case == "name":
+            named = [("a", named[0][1]), ("a", named[1][1])]
+        named = [("first", R(777))] + named + [("last", R(4097))]
+        grads = [R(p.numel()) for _, p in named]
+        ms = [R(p.numel()) for _, p in named]
+        vs = [R(p.numel()).square() for _, p in named]
+        if case == "name":
+            ms[2], vs[2] = ms[1], vs[1]
+        if case == "moments":
+            flat = R(2 * n).square()
+            ms[1], vs[2] = flat[:n], flat[4096:4096 + n]
+        return named, grads, ms, vs
+
+    named, grads, ms, vs = build()
+    for (_, p), g, m, v in zip(named, grads, ms, vs):
+        P.adamw_update(p, g, m, v, 3, 1e-2, 0.9, 0.95, 1e-8, 0.1)
+    got, grads2, ms2, vs2 = build()
+    opt = AdamW(0.9, 0.95, 1e-8, 0.1)
+    opt.step = 2
+    for i, (name, p) in enumerate(got):
+        p = p.detach().requires_grad_()
+        p.grad = grads2[i]
+        got[i] = (name, p)
+        opt.state[name] = (ms2[i], vs2[i])
+
+    class M:
+        def named_params(self):
+            return iter(got)
+    opt.update(M(), 1e-2)
+    for (_, p), (_, q), m, m2, v, v2 in zip(named, got, ms, ms2, vs, vs2):
+        assert torch.equal(p, q.detach()) and torch.equal(m, m2) and torch.equal(v, v2)
