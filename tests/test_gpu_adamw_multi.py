@@ -82,7 +82,7 @@ def test_tensors_that_share_memory_are_updated_in_order(case):
             ms[2], vs[2] = ms[1], vs[1]
         if case == "moments":
             flat = R(2 * n).square()
-            ms[1], vs[2] = flat[:n], flat[4096:4096 + n]
+            vs[1], vs[2] = flat[:n], flat[4096:4096 + n]
         return named, grads, ms, vs
 
     named, grads, ms, vs = build()
