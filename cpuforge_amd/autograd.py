@@ -1,9 +1,9 @@
 """torch autograd functions over the layer ops of include/cfops.h, so a host
 model can run cpuforge's Layer and LM head on the GPU with every hot op in
 libcfattn.so.  Each backward keeps the reference's gradient contract (the
-`Linear::backward` / `rmsnorm_backward` / `silu_mul_backward` formulas,
-accumulating into fresh zero buffers); frozen tensors (requires_grad False)
-get no gradient work, as an empty LinGrad vector does in the reference
+`Linear::backward` / `rmsnorm_backward` / `silu_mul_backward` formulas), into
+new buffers that the ops overwrite; frozen tensors (requires_grad False) get no
+gradient work, as an empty LinGrad vector does in the reference
 (crates/model/src/linear.rs:22-27)."""
 from __future__ import annotations
 
@@ -16,20 +16,9 @@ def _flat(x: torch.Tensor, cols: int) -> torch.Tensor:
     return x.contiguous().view(-1, cols)
 
 
-def _zeros(*likes):
-    """Zero-filled buffers shaped like `likes` (None entries stay None), cut
-    from one allocation so they cost one fill launch."""
-    sizes = [t.numel() if t is not None else 0 for t in likes]
-    flat = torch.zeros(sum(sizes), device=next(t for t in likes if t is not None).device, dtype=torch.float32)
-    out, off = [], 0
-    for t, n in zip(likes, sizes):
-        out.append(None if t is None else flat[off:off + n].view(t.shape))
-        off += n
-    return out
-
-
 def _empty(*likes):
-    """_zeros without the fill, for buffers an op overwrites."""
+    """Buffers shaped like `likes` (None entries stay None) for an op to
+    overwrite, cut from one allocation."""
     sizes = [t.numel() if t is not None else 0 for t in likes]
     flat = torch.empty(sum(sizes), device=next(t for t in likes if t is not None).device, dtype=torch.float32)
     return [None if t is None else v.view(t.shape) for t, v in zip(likes, flat.split(sizes))]
@@ -77,55 +66,71 @@ class SiluMulFn(torch.autograd.Function):
         return dg, du
 
 
-class LinearsFn(torch.autograd.Function):
-    """y = x W^T (+ scale (x A^T) B^T) (crates/model/src/linear.rs:56-91) of one
-    linear or of several of one input (the q/k/v projections of a layer, or its
-    gate and up projections), whose dx is one sum, as the reference's
-    Layer::backward forms dn2 (crates/model/src/layer.rs:170-171) and dn1
-    (layer.rs:208-211).  `flat` holds (w, a, b) per linear."""
+def _linears_forward(ctx, x, scales, flat):
+    inn = flat[0].shape[1]
+    x2 = _flat(x, inn)
+    t = x2.shape[0]
+    lins, ys, xss = [], [], []
+    for i, scale in enumerate(scales):
+        w, a, b = flat[3 * i:3 * i + 3]
+        y = torch.empty(t, w.shape[0], device=x.device, dtype=torch.float32)
+        xs = torch.empty(t, a.shape[0], device=x.device, dtype=torch.float32) if a is not None else None
+        lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, y=y, xs=xs))
+        ys.append(y.view(*x.shape[:-1], w.shape[0]))
+        xss.append(xs)
+    P.linears_forward(x2, t, inn, lins)
+    ctx.save_for_backward(x2, *flat, *xss)
+    ctx.scales = scales
+    ctx.shape = x.shape
+    return ys
+
+
+def _linears_backward(ctx, need, dys):
+    """The gradients of x and of every (w, a, b) that `need` asks for."""
+    saved = ctx.saved_tensors
+    n = len(ctx.scales)
+    x2, flat, xss = saved[0], saved[1:1 + 3 * n], saved[1 + 3 * n:]
+    t, inn = x2.shape
+    if not any(need):
+        return (None,) * (1 + 3 * n)
+    dx, *grads = _empty(*[x if f else None for x, f in zip((x2, *flat), need)])
+    lins = []
+    for i, scale in enumerate(ctx.scales):
+        w, a, b = flat[3 * i:3 * i + 3]
+        gw, ga, gb = grads[3 * i:3 * i + 3]
+        lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, xs=xss[i], dy=_flat(dys[i], w.shape[0]), gw=gw, ga=ga,
+                         gb=gb))
+    P.linears_backward(x2, t, inn, dx, lins, acc=False)
+    return (None if dx is None else dx.view(ctx.shape), *grads)
+
+
+class LinearFn(torch.autograd.Function):
+    """y = x W^T (+ scale (x A^T) B^T) (crates/model/src/linear.rs:56-91)."""
+
+    @staticmethod
+    def forward(ctx, x, w, a, b, scale: float):
+        return _linears_forward(ctx, x, (scale,), (w, a, b))[0]
+
+    @staticmethod
+    def backward(ctx, dy):
+        return (*_linears_backward(ctx, ctx.needs_input_grad[:4], (dy,)), None)
+
+
+class SharedInputLinearsFn(torch.autograd.Function):
+    """Several linears of one input (the q/k/v projections of a layer, or its
+    gate and up projections): each forward as LinearFn, and one dx, as the
+    reference's Layer::backward forms dn2 (crates/model/src/layer.rs:170-171)
+    and dn1 (layer.rs:208-211).  `flat` holds (w, a, b) per linear."""
 
     @staticmethod
     def forward(ctx, x, scales, *flat):
-        inn = flat[0].shape[1]
-        x2 = _flat(x, inn)
-        t = x2.shape[0]
-        lins, ys, xss = [], [], []
-        for i, scale in enumerate(scales):
-            w, a, b = flat[3 * i:3 * i + 3]
-            y = torch.empty(t, w.shape[0], device=x.device, dtype=torch.float32)
-            xs = torch.empty(t, a.shape[0], device=x.device, dtype=torch.float32) if a is not None else None
-            lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, y=y, xs=xs))
-            ys.append(y.view(*x.shape[:-1], w.shape[0]))
-            xss.append(xs)
-        P.linears_forward(x2, t, inn, lins)
-        ctx.save_for_backward(x2, *flat, *xss)
-        ctx.scales = scales
-        ctx.shape = x.shape
-        return tuple(ys)
+        return tuple(_linears_forward(ctx, x, scales, flat))
 
     @staticmethod
     def backward(ctx, *dys):
-        saved = ctx.saved_tensors
-        n = len(ctx.scales)
-        x2, flat, xss = saved[0], saved[1:1 + 3 * n], saved[1 + 3 * n:]
-        t, inn = x2.shape
-        need = [ctx.needs_input_grad[0]] + list(ctx.needs_input_grad[2:])
-        if not any(need):
-            return (None,) * (2 + 3 * n)
-        # Everything is overwritten, except where an output was not used: its
-        # linear's gradients stay zero.
-        likes = [x if f else None for x, f in zip((x2, *flat), need)]
-        dx, *grads = _zeros(*likes) if any(dy is None for dy in dys) else _empty(*likes)
-        lins = []
-        for i, scale in enumerate(ctx.scales):
-            w, a, b = flat[3 * i:3 * i + 3]
-            if dys[i] is None:
-                continue
-            gw, ga, gb = grads[3 * i:3 * i + 3]
-            lins.append(dict(w=w, lora_a=a, lora_b=b, scale=scale, xs=xss[i], dy=_flat(dys[i], w.shape[0]), gw=gw,
-                             ga=ga, gb=gb))
-        P.linears_backward(x2, t, inn, dx, lins, acc=False)
-        return (None if dx is None else dx.view(ctx.shape), None, *grads)
+        need = (ctx.needs_input_grad[0], *ctx.needs_input_grad[2:])
+        dx, *grads = _linears_backward(ctx, need, dys)
+        return (dx, None, *grads)
 
 
 class LMHeadCEFn(torch.autograd.Function):
@@ -187,14 +192,14 @@ def silu_mul(g, u):
 
 
 def linear(x, w, a=None, b=None, scale=1.0):
-    return LinearsFn.apply(x, (float(scale),), w, a, b)[0]
+    return LinearFn.apply(x, w, a, b, scale)
 
 
 def shared_input_linears(x, specs):
     """[(w, a, b, scale), ...] -> the linears' outputs for input x, with one
     dx in the backward."""
     flat = [t for w, a, b, _ in specs for t in (w, a, b)]
-    return LinearsFn.apply(x, tuple(float(s) for *_, s in specs), *flat)
+    return SharedInputLinearsFn.apply(x, tuple(float(s) for *_, s in specs), *flat)
 
 
 def lm_head_ce(hn, head, targets):

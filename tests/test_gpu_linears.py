@@ -104,3 +104,19 @@ def test_linears_autograd_unused_output_and_frozen_input():
     z = A.linear(x.detach(), w, a, b, 2.0)
     ga2, = torch.autograd.grad(z.sum(), [a])
     assert torch.allclose(ga2, ga, rtol=1e-5, atol=1e-4)
+
+
+def test_linear_functions_by_name():
+    """autograd.LinearFn and SharedInputLinearsFn are what linear() and
+    shared_input_linears() apply."""
+    from cpuforge_amd import autograd as A
+    g = torch.Generator(device=DEV).manual_seed(4)
+    R = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    x, w, a, b = (t.requires_grad_() for t in (R(2, 9, 40), R(50, 40), R(8, 40), R(50, 8)))
+    dy = R(2, 9, 50)
+    outs = [A.linear(x, w, a, b, 2.0), A.LinearFn.apply(x, w, a, b, 2.0),
+            A.SharedInputLinearsFn.apply(x, (2.0,), w, a, b)[0]]
+    grads = [torch.autograd.grad(y, (x, w, a, b), dy) for y in outs]
+    for y, got in zip(outs[1:], grads[1:]):
+        assert torch.equal(y, outs[0]) and all(torch.equal(p, q) for p, q in zip(got, grads[0]))
+    assert A.LinearFn.apply(x, w, None, None, 1.0).shape == (2, 9, 50)
