@@ -410,6 +410,7 @@ int cfops_linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, f
             CF_TRY(zero_grad(c, l.ga, l.rank * in, to_stream(stream)));
             CF_TRY(zero_grad(c, l.gb, l.out * l.rank, to_stream(stream)));
         }
+    if (n == 0 && !acc) return zero_grad(c, dx, t * in, to_stream(stream));
     if (t == 0 || n == 0) return CFATTN_OK;
     if (!x || !lin) return fail(c, CFATTN_ERR_ARG, "null buffer");
     for (size_t i = 0; i < n; i++) {

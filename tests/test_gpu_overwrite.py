@@ -67,3 +67,6 @@ def test_gradients_of_no_rows_are_zero():
     leaves = [t.requires_grad_() for t in (w, a, b)]
     grads = torch.autograd.grad(A.linear(x, w, a, b, 2.0).sum(), leaves)
     assert all(bool((g == 0).all()) for g in grads)
+    dx = nan(5, 24)
+    P.linears_backward(torch.randn(5, 24, device=DEV), 5, 24, dx, [], acc=False)  # of no linears
+    assert bool((dx == 0).all())
