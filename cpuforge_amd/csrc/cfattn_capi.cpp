@@ -291,6 +291,7 @@ int cfattn_destroy(cfattn_ctx* c) {
         if (c->fwd_settles) (void)hipFree(c->fwd_settles);
         for (int i = 0; i < cfattn_ctx::NSLOT; i++)
             if (c->buf[i]) (void)hipFree(c->buf[i]);
+        for (void* p : c->retired) (void)hipFree(p);
     }
     delete c;
     return CFATTN_OK;
@@ -514,6 +515,7 @@ int cfattn_prologue_bwd(cfattn_ctx* c, cfattn_shape s, size_t batch, const cfatt
     if (!c) return CFATTN_ERR_ARG;
     std::lock_guard<std::mutex> lk(c->mu);
     c->err.clear();
+    note_capture(c, pick_stream(c, stream));
     return cfattn_prologue_bwd_locked(c, s, batch, pr, dq, dk, q_pre, k_pre, q_rstd, k_rstd, dq_pre, dk_pre, dq_norm, dk_norm, stream);
 }
 
@@ -709,9 +711,7 @@ int cfattn_set_ds_limit(cfattn_ctx* c, size_t bytes) {
     for (int sl : {(int)cfattn_ctx::DS, (int)cfattn_ctx::FWD_SPLIT}) {
         if (c->buf[sl] && c->cap[sl] > bytes) {
             DeviceGuard dg(c->device);
-            (void)hipFree(c->buf[sl]);
-            c->buf[sl] = nullptr;
-            c->cap[sl] = 0;
+            CF_TRY(release_slot(c, sl));
         }
     }
     return CFATTN_OK;

@@ -5,11 +5,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -117,6 +119,11 @@ struct cfattn_ctx {
     };
     void* buf[NSLOT] = {};
     size_t cap[NSLOT] = {};
+    // Set by the first call that is recorded into a HIP graph: the graph's
+    // replays use the buffers of that time, so from then on an outgrown or
+    // released one is kept in `retired` until cfattn_destroy.
+    bool captured = false;
+    std::vector<void*> retired;
     EventTimer* timer = nullptr;  // non-null while profiling is on
     unsigned prof_mask = ~0u;     // kernels profiling brackets (cfattn_profile_select)
     size_t ds_limit = (size_t)8 << 30;  // stored-dS scratch limit (cfattn_set_ds_limit)
@@ -204,25 +211,61 @@ struct DeviceGuard {
     }
 };
 
+// Whether `st` is being captured into a HIP graph, which the context then
+// remembers.  Called by every entry point that takes a stream and scratch.
+inline bool note_capture(cfattn_ctx* c, hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (status == hipStreamCaptureStatusNone) return false;
+    return c->captured = true;
+}
+
+// Gives a slot's buffer back, or retires it (cfattn_ctx::captured).
+inline int release_slot(cfattn_ctx* c, int s) {
+    if (c->captured) {
+        try {
+            c->retired.push_back(c->buf[s]);
+        } catch (const std::bad_alloc&) {
+            return fail(c, CFATTN_ERR_NOMEM, "out of host memory");
+        }
+    } else {
+        (void)hipFree(c->buf[s]);
+    }
+    c->buf[s] = nullptr;
+    c->cap[s] = 0;
+    return CFATTN_OK;
+}
+
 // Grow-only device buffer of a pool slot.
 inline void* slot(cfattn_ctx* c, int s, size_t bytes, int* rc) {
     if (bytes == 0) bytes = 256;
     if (c->cap[s] >= bytes) return c->buf[s];
-    if (c->buf[s]) {
-        (void)hipFree(c->buf[s]);
-        c->buf[s] = nullptr;
-        c->cap[s] = 0;
+    const size_t old = c->cap[s];
+    if (c->buf[s] && (*rc = release_slot(c, s)) != CFATTN_OK) return nullptr;
+    // Where outgrown buffers are kept, a slot grows by half of its size at
+    // least, so that all it has retired are less than twice what it holds
+    // (the slots under cfattn_set_ds_limit only up to that limit).
+    size_t sizes[2] = {bytes, bytes};
+    if (c->captured) {
+        const bool limited = s == cfattn_ctx::DS || s == cfattn_ctx::FWD_SPLIT;
+        sizes[0] = std::max(bytes, limited ? std::min(old + old / 2, c->ds_limit) : old + old / 2);
     }
-    size_t want = (bytes + 4095) & ~(size_t)4095;
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) {
-        *rc = fail(c, CFATTN_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", want, hipGetErrorString(e));
-        return nullptr;
+    hipError_t e = hipSuccess;
+    for (size_t want : sizes) {
+        want = (want + 4095) & ~(size_t)4095;
+        void* p = nullptr;
+        e = hipMalloc(&p, want);
+        if (e == hipSuccess) {
+            c->buf[s] = p;
+            c->cap[s] = want;
+            return p;
+        }
     }
-    c->buf[s] = p;
-    c->cap[s] = want;
-    return p;
+    *rc = fail(c, CFATTN_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+    return nullptr;
 }
 
 // Host-slice staging (host_stage.cpp): copies through two pinned chunks on
@@ -236,7 +279,7 @@ int stage_download(cfattn_ctx* c, void* host, const void* dev, size_t bytes);
 struct DeviceCallMark {
     cfattn_ctx* c;
     hipStream_t st;
-    DeviceCallMark(cfattn_ctx* c_, hipStream_t st_) : c(c_), st(st_) {}
+    DeviceCallMark(cfattn_ctx* c_, hipStream_t st_) : c(c_), st(st_) { note_capture(c, st); }
     ~DeviceCallMark() {
         if (c->dev_done && hipEventRecord(c->dev_done, st) == hipSuccess) c->dev_pending = true;
     }

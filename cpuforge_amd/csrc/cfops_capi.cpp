@@ -190,12 +190,13 @@ int ce_result(cfattn_ctx* c, const void* misc, const int64_t* targets, size_t vo
     return CFATTN_OK;
 }
 
-#define CF_LOCK(c)                                                                        \
+#define CF_LOCK(c, stream)                                                                  \
     if (!(c)) return CFATTN_ERR_ARG;                                                      \
     std::lock_guard<std::mutex> lk((c)->mu);                                              \
     (c)->err.clear();                                                                     \
     DeviceGuard dev_guard_((c)->device);                                                  \
-    if (!dev_guard_.ok) return fail((c), CFATTN_ERR_HIP, "hipSetDevice(%d) failed", (c)->device);
+    if (!dev_guard_.ok) return fail((c), CFATTN_ERR_HIP, "hipSetDevice(%d) failed", (c)->device); \
+    note_capture((c), to_stream(stream))
 
 }  // namespace
 
@@ -203,14 +204,14 @@ extern "C" {
 
 int cfops_matmul(cfattn_ctx* c, int kind, const float* a, const float* b, float* out, size_t m, size_t k, size_t n,
                  int acc, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if ((m && n && !out) || (m && n && k && (!a || !b))) return fail(c, CFATTN_ERR_ARG, "null buffer");
     return gemm(c, kind, a, b, out, m, k, n, acc != 0, to_stream(stream));
 }
 
 int cfops_rmsnorm_forward(cfattn_ctx* c, const float* x, const float* w, float* y, float* rstd, size_t rows,
                           size_t dim, float eps, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (rows == 0 || dim == 0) return CFATTN_OK;
     if (!x || !w || !y || !rstd) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (!fits_int(dim)) return fail(c, CFATTN_ERR_UNSUPPORTED, "dim=%zu above 2^31", dim);
@@ -225,7 +226,7 @@ int cfops_rmsnorm_backward(cfattn_ctx* c, const float* dy, const float* x, const
 
 int cfops_rmsnorm_grad(cfattn_ctx* c, const float* dy, const float* x, const float* w, const float* rstd, float* dx,
                        float* dw, size_t rows, size_t dim, int acc, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (rows == 0 && !acc) return zero_grad(c, dw, dim, to_stream(stream));
     if (rows == 0 || dim == 0) return CFATTN_OK;
     if (!dy || !x || !w || !rstd || !dx) return fail(c, CFATTN_ERR_ARG, "null buffer");
@@ -243,7 +244,7 @@ int cfops_rmsnorm_grad(cfattn_ctx* c, const float* dy, const float* x, const flo
 }
 
 int cfops_silu_mul_forward(cfattn_ctx* c, const float* g, const float* u, float* h, size_t n, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (n == 0) return CFATTN_OK;
     if (!g || !u || !h) return fail(c, CFATTN_ERR_ARG, "null buffer");
     CF_HIP(c, cfattn::launch_silu_mul_fwd(g, u, h, n, to_stream(stream)), "silu_mul forward launch");
@@ -257,7 +258,7 @@ int cfops_silu_mul_backward(cfattn_ctx* c, const float* dh, const float* g, cons
 
 int cfops_silu_mul_grad(cfattn_ctx* c, const float* dh, const float* g, const float* u, float* dg, float* du, size_t n,
                         int acc, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (n == 0) return CFATTN_OK;
     if (!dh || !g || !u || !dg || !du) return fail(c, CFATTN_ERR_ARG, "null buffer");
     CF_HIP(c, cfattn::launch_silu_mul_bwd(dh, g, u, dg, du, n, acc != 0, to_stream(stream)), "silu_mul backward launch");
@@ -266,7 +267,7 @@ int cfops_silu_mul_grad(cfattn_ctx* c, const float* dh, const float* g, const fl
 
 int cfops_cross_entropy_fwd_bwd(cfattn_ctx* c, const float* logits, const int64_t* targets, float* dlogits,
                                 size_t rows, size_t vocab, float* loss, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (!loss) return fail(c, CFATTN_ERR_ARG, "null loss");
     *loss = 0.0f;
     if (rows == 0) return CFATTN_OK;
@@ -322,7 +323,7 @@ static int lm_head_ce_queue(cfattn_ctx* c, const float* hn, const float* head, c
 
 int cfops_lm_head_ce(cfattn_ctx* c, const float* hn, const float* head, const int64_t* targets, size_t t, size_t d,
                      size_t vocab, float* dhn, float* dhead, float* loss, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (!loss) return fail(c, CFATTN_ERR_ARG, "null loss");
     *loss = 0.0f;
     if (t == 0) return CFATTN_OK;
@@ -344,7 +345,7 @@ static_assert(sizeof(cfops_ce_result) == sizeof(cfattn::CeMisc) &&
 
 int cfops_lm_head_ce_dev(cfattn_ctx* c, const float* hn, const float* head, const int64_t* targets, size_t t,
                          size_t d, size_t vocab, float* dhn, float* dhead, cfops_ce_result* result, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (!result) return fail(c, CFATTN_ERR_ARG, "null result");
     if (t == 0) return fail(c, CFATTN_ERR_ARG, "t must be positive");
     if (!hn || !head || !targets || !dhn) return fail(c, CFATTN_ERR_ARG, "null buffer");
@@ -356,7 +357,7 @@ int cfops_lm_head_ce_dev(cfattn_ctx* c, const float* hn, const float* head, cons
 int cfops_linear_forward(cfattn_ctx* c, const float* x, const float* w, const float* lora_a, const float* lora_b,
                          float lora_scale, size_t t, size_t in, size_t out, size_t rank, float* y, float* xs,
                          void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (t == 0 || out == 0) return CFATTN_OK;
     if (!x || !w || !y) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (lora_a && (!lora_b || !xs || rank == 0)) return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
@@ -370,7 +371,7 @@ int cfops_linear_forward(cfattn_ctx* c, const float* x, const float* w, const fl
 int cfops_linear_backward(cfattn_ctx* c, const float* x, const float* xs, const float* dy, const float* w,
                           const float* lora_a, const float* lora_b, float lora_scale, size_t t, size_t in, size_t out,
                           size_t rank, float* dx, float* gw, float* ga, float* gb, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (t == 0) return CFATTN_OK;
     if (!x || !dy || !w || !dx) return fail(c, CFATTN_ERR_ARG, "null buffer");
     if (lora_a && (!lora_b || !xs || rank == 0)) return fail(c, CFATTN_ERR_ARG, "adapter needs A, B, xs and rank > 0");
@@ -383,7 +384,7 @@ int cfops_linear_backward(cfattn_ctx* c, const float* x, const float* xs, const 
 
 int cfops_linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, const cfops_linear* lin, size_t n,
                           void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (t == 0 || n == 0) return CFATTN_OK;
     if (!x || !lin) return fail(c, CFATTN_ERR_ARG, "null buffer");
     for (size_t i = 0; i < n; i++) {
@@ -402,7 +403,7 @@ int cfops_linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, co
 
 int cfops_linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin,
                            size_t n, int acc, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (t == 0 && !acc)
         for (size_t i = 0; lin && i < n; i++) {
             const cfops_linear& l = lin[i];
@@ -435,7 +436,7 @@ int cfops_adamw_update(cfattn_ctx* c, float* p, const float* g, float* m, float*
 int cfops_adamw_update_multi(cfattn_ctx* c, size_t count, float* const* p, const float* const* g, float* const* m,
                              float* const* v, const size_t* n, const float* weight_decay, uint64_t t, float lr,
                              float beta1, float beta2, float eps, void* stream) {
-    CF_LOCK(c);
+    CF_LOCK(c, stream);
     if (count && (!p || !g || !m || !v || !n || !weight_decay)) return fail(c, CFATTN_ERR_ARG, "null array");
     for (size_t i = 0; i < count; i++)
         if (n[i] && (!p[i] || !g[i] || !m[i] || !v[i])) return fail(c, CFATTN_ERR_ARG, "null buffer");

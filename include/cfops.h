@@ -7,7 +7,10 @@
  * slices, so a layer's activations stay in HBM between the projections, the
  * norms and the attention (include/cfattn.h).  `stream` NULL is the device's
  * null stream.  A context (cfattn_create) provides the device and the
- * scratch pool; calls on one context are serialised.  Status codes and cfattn_last_error() are those of cfattn.h.
+ * scratch pool.  Its calls are queued one at a time and share the scratch: on
+ * different streams they must not overlap, and neither may a graph's replays
+ * that such calls were recorded into (their scratch stays allocated until
+ * cfattn_destroy).  Status codes and cfattn_last_error() are those of cfattn.h.
  *
  * Reference sources (Sm0r3s-source/cpuforge, crates/...):
  *   core/src/matmul.rs:127-147   matmul_nn / matmul_nt / matmul_tn

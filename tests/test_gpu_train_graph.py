@@ -51,6 +51,48 @@ def test_graph_replays_match_the_eager_step():
         torch.cuda.synchronize()
 
 
+def test_replays_after_eager_calls_that_need_more_scratch(monkeypatch):
+    """Eager work between replays that outgrows every scratch buffer the graph
+    uses (adapters of more linears and a higher rank, a larger LM head, longer
+    attention, a wider norm) leaves the graph's own buffers in place."""
+    from cpuforge_amd import Context, attention
+    from cpuforge_amd import autograd as A
+    from cpuforge_amd import device as D
+    monkeypatch.setattr(attention, "_default", Context(0))  # none of its scratch grown yet
+    B, S, vocab = 1, 64, 2048
+    model = SmolLM(layers=1, seq=S, rank=8, dtype=torch.float32, device="cuda", backend="cfops",
+                   config={"vocab": vocab})
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    tokens, targets = (torch.randint(0, vocab, (B, S), generator=gen, device="cuda") for _ in range(2))
+    params = model.params()
+    loss = model.loss(tokens, targets)
+    loss.backward()
+    ref_loss, ref = loss.item(), [p.grad.clone() for p in params]
+    del loss
+    model.ce_on_device = True
+    graph, static_loss = capture_step(model, tokens, targets)
+    R = lambda *s: torch.randn(*s, generator=gen, device="cuda").requires_grad_()  # noqa: E731
+    for rep in range(3):
+        print(f"replay {rep}", flush=True)
+        t, d, r = 900 << rep, 1024, 16 << rep
+        x, gain = R(t, d), R(d)
+        ys = A.shared_input_linears(A.rmsnorm(x, gain, 1e-5), [(R(d, d), R(r, d), R(d, r), 2.0) for _ in range(4)])
+        loss = A.lm_head_ce(ys[0] + ys[1] + ys[2] + ys[3], R(9000 << rep, d), torch.zeros(t, dtype=torch.long, device="cuda"))
+        loss.backward()
+        q, k = (torch.randn(2, 1024 << rep, h, 64, generator=gen, device="cuda") for h in (9, 3))
+        D.bwd(q, q, k, k, *D.fwd(q, k, k))
+        # What was given back, if anything was, is in use by others.
+        junk = [torch.full((1 << 22,), float("nan"), device="cuda") for _ in range(16)]
+        graph.replay()
+        torch.cuda.synchronize()
+        model.check_targets()
+        assert static_loss.item() == ref_loss, rep
+        for i, (p, g) in enumerate(zip(params, ref)):
+            assert torch.equal(p.grad, g), (rep, i)
+        assert all(bool(j.isnan().all()) for j in junk)
+
+
 def test_device_loss_matches_the_host_loss_and_reports_a_bad_target():
     t, d, vocab = 8, 64, 5
     gen = torch.Generator(device="cuda")
