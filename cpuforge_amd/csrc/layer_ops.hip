@@ -266,9 +266,8 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const float* __re
     float4 wv[V], gain[V];
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const int c = lane + 64 * i;
-        wv[i] = c < n4 ? reinterpret_cast<const float4*>(w)[c] : zero;
-        gain[i] = zero;
+        wv[i] = gain[i] = zero;
+        if (lane + 64 * i < n4) wv[i] = reinterpret_cast<const float4*>(w)[lane + 64 * i];
     }
     const long r0 = (long)blockIdx.x * kRmsBlockRows + wave * kRmsWaveRows;
     float4 xv[kRmsWaveRows][V], gv[kRmsWaveRows][V];
@@ -279,9 +278,13 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const float* __re
         inv[k] = rstd[r];
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const int c = lane + 64 * i;
-            xv[k][i] = c < n4 ? reinterpret_cast<const float4*>(x + r * dim)[c] : zero;
-            gv[k][i] = c < n4 ? reinterpret_cast<const float4*>(dy + r * dim)[c] : zero;
+            // (Not `? :`: both sides are lvalues, which makes one flat load of
+            // either memory or a zero in scratch.)
+            xv[k][i] = gv[k][i] = zero;
+            if (lane + 64 * i < n4) {
+                xv[k][i] = reinterpret_cast<const float4*>(x + r * dim)[lane + 64 * i];
+                gv[k][i] = reinterpret_cast<const float4*>(dy + r * dim)[lane + 64 * i];
+            }
         }
     }
 #pragma unroll
