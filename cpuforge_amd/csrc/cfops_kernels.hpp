@@ -106,6 +106,7 @@ struct LoraDownJob {
 struct LoraDown {
     LoraDownJob job[kGemmProblems];
     int njobs = 0, t = 0;
+    int y0 = 0;  // set by launch_lora_down
 };
 hipError_t launch_lora_down(const LoraDown& g, bool m_rows, hipStream_t st);
 struct LoraGradJob {

@@ -181,8 +181,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
     int tn = g.n_inner ? id % g.nt : id / g.mt;
     int pi = 0;
     long part_off = 0;  // columns of the problems before this one
-    for (; pi + 1 < g.npr && tn >= (g.pr[pi].n + BN - 1) / BN; pi++) {
-        tn -= (g.pr[pi].n + BN - 1) / BN;
+    for (; pi + 1 < g.npr && tn > (g.pr[pi].n - 1) / BN; pi++) {
+        tn -= (g.pr[pi].n - 1) / BN + 1;
         part_off += g.pr[pi].n;
     }
     const GemmProblem& p = g.pr[pi];
@@ -327,19 +327,21 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
             for (int j = 0; j < NB; j++) acc[i][j] = zero16();
         auto run = [&](const GemmSeg& s, int k0, int k1) {
             // Two groups of eight k: the loads of both are in flight together.
-            for (int k = k0; k < k1; k += 16) {
+            const unsigned n = max(k1 - k0, 0);
+            for (unsigned d = 0; d < n; d += 16) {
                 float a[2][MB][4], b[2][NB][4];
 #pragma unroll
                 for (int h = 0; h < 2; h++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const int ke = k + 8 * h + 4 * hh + e;
+                        const unsigned de = d + 8 * h + 4 * hh + e;
+                        const long k = k0 + (long)de;
 #pragma unroll
                         for (int i = 0; i < MB; i++)
-                            a[h][i][e] = ke < k1 ? elem<AS>(s.a, s.lda, m0 + min(ar + 32 * i, lastA), ke) : 0.0f;
+                            a[h][i][e] = de < n ? elem<AS>(s.a, s.lda, m0 + min(ar + 32 * i, lastA), k) : 0.0f;
 #pragma unroll
                         for (int j = 0; j < NB; j++)
-                            b[h][j][e] = ke < k1 ? elem<BS>(s.b, s.ldb, n0 + min(br + 32 * j, lastB), ke) : 0.0f;
+                            b[h][j][e] = de < n ? elem<BS>(s.b, s.ldb, n0 + min(br + 32 * j, lastB), k) : 0.0f;
                     }
 #pragma unroll
                 for (int h = 0; h < 2; h++)
@@ -364,7 +366,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
             run(p.seg[oc.seg], oc.k, oc.k + oc.len);
         }
     }
-    const int mw = m0 + (wave >> 1) * (BM / WR) + 4 * hh, nw = n0 + br;
+    // (Unsigned: a tile's last rows and columns may lie past 2^31.)
+    const unsigned mw = (unsigned)m0 + (wave >> 1) * (BM / WR) + 4 * hh, nw = (unsigned)n0 + br;
 
     // Partial products: [split][m][all problems' columns, problem by problem].
     float* out = p.c;
@@ -378,12 +381,12 @@ __global__ __launch_bounds__(NT, 2) void gemm_f32_kernel(const GemmArgs g) {
     for (int i = 0; i < MB; i++)
 #pragma unroll
         for (int j = 0; j < NB; j++) {
-            const int col = nw + 32 * j;
-            if (col >= p.n) continue;
+            const unsigned col = nw + 32 * j;
+            if (col >= (unsigned)p.n) continue;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int row = mw + 32 * i + 8 * (r >> 2) + (r & 3);
-                if (row >= g.m) continue;
+                const unsigned row = mw + 32 * i + 8 * (r >> 2) + (r & 3);
+                if (row >= (unsigned)g.m) continue;
                 float* o = out + (long)row * p.n + col;
                 *o = add ? *o + acc[i][j][r] : acc[i][j][r];
             }
@@ -404,7 +407,7 @@ __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmArgs g, 
     }
 }
 
-int cdiv(int a, int b) { return (a + b - 1) / b; }
+int cdiv(int a, int b) { return (a - 1) / b + 1; }  // a > 0
 
 // The tiles.  A step (32 k) of each, measured with one workgroup to a CU and
 // with the chip full (power then holds the clock near 1.8 of 2.4 GHz):
@@ -417,6 +420,7 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // or three, and 256 x 256 were never the best.)
 enum Tile { kTile256, kTile128, kTile64, kNumTiles };
 constexpr int kTileM[kNumTiles] = {256, 128, 64}, kTileN[kNumTiles] = {128, 128, 64};
+constexpr int kTileLogThreads[kNumTiles] = {9, 9, 8};
 constexpr int kCus = 256;
 
 // Modelled time of one launch, in us: rounds over the CUs of a workgroup's steps
@@ -472,6 +476,7 @@ hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipSt
             const int per = cdiv(steps, sp);
             if (cdiv(steps, per) != sp) continue;
             if (sp > 1 && (size_t)(sp * cols) * g.m > ws_floats) break;
+            if ((tiles * sp) << kTileLogThreads[ti] > UINT32_MAX) break;  // threads of a launch
             double t = tile_time((Tile)ti, tiles * sp, per);
             if (sp > 1) t += 4.0 + (2.0 * sp + 1.0) * cols * g.m * 4.0 / 4e6;
             if (best < 0 || t < best) best = t, tile = (Tile)ti, splits = sp;
@@ -486,7 +491,7 @@ hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipSt
     // the smaller operand (each XCD then reads all of it), else over m.
     g.n_inner = cols < g.m;
     const long grid = (long)g.mt * g.nt * splits;
-    if (grid > INT32_MAX) return hipErrorInvalidConfiguration;
+    if (best < 0) return hipErrorInvalidConfiguration;
     if (in.a_strided)
         launch_tile<true, true>(g, tile, far, (int)grid, st);
     else if (in.b_strided)

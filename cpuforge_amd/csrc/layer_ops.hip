@@ -391,9 +391,11 @@ hipError_t launch_rmsnorm_bwd(const float* dy, const float* x, const float* w, c
     if (rows == 0 || dim == 0) return hipSuccess;
     float* part = dw ? partial : nullptr;
     size_t nblk;
-    if (dim % 4 == 0 && dim <= 2048 && aligned16(dy) && aligned16(x) && aligned16(dx) && aligned16(w)) {
-        nblk = (rows + kRmsBlockRows - 1) / kRmsBlockRows;
-        if (nblk > 0x7fffffffu) return hipErrorInvalidConfiguration;
+    // (A launch has fewer than 2^32 threads; more rows than that take the
+    // staged kernel, whose blocks hold up to 16.)
+    nblk = (rows + kRmsBlockRows - 1) / kRmsBlockRows;
+    if (dim % 4 == 0 && dim <= 2048 && nblk < (1u << 24) && aligned16(dy) && aligned16(x) && aligned16(dx) &&
+        aligned16(w)) {
         const size_t lds = part ? 4 * dim * sizeof(float) : 0;
         const auto kernel = dim <= 256   ? rmsnorm_bwd_wave_kernel<1>
                             : dim <= 512 ? rmsnorm_bwd_wave_kernel<2>

@@ -19,6 +19,7 @@
 // the down products of a group, 12.5 + 4.6 the gradients).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "cfops_kernels.hpp"
@@ -53,7 +54,7 @@ constexpr int kBatch = 4;  // runs of a wave whose loads are in flight together
 template <bool MROW>
 __global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(const LoraDown g) {
     __shared__ float red[kDownWaves][16][17];
-    int y = blockIdx.y, ji = 0;
+    int y = blockIdx.y + g.y0, ji = 0;
     while (y >= (g.job[ji].r + 15) / 16) y -= (g.job[ji++].r + 15) / 16;
     const LoraDownJob& p = g.job[ji];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -120,11 +121,13 @@ __global__ __launch_bounds__(256) void lora_grad_kernel(const LoraGrad g) {
     const int n0 = b / nrb * 64, j0 = b % nrb * 16;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int l16 = lane & 15, tq = lane >> 4;
-    const int i0 = blockIdx.y * g.tokens, i1 = min(g.t, i0 + g.tokens);
-    const int col = n0 + 4 * l16, left = max(0, min(4, p.ncol - col));
+    // (Unsigned: past the last token by up to a batch without overflow.)
+    const unsigned i0 = blockIdx.y * g.tokens, i1 = min((unsigned)g.t, i0 + g.tokens);
+    const int left = max(0, min(4, p.ncol - n0 - 4 * l16));
+    const long col = (long)n0 + 4 * l16;
     const int j = min(j0 + l16, p.r - 1);
     f32x4 acc[4] = {};
-    auto add = [&](int i, bool in) {
+    auto add = [&](unsigned i, bool in) {
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         float s = 0.0f;
         if (in) {
@@ -134,8 +137,8 @@ __global__ __launch_bounds__(256) void lora_grad_kernel(const LoraGrad g) {
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] = mfma16(v[q], s, acc[q]);
     };
-    int i = i0 + 4 * wave;
-    if (n0 + 64 <= p.ncol)
+    unsigned i = i0 + 4 * wave;
+    if (p.ncol - n0 >= 64)
         for (; i + 16 * (kBatch - 1) + 4 <= i1; i += 16 * kBatch) {
             f32x4 v[kBatch];
             float s[kBatch];
@@ -160,8 +163,8 @@ __global__ __launch_bounds__(256) void lora_grad_kernel(const LoraGrad g) {
     float* out = g.part + p.off + (long)blockIdx.y * p.ncol * p.r;
     for (int e = tid; e < 1024; e += 256) {
         const int n = e >> 4, jj = e & 15;
-        if (n0 + n >= p.ncol || j0 + jj >= p.r) continue;
-        out[(long)(n0 + n) * p.r + j0 + jj] = red[0][n][jj] + red[1][n][jj] + red[2][n][jj] + red[3][n][jj];
+        if (n >= p.ncol - n0 || jj >= p.r - j0) continue;
+        out[((long)n0 + n) * p.r + j0 + jj] = red[0][n][jj] + red[1][n][jj] + red[2][n][jj] + red[3][n][jj];
     }
 }
 
@@ -192,14 +195,26 @@ int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 hipError_t launch_lora_down(const LoraDown& g, bool m_rows, hipStream_t st) {
     int blocks = 0;
     for (int i = 0; i < g.njobs; i++) blocks += cdiv(g.job[i].r, 16);
-    if (blocks == 0) return hipSuccess;
-    if (blocks > 65535) return hipErrorInvalidConfiguration;
-    const dim3 grid(cdiv(g.t, 16), blocks);
-    if (m_rows)
-        lora_down_kernel<true><<<grid, 64 * kDownWaves, 0, st>>>(g);
-    else
-        lora_down_kernel<false><<<grid, 64 * kDownWaves, 0, st>>>(g);
-    return hipGetLastError();
+    // One launch up to 2^27 tokens and 65535 blocks of ranks (a grid has fewer
+    // than 2^32 threads along x and 2^16 blocks along y).
+    constexpr int kTokens = (1 << 27) - 16, kBlocksY = 65535;
+    LoraDown l = g;
+    for (l.y0 = 0; l.y0 < blocks; l.y0 += kBlocksY)
+        for (int t0 = 0; t0 < g.t; t0 += l.t) {
+            l.t = std::min(g.t - t0, kTokens);
+            for (int i = 0; i < g.njobs; i++) {
+                l.job[i].src = g.job[i].src + (long)t0 * g.job[i].k;
+                l.job[i].out = g.job[i].out + (long)t0 * g.job[i].r;
+            }
+            const dim3 grid(cdiv(l.t, 16), std::min(blocks - l.y0, kBlocksY));
+            if (m_rows)
+                lora_down_kernel<true><<<grid, 64 * kDownWaves, 0, st>>>(l);
+            else
+                lora_down_kernel<false><<<grid, 64 * kDownWaves, 0, st>>>(l);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
 }
 
 size_t lora_grad_plan(LoraGrad& g) {
@@ -210,7 +225,7 @@ size_t lora_grad_plan(LoraGrad& g) {
     const int most = cdiv(g.t, 64);
     int chunks = blocks ? cdiv(768, blocks) : 1;
     if (chunks > most) chunks = most;
-    g.tokens = cdiv(cdiv(g.t, chunks), 64) * 64;
+    g.tokens = std::min((long)cdiv(cdiv(g.t, chunks), 64) * 64, (long)INT32_MAX);
     g.chunks = cdiv(g.t, g.tokens);
     long off = 0;
     for (int i = 0; i < g.njobs; i++) {

@@ -120,3 +120,30 @@ def test_linear_functions_by_name():
     for y, got in zip(outs[1:], grads[1:]):
         assert torch.equal(y, outs[0]) and all(torch.equal(p, q) for p, q in zip(got, grads[0]))
     assert A.LinearFn.apply(x, w, None, None, 1.0).shape == (2, 9, 50)
+
+
+@pytest.mark.parametrize("t,inn,out,r", [((1 << 27) + 50, 2, 1, 1), (3, 2, 2, 65536 * 16 + 3)])
+def test_adapter_beyond_one_launch(t, inn, out, r):
+    """More tokens, and a higher rank, than the threads and blocks of one launch."""
+    from cpuforge_amd import ops as P
+    g = torch.Generator(device=DEV).manual_seed(r)
+    R = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    x, w, a, b = R(t, inn), R(out, inn), R(r, inn), R(out, r)
+    xs, y = torch.full((t, r), float("nan"), device=DEV), torch.full((t, out), float("nan"), device=DEV)
+    li = dict(w=w, lora_a=a, lora_b=b, scale=0.5)
+    P.linears_forward(x, t, inn, [dict(li, y=y, xs=xs)])
+    dy = R(t, out)
+    dx, ga, gb = torch.full_like(x, float("nan")), torch.empty_like(a), torch.empty_like(b)
+    P.linears_backward(x, t, inn, dx, [dict(li, xs=xs, dy=dy, ga=ga, gb=gb)], acc=False)
+    n = min(t, 500)
+    for part in (slice(0, n), slice(t - n, t)):
+        xd, wxs = x[part].double(), 0.5 * (x[part].double() @ a.double().t())
+        close = lambda u, v, m: bool(((u[part] - v).abs() <= 2.0 ** -20 * m + 1e-30).all())  # noqa: E731
+        assert close(xs, wxs, xd.abs() @ a.double().abs().t())
+        assert close(y, xd @ w.double().t() + wxs @ b.double().t(), 1e3 + wxs.abs() @ b.double().abs().t())
+        gd = dy[part].double()
+        want = gd @ w.double() + (0.5 * (gd @ b.double())) @ a.double()
+        assert close(dx, want, 1e3 + 0.5 * (gd.abs() @ b.double().abs()) @ a.double().abs())
+    sums = dy.double().t() @ xs.double()
+    assert bool(((gb - sums).abs() <= 1e-4 * sums.abs().max()).all())
+    assert bool(ga.isfinite().all())

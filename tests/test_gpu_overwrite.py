@@ -70,3 +70,23 @@ def test_gradients_of_no_rows_are_zero():
     dx = nan(5, 24)
     P.linears_backward(torch.randn(5, 24, device=DEV), 5, 24, dx, [], acc=False)  # of no linears
     assert bool((dx == 0).all())
+
+
+def test_rmsnorm_backward_of_more_rows_than_a_launch_has_waves():
+    """2^27 rows and more: one wave to two rows would be 2^32 threads."""
+    from cpuforge_amd import ops as P
+    rows, dim = (1 << 27) + 100, 4
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, dy = (torch.randn(rows, dim, generator=g, device=DEV) for _ in range(2))
+    w = torch.tensor([1.0, 0.5, -2.0, 1.5], device=DEV)
+    rstd, dx = torch.empty(rows, device=DEV), torch.full_like(x, float("nan"))
+    y = torch.empty_like(x)
+    P.rmsnorm_forward(x, w, y, rstd, rows, dim, 1e-5)
+    P.rmsnorm_backward(dy, x, w, rstd, dx, None, rows, dim, acc=False)
+    for part in (slice(0, 1000), slice(rows - 1000, rows)):
+        xd, gd, inv = x[part].double(), dy[part].double(), rstd[part].double()[:, None]
+        xh = xd * inv
+        want = inv * (gd * w.double() - xh * (gd * w.double() * xh).mean(-1, keepdim=True))
+        mag = inv * ((gd * w).abs() + xh.abs() * (gd * w * xh).abs().mean(-1, keepdim=True))
+        assert bool(((dx[part] - want).abs() <= 2.0 ** -24 * 20 * mag).all())
+    assert not bool(dx.isnan().any())
