@@ -1,13 +1,15 @@
 // f32 values as three bf16 pieces, for f32 products on the bf16 matrix cores.
 //
-// x = p0 + p1 + p2 with p0 = bf16(x), p1 = bf16(x - p0), p2 = x - p0 - p1:
-// each rounding (to nearest even) leaves a residual of at most 2^-9 of what
-// it rounded, both subtractions are exact in f32, and 8 + 8 + 8 significand
-// bits with the residuals' signs hold all 24 of x.  A product of two split
-// values is the six piece products of weight 2^-18 and above,
+// x = p0 + p1 + p2 with p0 = bf16(x), p1 = bf16(x - p0), p2 = x - p0 - p1: both
+// subtractions are exact in f32, p1 is at most 2^-8 and p2 2^-17 of x, and the
+// three 8-bit significands with the residuals' signs hold all 24 bits of x.  A
+// product of two split values is the six piece products
 //   a0 b0 + a0 b1 + a1 b0 + a1 b1 + a0 b2 + a2 b0,
-// each exact (8 x 8 bits), summed in f32 by the MFMA; the three products
-// left out are below 2^-26 of |a b| together, a quarter of an f32 rounding.
+// each exact (8 x 8 bits), summed in f32 by the MFMA; the three left out are
+// together at most 2^-24 of |a b|, about one f32 rounding, and 2^-28 as a rule
+// (2^-26 is passed by 3.5% of random pairs).  (The split and the choice of
+// products: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", ARITH 2019.)
 // v_mfma_f32_32x32x16_bf16 does 16x the work of v_mfma_f32_32x32x2_f32 in the
 // same number of passes: six of them are 2.7x the f32 MFMA rate.
 //
