@@ -99,20 +99,22 @@ int check_linears(cfattn_ctx* c, size_t t, size_t in, const cfops_linear* lin, s
 // input: xs_i = scale_i x A_i^T in one launch, then y_i = [x xs_i] [W_i B_i]^T in one.
 int linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, const cfops_linear* lin, size_t n,
                     hipStream_t st) {
-    cfattn::LoraDown d;
-    cfattn::GemmF32 g;
-    d.t = g.m = (int)t;
+    cfattn::GemmF32 g, down;
+    down.m = g.m = (int)t;
     for (size_t i = 0; i < n; i++) {
         const cfops_linear& l = lin[i];
-        if (l.lora_a)
-            d.job[d.njobs++] = {x, l.lora_a, l.xs, l.lora_scale, (int)in, (int)l.rank};
+        if (l.lora_a) {
+            cfattn::GemmProblem& p = down.pr[down.npr++];
+            p.seg[p.nseg++] = {x, l.lora_a, (long)in, (long)in, (int)in};
+            p.c = l.xs, p.n = (int)l.rank, p.scale = l.lora_scale;
+        }
         if (l.out == 0) continue;
         cfattn::GemmProblem& p = g.pr[g.npr++];
         p.c = l.y, p.n = (int)l.out;
         p.seg[p.nseg++] = {x, l.w, (long)in, (long)in, (int)in};
         if (l.lora_a) p.seg[p.nseg++] = {l.xs, l.lora_b, (long)l.rank, (long)l.rank, (int)l.rank};
     }
-    CF_HIP(c, cfattn::launch_lora_down(d, true, st), "lora launch");
+    CF_HIP(c, cfattn::launch_gemm_rows(down, st), "GEMM launch");
     return g.npr ? launch_gemm(c, g, st) : CFATTN_OK;
 }
 
@@ -121,8 +123,7 @@ int linears_forward(cfattn_ctx* c, const float* x, size_t t, size_t in, const cf
 // [W_1; A_1; W_2; ..] in one; the adapters' gradients in two.
 int linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* dx, const cfops_linear* lin, size_t n,
                      bool acc_dx, bool acc, hipStream_t st) {
-    cfattn::LoraDown d;
-    cfattn::GemmF32 g;
+    cfattn::GemmF32 g, down;
     cfattn::LoraGrad lg;
     int rc = CFATTN_OK;
     size_t dxa_floats = 0;
@@ -132,8 +133,8 @@ int linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* 
         dxa = static_cast<float*>(slot(c, cfattn_ctx::OPS_DXA, dxa_floats * sizeof(float), &rc));
         if (!dxa) return rc;
     }
-    d.t = g.m = lg.t = (int)t;
-    g.b_strided = true, g.acc = acc_dx, lg.acc = acc;
+    down.m = g.m = lg.t = (int)t;
+    down.b_strided = g.b_strided = true, g.acc = acc_dx, lg.acc = acc;
     g.npr = 1, g.pr[0].c = dx, g.pr[0].n = (int)in;
     for (size_t i = 0; i < n; i++) {
         const cfops_linear& l = lin[i];
@@ -141,14 +142,16 @@ int linears_backward(cfattn_ctx* c, const float* x, size_t t, size_t in, float* 
         seg[g.pr[0].nseg++] = {l.dy, l.w, (long)l.out, (long)in, (int)l.out};
         if (!l.lora_a) continue;
         if (dx || l.ga) {
-            d.job[d.njobs++] = {l.dy, l.lora_b, dxa, l.lora_scale, (int)l.out, (int)l.rank};
+            cfattn::GemmProblem& p = down.pr[down.npr++];
+            p.seg[p.nseg++] = {l.dy, l.lora_b, (long)l.out, (long)l.rank, (int)l.out};
+            p.c = dxa, p.n = (int)l.rank, p.scale = l.lora_scale;
             seg[g.pr[0].nseg++] = {dxa, l.lora_a, (long)l.rank, (long)in, (int)l.rank};
         }
         if (l.gb && l.out) lg.job[lg.njobs++] = {l.dy, l.xs, l.gb, (int)l.out, (int)l.rank, 0, 0};
         if (l.ga && in) lg.job[lg.njobs++] = {x, dxa, l.ga, (int)in, (int)l.rank, 1, 0};
         dxa += t * l.rank;
     }
-    CF_HIP(c, cfattn::launch_lora_down(d, false, st), "lora launch");
+    CF_HIP(c, cfattn::launch_gemm_rows(down, st), "GEMM launch");
     if (dx && in) CF_TRY(launch_gemm(c, g, st));
     for (size_t i = 0; i < n; i++)
         if (lin[i].gw) CF_TRY(gemm(c, CFOPS_TN, lin[i].dy, x, lin[i].gw, lin[i].out, t, in, acc, st));

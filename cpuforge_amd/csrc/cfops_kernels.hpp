@@ -80,6 +80,7 @@ struct GemmProblem {
     int nseg = 0;
     float* c = nullptr;
     int n = 0;
+    float scale = 1.0f;  // of the sum (launch_gemm_rows only)
 };
 struct GemmF32 {
     GemmProblem pr[kGemmProblems];
@@ -89,26 +90,15 @@ struct GemmF32 {
 };
 // `ws` is scratch for the partial sums of a split contraction.
 hipError_t launch_gemm_f32(const GemmF32& g, float* ws, size_t ws_floats, hipStream_t st);
+// The same products on the f32 MFMA, a workgroup to 16 rows and 16 columns, for
+// a_strided = false: an adapter's products with its rank as n, and those of few
+// rows, which launch_gemm_f32 passes on.
+hipError_t launch_gemm_rows(const GemmF32& g, hipStream_t st);
 
-// LoRA adapter products of Linear::forward / backward (linear.rs:56-91) with
-// the rank as a dimension of the result (lora.hip), for up to kGemmProblems
-// linears over the same t tokens in one launch:
-//   down:  out = scale * src m^T (m [r x k], m_rows: xs = scale x A^T) or
-//          scale * src m (m [k x r]: dxa = scale dy B), out [t x r];
-//   grad:  out (+)= big^T small, [ncol x r] (gb from dy and xs), or its
-//          transpose [r x ncol] (ga from x and dxa).
-struct LoraDownJob {
-    const float *src, *m;
-    float* out;
-    float scale;
-    int k, r;
-};
-struct LoraDown {
-    LoraDownJob job[kGemmProblems];
-    int njobs = 0, t = 0;
-    int y0 = 0;  // set by launch_lora_down
-};
-hipError_t launch_lora_down(const LoraDown& g, bool m_rows, hipStream_t st);
+// The gradients of LoRA adapters in Linear::backward (linear.rs:75-90), for up
+// to kGemmProblems linears over the same t tokens in one launch (lora.hip):
+//   out (+)= big^T small, [ncol x r] (gb from dy and xs), or its transpose
+//   [r x ncol] (ga from x and dxa).
 struct LoraGradJob {
     const float *big, *small;
     float* out;

@@ -29,6 +29,7 @@
 // further off than before).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -50,6 +51,7 @@ struct GemmArgs {
     int per;             // k steps per split
     int n_inner;
     float* part;         // partial products of the splits, or null
+    int y0;              // rows kernel: first column block of the launch
 };
 
 template <bool STRIDED>
@@ -407,6 +409,105 @@ __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const GemmArgs g, 
     }
 }
 
+// ------------------------------------------------------------------- rows
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// p[0..3], elements at or past n zero (and not read).
+__device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int n) {
+    if (n >= 4) return *reinterpret_cast<const f32x4u*>(p);
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < n; i++) v[i] = p[i];
+    return v;
+}
+
+constexpr int kRowWaves = 8;
+constexpr int kRowBatch = 4;  // runs of a wave whose loads are in flight together
+
+// The product on the f32 MFMA for few rows or few columns, where a tile of the
+// kernel above is mostly padding and its chain of steps (and the pass that adds
+// a split's sums) all there is: a workgroup takes 16 rows and 16 columns, its
+// waves every kRowWaves-th run of 16 k, straight from memory in MFMA layout (lane
+// l: row and column l % 16, four consecutive k, one per MFMA), and their sums
+// are added in wave order.  Bound: the latency of a wave's loads, four runs in
+// flight (1.7 us a batch), on each CU one workgroup after the other.
+// In us for m x k x n, a library's f32 kernels, the kernel above and this: 1 x 576 x
+// 1536 4.8, 8.5, 3.8; 16 x 576 x 1536 4.8, 8.8, 4.5; 16 x 1536 x 576 6.1, 10.2, 7.6; 64 x
+// 576 x 1536 6.6, 9.8, 6.3; 1 x 576 x 49152 20.3, 29.6, 19.7; 16 x 2048 x 8192 13.8, 22.8,
+// 17.5.  An adapter's products at 4096 tokens, rank 16: 7.7 (xs) and 9.4 (dxa) for
+// the gate and up projections.  (32 x 32 tiles, and eight runs in flight: slower.)
+// Relative error against 64 bits, the same three: k = 576 2.2e-7, 0.8e-7, 1.0e-7; k
+// = 2048 4.1e-7, 1.3e-7, 1.6e-7.
+// Off: type of a byte offset within 16 rows of B.
+template <bool BS, typename Off = uint32_t>
+__global__ __launch_bounds__(64 * kRowWaves) void gemm_rows_kernel(const GemmArgs g) {
+    __shared__ float red[kRowWaves][16][17];
+    int y = blockIdx.y + g.y0, pi = 0;
+    while (y > (g.pr[pi].n - 1) / 16) y -= (g.pr[pi++].n - 1) / 16 + 1;
+    const GemmProblem& p = g.pr[pi];
+    const int tid = threadIdx.x, wave = wave_uniform(tid >> 6), lane = tid & 63;
+    const int l16 = lane & 15, kq = (lane >> 4) * 4;
+    const int row0 = blockIdx.x * 16, j0 = y * 16;
+    const int row = row0 + min(l16, g.m - 1 - row0), j = j0 + min(l16, p.n - 1 - j0);
+    // Lane l of v_mfma_f32_16x16x4_f32 holds A[l % 16][l / 16], B[l / 16][l % 16]
+    // and C[4 * (l / 16) + i][l % 16], i = 0..3.
+    // Four chains of sums (and the waves' in pairs): a quarter of the roundings
+    // at the full sum's size.
+    f32x4 acc[4] = {};
+    auto add = [&](const f32x4& a, const f32x4& b) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc[i], 0, 0, 0);
+    };
+    for (int s = 0; s < p.nseg; s++) {
+        const GemmSeg& sg = p.seg[s];
+        const float* a = sg.a + (long)row * sg.lda + kq;
+        const float* b = BS ? sg.b : sg.b + (long)j * sg.ldb + kq;
+        const Off at = BS ? 4 * ((Off)kq * (Off)sg.ldb + (Off)j) : 0;
+        // Run c's k, of which this lane has n (at most four).
+        auto operand = [&](int c, int n) {
+            if constexpr (!BS) return load4(b + c * 16, n);
+            const float* q = b + (long)c * 16 * sg.ldb;
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const char* e = reinterpret_cast<const char*>(q + i * sg.ldb) + at;
+                v[i] = i < n ? *reinterpret_cast<const float*>(e) : 0.0f;
+            }
+            return v;
+        };
+        const int whole = sg.k / 16;
+        int c = wave;
+        for (; c + (kRowBatch - 1) * kRowWaves < whole; c += kRowBatch * kRowWaves) {
+            f32x4 av[kRowBatch], bv[kRowBatch];
+#pragma unroll
+            for (int u = 0; u < kRowBatch; u++) {
+                av[u] = load4(a + (c + u * kRowWaves) * 16, 4);
+                bv[u] = operand(c + u * kRowWaves, 4);
+            }
+#pragma unroll
+            for (int u = 0; u < kRowBatch; u++) add(av[u], bv[u]);
+        }
+#pragma unroll 1
+        for (; c < whole; c += kRowWaves) add(load4(a + c * 16, 4), operand(c, 4));
+        if (c == whole && sg.k % 16) {
+            const int n = max(0, min(4, sg.k - c * 16 - kq));
+            add(load4(a + c * 16, n), operand(c, n));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[wave][kq + i][l16] = (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]);
+    __syncthreads();
+    if (tid >= 256) return;
+    const int r = tid >> 4, jj = tid & 15;
+    if (r > g.m - 1 - row0 || jj > p.n - 1 - j0) return;
+    float w[kRowWaves];
+#pragma unroll
+    for (int i = 0; i < kRowWaves; i++) w[i] = red[i][r][jj];
+    static_assert(kRowWaves == 8, "the sum below");
+    const float sum = p.scale * (((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7])));
+    float* o = p.c + ((long)row0 + r) * p.n + j0 + jj;
+    *o = g.acc ? *o + sum : sum;
+}
+
 int cdiv(int a, int b) { return (a - 1) / b + 1; }  // a > 0
 
 // The tiles.  A step (32 k) of each, measured with one workgroup to a CU and
@@ -444,7 +545,56 @@ void launch_tile(const GemmArgs& g, Tile tile, bool far, int grid, hipStream_t s
         gemm_f32_kernel<AS, BS, 64, 64, 256><<<grid, 256, 0, st>>>(g);
 }
 
+// Modelled time of the rows kernel: rounds over the CUs of a workgroup's batches.
+double rows_time(const GemmF32& g) {
+    long wgs = 0, longest = 0;
+    for (int i = 0; i < g.npr; i++) {
+        long k = 0;
+        for (int s = 0; s < g.pr[i].nseg; s++) k += g.pr[i].seg[s].k;
+        longest = std::max(longest, k);
+        wgs += cdiv(g.pr[i].n, 16);
+    }
+    wgs *= cdiv(g.m, 16);
+    return 2.5 + (double)((wgs + kCus - 1) / kCus) * 1.65 * (double)longest / (16 * kRowWaves * kRowBatch);
+}
+
+template <bool BS, typename Off = uint32_t>
+hipError_t launch_rows(const GemmF32& in, hipStream_t st) {
+    GemmArgs g{};
+    int blocks = 0;
+    for (int i = 0; i < in.npr; i++) {
+        g.pr[i] = in.pr[i];
+        blocks += cdiv(in.pr[i].n, 16);
+    }
+    // A launch has fewer than 2^32 threads along x and 2^16 blocks along y.
+    constexpr int kRows = (1 << 27) - 16, kBlocksY = 65535;
+    g.npr = in.npr, g.acc = in.acc;
+    for (g.y0 = 0; g.y0 < blocks; g.y0 += kBlocksY)
+        for (int m0 = 0; m0 < in.m; m0 += g.m) {
+            g.m = std::min(kRows, in.m - m0);
+            for (int i = 0; i < in.npr; i++) {
+                for (int s = 0; s < in.pr[i].nseg; s++)
+                    g.pr[i].seg[s].a = in.pr[i].seg[s].a + m0 * in.pr[i].seg[s].lda;
+                g.pr[i].c = in.pr[i].c + (long)m0 * in.pr[i].n;
+            }
+            const dim3 grid(cdiv(g.m, 16), std::min(blocks - g.y0, kBlocksY));
+            gemm_rows_kernel<BS, Off><<<grid, 64 * kRowWaves, 0, st>>>(g);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
+}
+
 }  // namespace
+
+hipError_t launch_gemm_rows(const GemmF32& g, hipStream_t st) {
+    if (g.npr == 0 || g.m == 0) return hipSuccess;
+    if (!g.b_strided) return launch_rows<false>(g, st);
+    long ldb = 0;
+    for (int i = 0; i < g.npr; i++)
+        for (int s = 0; s < g.pr[i].nseg; s++) ldb = std::max(ldb, g.pr[i].seg[s].ldb);
+    return ldb < 1L << 26 ? launch_rows<true>(g, st) : launch_rows<true, uint64_t>(g, st);
+}
 
 hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipStream_t st) {
     GemmArgs g{};
@@ -482,6 +632,8 @@ hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipSt
             if (best < 0 || t < best) best = t, tile = (Tile)ti, splits = sp;
         }
     }
+    if (!in.a_strided && (best < 0 || rows_time(in) < best)) return launch_gemm_rows(in, st);
+    if (best < 0) return hipErrorInvalidConfiguration;
     g.per = cdiv(steps, splits);
     splits = cdiv(steps, g.per);
     g.mt = cdiv(g.m, kTileM[tile]);
@@ -491,7 +643,6 @@ hipError_t launch_gemm_f32(const GemmF32& in, float* ws, size_t ws_floats, hipSt
     // the smaller operand (each XCD then reads all of it), else over m.
     g.n_inner = cols < g.m;
     const long grid = (long)g.mt * g.nt * splits;
-    if (best < 0) return hipErrorInvalidConfiguration;
     if (in.a_strided)
         launch_tile<true, true>(g, tile, far, (int)grid, st);
     else if (in.b_strided)

@@ -562,10 +562,15 @@ __global__ __launch_bounds__(256) void ce_begin_kernel(const int64_t* __restrict
 // One row per workgroup (loss.rs:27-53).  With NV4 > 0 the row stays in
 // registers (NV4 float4 per thread) between the max, the exp sum and the
 // write, so it is read from memory once; NV4 == 0 streams it three times.
-// A CU must have the reads of one row beside the writes of another: with the
-// 64 registers of eight waves to a SIMD, two rows of 1024 threads are at work,
-// where 512 threads of 32 float4 left room for one and memory idle in its
-// reductions (2048 x 49152 on average, 805 MB: 232 -> 154 us, 3.5 -> 5.2 TB/s).
+// A CU must have the reads of one row beside the writes of another.  Up to 12
+// float4 of 1024 threads (49152 columns) fit the 64 registers of eight waves to a
+// SIMD, so that two rows are at work, where 512 threads of up to 32 float4 left
+// room for one and memory idle in its reductions (2048 x 49152 269 -> 211 us with
+// the count and the loss, 2048 x 32000 188 -> 147).  16 float4 take 83, one row to
+// a CU, and gain only the wider reads and reductions (1024 x 57344 170 -> 152,
+// 1024 x 65536 182 -> 164).  Longer rows, and those that are not whole aligned
+// float4, are streamed, which nothing here changed (1024 x 50001 220 us, 512 x
+// 128256 438).
 template <int NV4, int NT>
 __global__ __launch_bounds__(NT, NV4 == 12 || NV4 == 8 ? 8 : 1) void ce_rows_kernel(const float* logits, const int64_t* __restrict__ targets,
                                                              float* dlogits, float* __restrict__ row_loss, long row0,

@@ -1,22 +1,16 @@
-// LoRA adapter products of Linear::forward / Linear::backward
-// (crates/model/src/linear.rs:56-91) whose result has the adapter's rank as
-// a dimension, as streaming passes over their long operand on the f32 MFMA:
-//   forward   xs  = scale * x A^T
-//   backward  dxa = scale * dy B
-//             gb += dy^T xs,  ga += dxa^T x: per-chunk partial sums over the
-//             tokens, then the chunks added in order.
-// The products that widen again, xs B^T and dxa A, are the second segments of
-// the base products' GEMMs (gemm_f32.hip).  Several linears go in one launch.
-// Every sum has a fixed order (no atomics): results are reproducible bit for
-// bit.  Any rank, in blocks of 16; no alignment beyond a float's.
+// The gradients of LoRA adapters in Linear::backward (crates/model/src/
+// linear.rs:75-90), gb += dy^T xs and ga += dxa^T x, as streaming passes over
+// their long operand on the f32 MFMA: per-chunk partial sums over the tokens,
+// then the chunks added in order.  Several linears go in one launch.  Every sum
+// has a fixed order (no atomics): results are reproducible bit for bit.  Any
+// rank, in blocks of 16; no alignment beyond a float's.  (The adapters' other
+// products are gemm_f32.hip's: xs = scale x A^T and dxa = scale dy B on its rows
+// kernel, xs B^T and dxa A as segments of the base products.)
 //
 // Bound: latency of one pass over the long operand (9.4 MB for 4096 x 576,
 // resident in the memory-side cache).  The operands come straight from
 // memory in MFMA layout, 16 bytes a lane: no LDS but for the waves' sums.
-// SmolLM's MLP half of a layer (4096 tokens, rank 16; both directions of three
-// linears): 177 us in 24 launches of the row-dot, update, weight-merge, partial
-// and reduction kernels that were here before, 70 in 8 of these (8.4 and 9.7 us
-// the down products of a group, 12.5 + 4.6 the gradients).
+// 4096 tokens, rank 16, SmolLM's gate and up projections: 15 + 4.8 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,66 +37,7 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int n) {
     return v;
 }
 
-constexpr int kDownWaves = 8;
 constexpr int kBatch = 4;  // runs of a wave whose loads are in flight together
-
-// out[row][j] = scale * sum over k of src[row][k] * m(j, k), with m(j, k) =
-// m[j * K + k] (MROW: the forward's A) or m[k * r + j] (the backward's B).  A
-// workgroup takes 16 rows and 16 j; its waves take every kDownWaves-th run of
-// 16 k (lane l four consecutive k of its row, one per MFMA) and their sums are
-// added in wave order.
-template <bool MROW>
-__global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(const LoraDown g) {
-    __shared__ float red[kDownWaves][16][17];
-    int y = blockIdx.y + g.y0, ji = 0;
-    while (y >= (g.job[ji].r + 15) / 16) y -= (g.job[ji++].r + 15) / 16;
-    const LoraDownJob& p = g.job[ji];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int l16 = lane & 15, kq = (lane >> 4) * 4;
-    const int row0 = blockIdx.x * 16, j0 = y * 16;
-    const float* src = p.src + (long)min(row0 + l16, g.t - 1) * p.k;
-    const int j = min(j0 + l16, p.r - 1);
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto add = [&](const f32x4& a, const f32x4& b) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc = mfma16(a[i], b[i], acc);
-    };
-    auto operand = [&](int k, int n) {
-        if constexpr (MROW) return load4(p.m + (long)j * p.k + k, n);
-        f32x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = i < n ? p.m[(long)(k + i) * p.r + j] : 0.0f;
-        return v;
-    };
-    const int whole = p.k / 16;
-    int c = wave;
-    for (; c + (kBatch - 1) * kDownWaves < whole; c += kBatch * kDownWaves) {
-        f32x4 a[kBatch], b[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int k = (c + u * kDownWaves) * 16 + kq;
-            a[u] = load4(src + k, 4);
-            b[u] = operand(k, 4);
-        }
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) add(a[u], b[u]);
-    }
-    for (; c < whole; c += kDownWaves) add(load4(src + c * 16 + kq, 4), operand(c * 16 + kq, 4));
-    if (c == whole && p.k % 16) {
-        const int k = c * 16 + kq, n = max(0, min(4, p.k - k));
-        add(load4(src + k, n), operand(k, n));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) red[wave][kq + i][l16] = acc[i];
-    __syncthreads();
-    if (tid >= 256) return;
-    const int r = tid >> 4, jj = tid & 15;
-    if (row0 + r >= g.t || j0 + jj >= p.r) return;
-    float s = red[0][r][jj];
-#pragma unroll
-    for (int w = 1; w < kDownWaves; w++) s += red[w][r][jj];
-    p.out[(long)(row0 + r) * p.r + j0 + jj] = p.scale * s;
-}
 
 // part[chunk][n][j] = sum over the chunk's tokens i of big[i][n] * small[i][j].
 // A workgroup takes 64 columns n and 16 j of one chunk; lane l loads columns
@@ -191,31 +126,6 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(const LoraGrad g)
 int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
 }  // namespace
-
-hipError_t launch_lora_down(const LoraDown& g, bool m_rows, hipStream_t st) {
-    int blocks = 0;
-    for (int i = 0; i < g.njobs; i++) blocks += cdiv(g.job[i].r, 16);
-    // One launch up to 2^27 tokens and 65535 blocks of ranks (a grid has fewer
-    // than 2^32 threads along x and 2^16 blocks along y).
-    constexpr int kTokens = (1 << 27) - 16, kBlocksY = 65535;
-    LoraDown l = g;
-    for (l.y0 = 0; l.y0 < blocks; l.y0 += kBlocksY)
-        for (int t0 = 0; t0 < g.t; t0 += l.t) {
-            l.t = std::min(g.t - t0, kTokens);
-            for (int i = 0; i < g.njobs; i++) {
-                l.job[i].src = g.job[i].src + (long)t0 * g.job[i].k;
-                l.job[i].out = g.job[i].out + (long)t0 * g.job[i].r;
-            }
-            const dim3 grid(cdiv(l.t, 16), std::min(blocks - l.y0, kBlocksY));
-            if (m_rows)
-                lora_down_kernel<true><<<grid, 64 * kDownWaves, 0, st>>>(l);
-            else
-                lora_down_kernel<false><<<grid, 64 * kDownWaves, 0, st>>>(l);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-    return hipSuccess;
-}
 
 size_t lora_grad_plan(LoraGrad& g) {
     // Chunks of whole 64-token batches, as many as make about 768 workgroups

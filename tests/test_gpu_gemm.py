@@ -74,6 +74,30 @@ def test_gemm_rows_longer_than_32_bit_offsets():
     check("nt", 65, (1 << 22) + 5, 3)
 
 
+def test_gemm_few_rows_of_long_strides():
+    """B rows more than 2^26 values apart: 12 of them pass 2^32 bytes."""
+    from cpuforge_amd import ops as P
+    m, k, n = 3, 21, (1 << 26) + 3
+    g = torch.Generator(device=DEV).manual_seed(2)
+    a, b = torch.randn(m, k, generator=g, device=DEV), torch.randn(k, n, generator=g, device=DEV)
+    c = torch.full((m, n), float("nan"), device=DEV)
+    P.matmul_nn(a, b, c, m, k, n, False)
+    for part in (slice(0, 1000), slice(n - 1000, n)):
+        ad, bd = a.double(), b[:, part].double()
+        assert bool(((c[:, part] - ad @ bd).abs() <= 2.0 ** -24 * (k + 8) * (ad.abs() @ bd.abs())).all())
+
+
+@pytest.mark.parametrize("kind", ["nn", "nt"])
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 40])
+@pytest.mark.parametrize("k,n", [(16, 16), (15, 17), (512, 33), (513, 15), (531, 700), (1100, 48)])
+def test_gemm_few_rows(kind, m, k, n):
+    """The kernel for few rows at the edges of its 16 x 16 tiles, its runs of 16
+    k and its batches of 512."""
+    print(kind, m, k, n, flush=True)
+    check(kind, m, k, n)
+    check(kind, m, k, n, acc=True)
+
+
 @pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
 def test_gemm_small_and_large_magnitudes(kind):
     """Inputs whose low pieces are bf16 subnormals keep their products'
