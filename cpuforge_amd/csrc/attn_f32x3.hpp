@@ -15,10 +15,10 @@
 // Each product keeps two sums, the leading pieces' and the other five's
 // (split3.hpp: in one sum the small products lose low bits in one direction).
 //
-// Bound: the two waves of a SIMD issue 48 MFMAs (1536 cycles) and about 290
+// Bound: the two waves of a SIMD issue 48 MFMAs (1536 cycles) and about 300
 // VALU instructions (softmax, the pieces of P and of the tiles) a step; with f32
-// MFMAs it was 64 of 64 cycles each.  B8 S2048 9/3 heads D64 0.362 -> 0.235 ms,
-// B4 S1024 16/8 D128 0.180 -> 0.155.  (dK/dV the same way: its K and V pieces,
+// MFMAs it was 64 of 64 cycles each.  B8 S2048 9/3 heads D64 0.362 -> 0.242 ms
+// (0.235 without the split's power of two), B4 S1024 16/8 D128 0.180 -> 0.155.  (dK/dV the same way: its K and V pieces,
 // four pairs of sums and scores take 460 registers, one wave to a SIMD, which
 // hides nothing: 850 us where two waves of the f32 kernel take 720.)
 #pragma once

@@ -5,14 +5,20 @@
 //
 // What bounds it: on a full chip the board's power.  2000 x 2048 x 8192 (m, k,
 // n) ran at 1.85 of 2.4 GHz with the matrix cores busy in 62% of the cycles:
-// 176-200 TFLOP/s of f32 work, 1050-1200 of bf16, against 140 for the f32 MFMA
+// 160-200 TFLOP/s of f32 work, 960-1200 of bf16, against 133-144 for the f32 MFMA
 // library GEMM it replaced (the bf16 MFMA alone reaches 1704 on random
 // operands).  On the small grids of a layer (160 tiles of 128 x 128 for 4096
 // x 576) it is a workgroup's own chain: two waves to a SIMD, 49% matrix-core
 // busy between the splitting, the LDS reads and one barrier a step.  Before
-// and after, in us: 4096 x 1536 x 576 70 and 64; 4096 x 576 x 1536 69 and 58;
-// the LM head's 2730 x 576 x 49152 1200 and 939, its gradients 2730 x 49152 x 576
-// 2640 and 947 and 49152 x 2730 x 576 1220 and 936.
+// and after, in us: 4096 x 1536 x 576 70 and 65 (A B^T), 71 and 70 (A B); 4096 x 576 x
+// 1536 65 and 53, 62 and 54; 2000 x 2048 x 8192 465 and 345; the LM head's 2730 x 576 x
+// 49152 1160 and 926, its gradients 2730 x 49152 x 576 2610 and 983 and 49152 x 2730 x
+// 576 1150 and 965.  (Of these 2-7% is the scaling of the values, split3.hpp: 885,
+// 933 and 917 for the last three without.)  From 128 to 512 rows by a layer's
+// widths it is slower than the library was: 128 x 1536 x 576 7.5 and 12.4, 256 x 576 x 1536
+// 8.1 and 14.6, 512 x 576 x 1536 10.8 and 15.0, 576 x 512 x 1536 (A^T B) 11.7 and 17.2; with
+// fewer rows the kernel for few rows (below) runs.  (There, two or three groups of
+// waves to a tile, each over its part of k: 12.6 where this takes 15.0, 16.0 for 18.0.)
 //
 // A workgroup splits its tiles as it stores them to LDS (three planes), so
 // memory is read in f32, once per tile.  Two LDS buffers and two register

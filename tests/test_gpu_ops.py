@@ -6,7 +6,7 @@ Bars: bitwise where the kernel keeps the reference's order of f32 operations
 (RMSNorm forward, AdamW); otherwise the reference's own test tolerance,
 `|a - r| / (1 + |r|)` (core/src/gradcheck.rs:31-48): 1e-5 for RMSNorm's
 backward, SwiGLU and cross-entropy, whose row sums run in a parallel order,
-and matmul.rs's 1e-4 (core/src/matmul.rs:200-282) for the hipBLASLt GEMMs."""
+and matmul.rs's 1e-4 (core/src/matmul.rs:200-282) for the GEMMs."""
 import numpy as np
 import pytest
 import torch
